@@ -52,9 +52,11 @@ constexpr int kChunkTiles = 1024;   // tiles of one band a coverage block handle
 // tile, whose bytes (8 rows of 8, row-major) sit at slot (band * tiles_x + k).
 constexpr uint32_t kTileEmpty = 0, kTileFull = 1, kTileSlot0 = 2;
 constexpr uint32_t kMaxTilesX = 65279u;  // widest job grid (a u16 table entry and tile state address its slots)
-// crossings per sub-scanline that the coverage kernel's variants hold (more keys,
-// more LDS per wave, fewer waves per CU)
+// edges of a band that the coverage kernel's variants hold (more edges, more LDS per
+// block, fewer waves per CU); a band that more edges meet is crowded and takes a kernel
+// of its own, so a flush has one list of bands per variant and one of the crowded ones
 constexpr uint32_t kCoverageKeys[3] = {128, 256, 512};
+constexpr int kBandLists = 4;
 
 // A coverage job computes u8 coverage for the pixel rect [x0, x0+w) x [y0, y0+h)
 // of its pixmap (coordinates of the edge space; coverage is 0 outside the rect).
@@ -262,6 +264,20 @@ struct JobPrep {
     std::vector<uint2> windows;
     std::vector<uint8_t> tier;       // per band: index into kCoverageKeys
     uint32_t tier_count[3] = {0, 0, 0};
+    std::vector<uint32_t> crowded;   // the bands (ascending, of the last tier) that more edges meet
+    // the band list that band g (visited in ascending order) goes to; `c` counts the
+    // crowded bands passed
+    int band_list(size_t g, size_t &c) const {
+        if (c < crowded.size() && crowded[c] == g) {
+            c++;
+            return 3;
+        }
+        return tier[g];
+    }
+    uint32_t list_count(int t) const {
+        const uint32_t n = (uint32_t)crowded.size();
+        return t == 3 ? n : tier_count[t] - (t == 2 ? n : 0u);
+    }
     uint64_t pieces = 0;             // piece slots of all edges
     uint64_t piece_base = 0;         // first piece slot in the draw list (add_job)
 };

@@ -5,17 +5,16 @@
 // update loop (Skia's forward differencing in 16.16 fixed point) from the state the
 // host left after the first piece, writing every non-empty line piece in order.
 //
-// Coverage (k_coverage): one 64-lane wave per (coverage job, band of 8 pixel rows).
-// Per row, the band's edge window comes from the job's table; each lane takes an
-// edge, binary-searches its pieces for the row and produces the crossings of the
-// row's sub-scanlines.  Per sub-scanline the crossings (keys: x, edge id, winding)
-// are sorted with a register-resident bitonic network (up to 8 keys per lane), the
-// windings are scanned into span events (tiny-skia's walk_edges spans), and the
-// SuperBlitter contributions (16 per covered sub-column of a partial pixel, 64 or 63
-// for a fully covered pixel) are accumulated per 512-pixel window in LDS,
-// prefix-summed and clamped to 255.  Coverage leaves the kernel as 8 x 8 tiles
-// aligned to the target: a u16 table entry per tile (empty, full, or the slot of a
-// partial tile's 64 bytes), so only tiles that an edge crosses cost memory.
+// Coverage (k_coverage): a block of eight 64-lane waves per (coverage job, band of 8
+// pixel rows), one wave per row.  The block's threads leave the crossings of the band's
+// edges with its sub-scanlines in LDS; each wave sorts its row's four sub-scanlines
+// (keys: x, edge id, winding) with a register-resident bitonic network and turns them
+// into span events (tiny-skia's walk_edges spans); the SuperBlitter contributions (16
+// per covered sub-column of a partial pixel, 64 or 63 for a fully covered pixel) are
+// accumulated per 512-pixel window in LDS, prefix-summed and clamped to 255.  Coverage
+// leaves the kernel as 8 x 8 tiles aligned to the target: a u16 table entry per tile
+// (empty, full, or the slot of a partial tile's 64 bytes), so only tiles that an edge
+// crosses cost memory.
 //
 // Compositing (k_draw): one thread per target pixel, one wave per 8 x 8 tile,
 // looping over the draw items in order with the pixel in a register: tile-table
@@ -156,28 +155,46 @@ struct CovArgs {
     int32_t *overflow;
 };
 
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-    for (int d = 1; d < kWave; d <<= 1) {
-        int t = __shfl_up(v, d, kWave);
-        if (lane >= d) v += t;
-    }
+// Inclusive sum over the wave's lanes in six DPP additions (shifts within the 16-lane
+// rows, then the row totals broadcast to the rows after them); no LDS traffic.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_from(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ int wave_incl_scan(int v) {
+    v += dpp_from<0x111, 0xf>(v);  // row_shr:1
+    v += dpp_from<0x112, 0xf>(v);
+    v += dpp_from<0x114, 0xf>(v);
+    v += dpp_from<0x118, 0xf>(v);
+    v += dpp_from<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    v += dpp_from<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
     return v;
 }
 
-__device__ __forceinline__ uint64_t shfl_xor64(uint64_t v, int m) {
-    const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)v, m, kWave);
-    const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), m, kWave);
-    return ((uint64_t)hi << 32) | lo;
+// set bits of `m` below this lane
+__device__ __forceinline__ int lanes_below(uint64_t m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-// Lane exchange across xor distance LD (1..32) for the bitonic network: an
-// immediate-pattern ds_swizzle within 32-lane halves, ds_bpermute across them.
+// Lane exchange across xor distance LD (1..32) for the bitonic network, all in the VALU
+// (the coverage kernel's LDS pipe is busy with keys and accumulators): DPP patterns
+// within the 16-lane rows, row and half swaps across them.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_perm(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xf, 0xf, true);
+}
 template <int LD>
-__device__ __forceinline__ uint32_t xor_lane(uint32_t v) {
-    if constexpr (LD < 32) {
-        return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, (LD << 10) | 0x1F);
+__device__ __forceinline__ uint32_t xor_lane(uint32_t v, int lane) {
+    if constexpr (LD == 1) return dpp_perm<0xB1>(v);                    // quad_perm [1, 0, 3, 2]
+    else if constexpr (LD == 2) return dpp_perm<0x4E>(v);               // quad_perm [2, 3, 0, 1]
+    else if constexpr (LD == 4) return dpp_perm<0x1B>(dpp_perm<0x141>(v));  // mirror of 8, then of 4
+    else if constexpr (LD == 8) return dpp_perm<0x128>(v);              // row_ror:8
+    else if constexpr (LD == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return (lane & 16) ? r[0] : r[1];
     } else {
-        return (uint32_t)__shfl_xor((int)v, LD, kWave);
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return (lane & 32) ? r[0] : r[1];
     }
 }
 
@@ -196,7 +213,8 @@ __device__ __forceinline__ void bitonic_stage(uint64_t (&v)[S][K], int lane) {
 #pragma unroll
             for (int j = 0; j < K; j++) {
                 const uint64_t x = v[s][j];
-                const uint64_t o = ((uint64_t)xor_lane<ld>((uint32_t)(x >> 32)) << 32) | xor_lane<ld>((uint32_t)x);
+                const uint64_t o = ((uint64_t)xor_lane<ld>((uint32_t)(x >> 32), lane) << 32) |
+                                   xor_lane<ld>((uint32_t)x, lane);
                 v[s][j] = ((o < x) == keep_min) ? o : x;
             }
     } else {
@@ -255,7 +273,7 @@ __device__ __forceinline__ void spans_of(uint64_t (*keys)[MK], const int *n, boo
             w[j] = e < n[s] ? ((v[s][j] & 1) ? 1 : -1) : 0;
             local += w[j];
         }
-        const int incl = wave_incl_scan(local, lane);
+        const int incl = wave_incl_scan(local);
         int before = base[s] + incl - local;
         const bool in0 = evenodd ? (base[s] & 1) != 0 : base[s] != 0;
         const int total = base[s] + __shfl(incl, kWave - 1, kWave);
@@ -271,7 +289,7 @@ __device__ __forceinline__ void spans_of(uint64_t (*keys)[MK], const int *n, boo
             nevt += evt[j] ? 1 : 0;
             before = after;
         }
-        const int eincl = wave_incl_scan(nevt, lane);
+        const int eincl = wave_incl_scan(nevt);
         int pos = eincl - nevt + (in0 ? 1 : 0);
         int32_t *ev = reinterpret_cast<int32_t *>(keys[s]);
 #pragma unroll
@@ -293,25 +311,334 @@ constexpr uint32_t kStatePartial = 256u;
 static_assert(rvkr::kMaxTilesX + kStatePartial <= 65536u, "a partial tile's state fits 16 bits");
 static_assert(kWin == 8 * kWave, "a lane holds one 8-pixel tile row of a window");
 
-// MK: crossings per sub-scanline the launch can hold (128, 256 or 512; the keys take
-// 4, 8 or 16 KB of LDS, so the smaller variants run two to three times the waves per
-// CU).  The host sends a band to the smallest variant that holds the number of edges
-// whose rows meet the band, an upper bound on any of its sub-scanlines' crossings.
+// ---- coverage of a band, one wave per pixel row ----
+// A sub-scanline's crossings, each lane's J of them in v[s] (element lane * J + j,
+// ~0 for none), sorted ascending; n[s] of them are real.  Writes the span events
+// (pixel-rounded supersampled columns; starts and ends alternate) to ev[s] and returns
+// their count.  Every real crossing changes the winding by one, so with U upward
+// crossings before element e the winding there is 2 U - e, and ballots give every
+// prefix; under the even-odd rule every crossing is an event.
+constexpr int32_t kOpenEnd = 0x3fffffff;  // the end of a span that its sub-scanline leaves open
+
+template <int J>
+__device__ __forceinline__ int row_events(const uint64_t (&v)[J], int n, bool evenodd, int32_t *ev, int lane) {
+    int32_t x[J];
+#pragma unroll
+    for (int j = 0; j < J; j++)
+        x[j] = ((int32_t)((uint32_t)(v[j] >> 32) ^ 0x80000000u) + 0x8000) >> 16;
+    if (evenodd) {
+#pragma unroll
+        for (int j = 0; j < J; j++)
+            if (lane * J + j < n) ev[lane * J + j] = x[j];
+        if (n & 1) {
+            if (lane == 0) ev[n] = kOpenEnd;
+            return n + 1;
+        }
+        return n;
+    }
+    bool up[J];
+    int before = -lane * J;  // the winding before this lane's first element
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        up[j] = lane * J + j < n && (v[j] & 1) != 0;
+        before += 2 * lanes_below(__ballot(up[j]));
+    }
+    bool evt[J];
+    int pos = 0, total = 0;
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const int after = before + (up[j] ? 1 : -1);
+        evt[j] = lane * J + j < n && (before == 0 || after == 0);
+        before = after;
+        const uint64_t m = __ballot(evt[j]);
+        pos += lanes_below(m);
+        total += __popcll(m);
+    }
+#pragma unroll
+    for (int j = 0; j < J; j++)
+        if (evt[j]) ev[pos++] = x[j];
+    if (total & 1) {
+        if (lane == 0) ev[total] = kOpenEnd;
+        total++;
+    }
+    return total;
+}
+
+// The span events of one row's sub-scanlines from the crossings in ev (element e's
+// sub-scanlines in bits shift .. shift + 3 of act[e], its id and direction in meta[e]),
+// which they replace; the event counts in nev.
+template <int J, int STRIDE>
+__device__ __forceinline__ void sort_row(int32_t (*ev)[STRIDE], const uint32_t *act, int shift, const uint32_t *meta,
+                                         int nact, bool evenodd, int *nev, int lane) {
+    uint64_t v[kMaxSub][J];
+    int cnt[kMaxSub] = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const int e = lane * J + j;
+        const uint32_t bits = e < nact ? act[e] >> shift : 0u;
+        const uint32_t lo = e < nact ? meta[e] : 0u;
+#pragma unroll
+        for (int s = 0; s < kMaxSub; s++) {
+            const bool on = (bits >> s) & 1u;
+            v[s][j] = on ? ((uint64_t)((uint32_t)ev[s][e] ^ 0x80000000u) << 32) | lo : ~0ull;
+            cnt[s] += __popcll(__ballot(on));
+        }
+    }
+    if (cnt[0] + cnt[1] + cnt[2] + cnt[3] != 0) bitonic_from<J, kMaxSub, 2, 1>(v, lane);
+#pragma unroll
+    for (int s = 0; s < kMaxSub; s++) nev[s] = row_events<J>(v[s], cnt[s], evenodd, ev[s], lane);
+}
+
+constexpr int kRowWaves = rvkr::kBandRows;        // waves of a block: one per pixel row of the band
+constexpr int kAccWords = kWin / 2 + 4;           // a window's pixel differences, two per word, and their spill
+
+// MK: edges that the band holds (128, 256 or 512).  The host sends a band to the
+// smallest variant that holds the edges whose rows meet it.
 //
-// Block b handles band bands[b].y (8 pixel rows) of job bands[b].x.  At the start of
-// the band the edges of its window that meet its rows are gathered into registers
-// (lane l holds active edges l, l + 64, ...) with the index of the piece each one is
-// on; row by row every active edge steps its piece forward and emits its crossings,
-// the sub-scanlines are sorted together and turned into spans, and the spans are
-// accumulated per 512-pixel window in LDS (each window visits only the spans that
-// reach it), prefix-summed and clamped to 255.  Each lane then holds one 8-pixel row
-// of a tile, which is tracked as uniform (every pixel so far one value) or partial: a
-// tile turns partial at the first row that differs, takes the band's next slot, and
-// from then on its rows are written there (the earlier, uniform rows are filled in at
-// that point); at the end of the band the tile table gets empty, full or the slot.
+// Block b handles band bands[b].y (8 pixel rows) of job bands[b].x, wave r its row r.
+// * The 512 threads pick the band's active edges out of its window.  Then MK / 64
+//   threads share an edge: each walks the pieces over its J rows and leaves the crossing
+//   of every sub-scanline in LDS (x by sub-scanline and edge, and an edge's sub-scanlines
+//   as a bit mask).
+// * Each wave sorts its row's sub-scanlines (a bitonic network over 64 J keys held in
+//   registers, exchanged in the VALU) and turns them into span events, which take the
+//   crossings' place in LDS.
+// * Per 512-pixel window a wave adds its spans' coverage as differences (16 bit, two
+//   pixels a word, exact modulo 2^32), each lane prefix-sums one 8-pixel tile row, and the
+//   waves agree on which of the window's 64 tiles are all 0, all 255 or partial through
+//   two 64-bit masks; each writes its row of the partial tiles.
+// Windows alternate between three mask slots, so one barrier a window is enough.
+//
+// Why a wave per row: a row's work is a chain of dependent steps (piece loads, sort
+// stages, window scans), and one wave walking its band's 8 rows took 90-200 us however
+// small the launch, with the wider variants' few bands leaving the chip idle (the 512
+// variant's VALU 13% busy).  Per row the old form issued 2400 VALU, 1600 SALU and 450 LDS
+// wave instructions, the LDS pipe as busy as the VALU; scans and sort exchanges moved to
+// DPP, winding prefixes to ballots, and differences instead of two packed sums.  With
+// 28 KB of LDS and 32 VGPRs the 128 variant runs 8 waves per SIMD (4 before).  Renders:
+// 4096^2, 2000 paths 150.4 -> 120.7 ms; 1201x843, 64 paths 3.36 -> 1.95 ms; 2048^2 with
+// 150 clipped or masked groups 90.1 -> 64.6 ms; 64 documents in a batch 109 -> 87 ms.
 template <int MK>
-__global__ __launch_bounds__(kWave) void k_coverage(CovArgs a) {
-    constexpr int J = MK / kWave;  // active edges per lane
+__global__ __launch_bounds__(kRowWaves * kWave) void k_coverage(CovArgs a) {
+    constexpr int J = MK / kWave;          // keys per lane, and rows per thread of the gather
+    constexpr int PARTS = rvkr::kBandRows / J;
+    constexpr int kThreads = kRowWaves * kWave;
+    static_assert(PARTS * MK == kThreads, "a thread per edge and J rows");
+    constexpr int kStride = MK + 4;        // a row of crossings, and its events with an open end
+    __shared__ __align__(16) int32_t xs[rvkr::kBandRows * kMaxSub][kStride];
+    __shared__ uint32_t act[PARTS][MK];    // bits (row in the part) * 4 + sub-scanline
+    __shared__ uint32_t meta[MK];          // id << 1 | upward
+    __shared__ uint32_t list[MK];
+    __shared__ __align__(16) uint32_t acc[kRowWaves][kAccWords];
+    __shared__ int wcount[kRowWaves];
+    __shared__ __align__(16) uint64_t masks[3][2];  // tiles of the window that are 0 / 255 in every row so far
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int r = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const uint2 bj = a.bands[blockIdx.x];
+    const CovJob job = a.jobs[bj.x];
+    const uint32_t band = bj.y;
+    const int shift = job.aa ? 2 : 0, nsub = 1 << shift;
+    const bool evenodd = job.rule == RVK_FILL_EVENODD;
+    const int32_t row0 = job.gy0 + (int32_t)band * rvkr::kBandRows;
+    const int32_t ry0 = max(row0, job.y0), ry1 = min(row0 + rvkr::kBandRows, job.y0 + job.h);  // covered rows
+    const EdgeCov *edges = a.edges + job.edge_offset;
+
+    // ---- the band's active edges ----
+    const int32_t sb0 = ry0 << shift, sb1 = (ry1 << shift) - 1;  // covered sub-scanlines
+    const uint2 win = a.windows[job.window_offset + band];
+    for (int i = tid; i < kRowWaves * kAccWords; i += kThreads) (&acc[0][0])[i] = 0;
+    if (tid < 6) masks[tid / 2][tid % 2] = ~0ull;
+    int nact = 0;
+    for (uint32_t base = win.x; base < win.y; base += kThreads) {
+        const uint32_t i = base + (uint32_t)tid;
+        bool meets = false;
+        if (i < win.y) {
+            const int2 rows = *reinterpret_cast<const int2 *>(&edges[i].first_y);  // first_y, ymax
+            meets = rows.x <= sb1 && rows.y >= sb0;
+        }
+        const uint64_t m = __ballot(meets);
+        if (lane == 0) wcount[r] = __popcll(m);
+        __syncthreads();
+        int pos = nact + lanes_below(m);
+#pragma unroll
+        for (int w = 0; w < kRowWaves; w++) {
+            const int c = wcount[w];
+            if (w < r) pos += c;
+            nact += c;
+        }
+        if (meets && pos < MK) list[pos] = i;
+        __syncthreads();
+    }
+    if (nact > MK) {  // the host's count was too small: reported, the rest dropped
+        if (tid == 0) atomicAdd(a.overflow, 1);
+        nact = MK;
+    }
+    // ---- their crossings ----
+    {
+        const int slot = tid % MK, part = tid / MK;
+        if (slot < nact) {
+            const uint32_t i = list[slot];
+            const EdgeCov e = edges[i];
+            const PieceDev *pc = a.pieces + e.piece_offset;
+            const uint32_t n = a.npieces[job.edge_offset + i];
+            const int32_t y0 = row0 + part * J;
+            const int32_t s0 = max(y0, ry0) << shift, s1 = min(y0 + J, ry1) << shift;
+            uint32_t bits = 0;
+            if (part == 0) meta[slot] = ((uint32_t)e.id << 1) | (e.winding > 0 ? 1u : 0u);
+            if (e.first_y < s1 && e.ymax >= s0) {
+                uint32_t k = 0;
+                if (e.first_y < s0) {  // the first piece that reaches s0
+                    uint32_t hi = n;
+                    while (k < hi) {
+                        const uint32_t mid = (k + hi) >> 1;
+                        if (pc[mid].last_y < s0) k = mid + 1;
+                        else hi = mid;
+                    }
+                }
+                if (k < n) {
+                    PieceDev p = pc[k];
+                    for (int32_t sy = s0; sy < s1; sy++) {
+                        while (p.last_y < sy && k + 1 < n) p = pc[++k];
+                        if (p.first_y <= sy && p.last_y >= sy) {
+                            const int32_t y = sy >> shift, s = sy - (y << shift);
+                            xs[(y - row0) * kMaxSub + s][slot] =
+                                (int32_t)((uint32_t)p.x + (uint32_t)(sy - p.first_y) * (uint32_t)p.dx);
+                            bits |= 1u << ((y - y0) * kMaxSub + s);
+                        }
+                    }
+                }
+            }
+            act[part][slot] = bits;
+        }
+    }
+    __syncthreads();
+    // ---- this row's span events ----
+    int32_t(*ev)[kStride] = &xs[r * kMaxSub];
+    int nev[kMaxSub];
+    if (J > 1 && nact <= kWave)
+        sort_row<1>(ev, act[r / J], r % J * kMaxSub, meta, nact, evenodd, nev, lane);
+    else
+        sort_row<J>(ev, act[r / J], r % J * kMaxSub, meta, nact, evenodd, nev, lane);
+    // ---- windows ----
+    const int sl = lane >> 4;  // lanes 16 s .. 16 s + 15 look at sub-scanline s's spans
+    const int nspl = (sl < 2 ? (sl == 0 ? nev[0] : nev[1]) : (sl == 2 ? nev[2] : nev[3])) >> 1;
+    const int32_t *evl = ev[sl];
+    const bool any = (nev[0] | nev[1] | nev[2] | nev[3]) != 0;
+    const int32_t maxv = job.aa ? (sl == 3 ? 63 : 64) : 255;
+    const int32_t rx0 = job.x0, rx1 = job.x0 + job.w;  // covered columns
+    const int32_t cw = (int32_t)job.tiles_x * rvkr::kTile;
+    uint32_t *wacc = acc[r];
+    uint16_t *tab = a.table + job.table_offset + (size_t)band * job.tiles_x;
+    uint8_t *slots = a.arena + job.cov_offset + (size_t)band * job.tiles_x * 64u;
+    uint32_t nslots = 0;  // partial tiles of the band so far
+    int kst = 0;          // the first span of this lane's sub-scanline not behind the windows
+    int mslot = 0, wi = 0;
+    for (int32_t wx0 = 0; wx0 < cw; wx0 += kWin, wi++) {
+        const int32_t ww = min(kWin, cw - wx0);  // a multiple of kTile
+        const int32_t wabs = job.gx0 + wx0;
+        uint32_t w0 = 0, w1 = 0;
+        if (any) {
+            // spans cut to the window and to the job's columns (coverage is 0 outside)
+            const int32_t colbase = wabs << shift, wend = colbase + (ww << shift);
+            const int32_t lo = max(0, rx0 - wabs) << shift, hi = max(0, min(ww, rx1 - wabs)) << shift;
+            // the next 16 spans of each sub-scanline: those that start before the window's
+            // end are a prefix of them, as are those that end at or before it
+            // (a sub-scanline whose 16 spans all end there is looked at again)
+            bool live = true;
+            do {
+                const int k = kst + (lane & 15);
+                int32_t L = INT32_MAX, R = INT32_MAX;
+                if (live && k < nspl) {
+                    L = evl[2 * k];
+                    R = evl[2 * k + 1];
+                }
+                const bool in = L < wend;
+                if (in) {
+                    const int32_t l = max(L - colbase, lo), h = min(R - colbase, hi);
+                    if (h > l) {
+                        auto add = [&](int32_t p, int32_t d) { atomicAdd(&wacc[p >> 1], (uint32_t)d << ((p & 1) * 16)); };
+                        if (!job.aa) {
+                            add(l, 255);
+                            add(h, -255);
+                        } else {
+                            const int32_t pl = l >> 2, pr = h >> 2, fb = l & 3, fe = (h & 3) * 16;
+                            if (pl == pr) {
+                                const int32_t d = fe - fb * 16;
+                                add(pl, d);
+                                add(pl + 1, -d);
+                            } else {
+                                const int32_t first = fb ? 64 - fb * 16 : maxv;  // pixel pl; then full ones, then fe
+                                add(pl, first);
+                                if (pr > pl + 1) {
+                                    if (first != maxv) add(pl + 1, maxv - first);
+                                    add(pr, fe - maxv);
+                                } else {
+                                    add(pr, fe - first);
+                                }
+                                if (fe) add(pr + 1, -fe);
+                            }
+                        }
+                    }
+                }
+                const uint64_t mdone = __ballot(R <= wend);
+                const uint32_t half = sl < 2 ? (uint32_t)mdone : (uint32_t)(mdone >> 32);
+                const uint32_t done = (half >> (16 * (sl & 1))) & 0xffffu;
+                kst += __popc(done);
+                live = done == 0xffffu;
+            } while (__ballot(live) != 0);
+            // ---- prefix sum: lane l holds pixels [8 l, 8 l + 8), one tile row; the
+            // accumulator is cleared behind the read ----
+            uint4 q = *reinterpret_cast<const uint4 *>(&wacc[4 * lane]);
+            *reinterpret_cast<uint4 *>(&wacc[4 * lane]) = make_uint4(0, 0, 0, 0);
+            if (lane == 0) wacc[kWin / 2] = 0;
+            // a word is lo + 65536 hi of two signed differences, so the words' sum is the
+            // sums of both, and word * 65537 the running pair
+            const uint32_t sum = q.x + q.y + q.z + q.w;
+            const int32_t slo = (int32_t)(int16_t)sum;
+            const int32_t loc = slo + ((int32_t)(sum - (uint32_t)slo) >> 16);
+            const uint32_t run = (uint32_t)(wave_incl_scan(loc) - loc);
+            auto pair = [](uint32_t before, uint32_t w) { return (before << 16) + before + (w << 16) + w; };
+            const uint32_t p0 = pair(run, q.x), p1 = pair(p0 >> 16, q.y), p2 = pair(p1 >> 16, q.z),
+                           p3 = pair(p2 >> 16, q.w);
+            // each field is a pixel's coverage, at most 256: 256 becomes 255
+            auto clamp2 = [](uint32_t p) { return p - ((p >> 8) & 0x00010001u); };
+            w0 = __builtin_amdgcn_perm(clamp2(p1), clamp2(p0), 0x06040200u);
+            w1 = __builtin_amdgcn_perm(clamp2(p3), clamp2(p2), 0x06040200u);
+        }
+        // ---- the window's tiles ----
+        const bool valid = 8 * lane < ww;
+        const uint64_t mz = __ballot(!valid || (w0 | w1) == 0u), mf = __ballot(valid && (w0 & w1) == ~0u);
+        if (lane == 0) {
+            atomicAnd((unsigned long long *)&masks[mslot][0], (unsigned long long)mz);
+            atomicAnd((unsigned long long *)&masks[mslot][1], (unsigned long long)mf);
+        }
+        const int next = mslot == 2 ? 0 : mslot + 1;
+        if (tid < 2) masks[next][tid] = ~0ull;  // last read before the previous barrier
+        __syncthreads();
+        const uint64_t zero = masks[mslot][0], full = masks[mslot][1];
+        const uint64_t part = ~(zero | full);
+        const uint32_t k = nslots + (uint32_t)lanes_below(part);
+        const bool mine = (part >> lane) & 1ull;
+        if (mine) *reinterpret_cast<uint2 *>(slots + (size_t)k * 64u + r * 8) = make_uint2(w0, w1);
+        if (r == (wi & (kRowWaves - 1)) && valid)
+            tab[wx0 / rvkr::kTile + lane] = (uint16_t)(mine ? rvkr::kTileSlot0 + k
+                                                            : ((zero >> lane) & 1ull ? rvkr::kTileEmpty : rvkr::kTileFull));
+        nslots += (uint32_t)__popcll(part);
+        mslot = next;
+    }
+}
+
+// A band that more edges meet than k_coverage<kMaxKeys> holds (many short edges, such as
+// the arcs of round joins): one 64-lane wave per band, row by row over every edge of the
+// band's window, with up to kMaxKeys crossings per sub-scanline sorted at a time.  A
+// sub-scanline with more is redone in narrower column chunks.  The spans are accumulated
+// per 512-pixel window in LDS, prefix-summed and clamped to 255.  Each lane then holds
+// one 8-pixel row of a tile, which is tracked as uniform (every pixel so far one value)
+// or partial: a tile turns partial at the first row that differs, takes the band's next
+// slot, and from then on its rows are written there (the earlier, uniform rows are filled
+// in at that point); at the end of the band the tile table gets empty, full or the slot.
+__global__ __launch_bounds__(kWave) void k_coverage_many(CovArgs a) {
+    constexpr int MK = kMaxKeys;
     __shared__ uint64_t keys[kMaxSub][MK];  // crossings; reused for span events
     __shared__ __align__(16) int32_t acc[kWin + 8];  // acc (low 16 bits) + run difference (high 16 bits)
     __shared__ uint16_t tstate[rvkr::kChunkTiles];
@@ -332,52 +659,7 @@ __global__ __launch_bounds__(kWave) void k_coverage(CovArgs a) {
     const uint32_t *npieces = a.npieces + job.edge_offset;
 
     for (int i = lane; i < kWin + 8; i += kWave) acc[i] = 0;  // each window clears it behind its read
-    // ---- the band's active edges: the window's edges whose rows meet the band ----
-    const int32_t sb0 = ry0 * nsub_aa, sb1 = ry1 * nsub_aa - 1;  // covered sub-scanlines
-    uint32_t eidx[J], ek[J];  // an active edge (index in the job) and the piece it is on
-    int nact = 0;
     const uint2 win = a.windows[job.window_offset + band];
-    {
-        uint32_t *list = reinterpret_cast<uint32_t *>(&keys[0][0]);
-        for (uint32_t base = win.x; base < win.y; base += kWave) {
-            const uint32_t i = base + (uint32_t)lane;
-            bool meets = false;
-            if (i < win.y) {
-                const EdgeCov e = edges[i];
-                meets = e.first_y <= sb1 && e.ymax >= sb0;
-            }
-            const uint64_t m = __ballot(meets);
-            const int pos = nact + __popcll(m & below);
-            if (meets && pos < MK) list[pos] = i;
-            nact += __popcll(m);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < J; j++) {
-            const int e = lane + kWave * j;
-            eidx[j] = e < nact && nact <= MK ? list[e] : 0u;
-            ek[j] = 0;
-        }
-        __syncthreads();  // the key area is free again
-        // the first piece that reaches the band's first sub-scanline (an edge that
-        // starts inside the band starts on its first piece)
-#pragma unroll
-        for (int j = 0; j < J; j++) {
-            if (lane + kWave * j < nact && nact <= MK) {
-                const EdgeCov e = edges[eidx[j]];
-                if (e.first_y < sb0) {
-                    const PieceDev *pc = a.pieces + e.piece_offset;
-                    uint32_t lo = 0, hi = npieces[eidx[j]];
-                    while (lo < hi) {
-                        const uint32_t mid = (lo + hi) >> 1;
-                        if (pc[mid].last_y < sb0) lo = mid + 1;
-                        else hi = mid;
-                    }
-                    ek[j] = lo;
-                }
-            }
-        }
-    }
 
     uint32_t nslots = 0;  // partial tiles of the band so far
     // The band is processed in column chunks of up to kChunkTiles tiles.  Normally a
@@ -394,10 +676,6 @@ __global__ __launch_bounds__(kWave) void k_coverage(CovArgs a) {
         const int32_t c0s = cut ? cx0 * nsub_aa : INT32_MIN, c1s = cut ? (cx0 + cw) * nsub_aa : INT32_MAX;
         const uint32_t nslots0 = nslots;
         bool redo = false;
-        // a chunk after the first walks the band's rows again from its start
-        uint32_t k0[J];
-#pragma unroll
-        for (int j = 0; j < J; j++) k0[j] = ek[j];
         for (int r = 0; r < rvkr::kBandRows && !redo; r++) {
             const int32_t y = row0 + r;
             const bool row_in = y >= ry0 && y < ry1;
@@ -445,34 +723,23 @@ __global__ __launch_bounds__(kWave) void k_coverage(CovArgs a) {
                         if (cut) bd[s] += __popcll(__ballot(left[s] > 0)) - __popcll(__ballot(left[s] < 0));
                     }
                 };
-                if (nact <= MK) {
-                    // the band's active edges, each on the piece it reached
-#pragma unroll
-                    for (int j = 0; j < J; j++) {
-                        if (kWave * j >= nact) break;
-                        gather(lane + kWave * j < nact, eidx[j], k0[j]);
-                    }
-                } else {
-                    // more edges meet the band than the registers hold (many short edges,
-                    // such as the arcs of round joins): every edge of the window, its
-                    // piece found by binary search
-                    for (uint32_t base = win.x; base < win.y; base += kWave) {
-                        const uint32_t i = base + (uint32_t)lane;
-                        uint32_t k = 0;
-                        if (i < win.y) {
-                            const EdgeCov e = edges[i];
-                            if (e.first_y < sy0) {
-                                const PieceDev *pc = a.pieces + e.piece_offset;
-                                uint32_t hi = npieces[i];
-                                while (k < hi) {
-                                    const uint32_t mid = (k + hi) >> 1;
-                                    if (pc[mid].last_y < sy0) k = mid + 1;
-                                    else hi = mid;
-                                }
+                // every edge of the window, its piece found by binary search
+                for (uint32_t base = win.x; base < win.y; base += kWave) {
+                    const uint32_t i = base + (uint32_t)lane;
+                    uint32_t k = 0;
+                    if (i < win.y) {
+                        const EdgeCov e = edges[i];
+                        if (e.first_y < sy0) {
+                            const PieceDev *pc = a.pieces + e.piece_offset;
+                            uint32_t hi = npieces[i];
+                            while (k < hi) {
+                                const uint32_t mid = (k + hi) >> 1;
+                                if (pc[mid].last_y < sy0) k = mid + 1;
+                                else hi = mid;
                             }
                         }
-                        gather(i < win.y, i, k);
                     }
+                    gather(i < win.y, i, k);
                 }
                 __syncthreads();
                 // ---- sort the sub-scanlines together and turn them into span events ----
@@ -618,7 +885,7 @@ __global__ __launch_bounds__(kWave) void k_coverage(CovArgs a) {
                     d[q] = packed >> 16;
                     loc += d[q];
                 }
-                const int incl = wave_incl_scan(loc, lane);
+                const int incl = wave_incl_scan(loc);
                 int run = incl - loc;
                 uint32_t w0 = 0, w1 = 0;
 #pragma unroll
@@ -1105,25 +1372,26 @@ rvk_status launch_expand(rvk_context *ctx, const EdgeRec *edges, uint32_t nedges
     return RVK_OK;
 }
 
-rvk_status launch_coverage(rvk_context *ctx, const CovJob *jobs, uint32_t njobs, const uint2 *bands128,
-                           uint32_t n128, const uint2 *bands256, uint32_t n256, const uint2 *bands512,
-                           uint32_t n512, const EdgeCov *edges, const uint2 *windows, const PieceDev *pieces,
-                           const uint32_t *npieces, uint16_t *table, uint8_t *arena, int32_t *overflow,
-                           double algo_bytes) {
-    (void)njobs;
+rvk_status launch_coverage(rvk_context *ctx, const CovJob *jobs, const uint2 *const bands[rvkr::kBandLists],
+                           const uint64_t n_bands[rvkr::kBandLists], const EdgeCov *edges, const uint2 *windows,
+                           const PieceDev *pieces, const uint32_t *npieces, uint16_t *table, uint8_t *arena,
+                           int32_t *overflow, double algo_bytes) {
     // the algorithmic bytes are split between the launches by their band counts
-    const double total = (double)n128 + (double)n256 + (double)n512;
-    auto launch = [&](auto kernel, const uint2 *bands, uint32_t n) -> rvk_status {
-        if (n == 0) return RVK_OK;
-        CovArgs a{bands, jobs, edges, windows, pieces, npieces, table, arena, overflow};
-        timed_launch(ctx, "coverage", algo_bytes * (double)n / total,
-                     [&] { hipLaunchKernelGGL(kernel, dim3(n), dim3(kWave), 0, ctx->stream, a); });
+    double total = 0.0;
+    for (int t = 0; t < rvkr::kBandLists; t++) total += (double)n_bands[t];
+    auto launch = [&](auto kernel, int t, int threads) -> rvk_status {
+        if (n_bands[t] == 0) return RVK_OK;
+        CovArgs a{bands[t], jobs, edges, windows, pieces, npieces, table, arena, overflow};
+        timed_launch(ctx, "coverage", algo_bytes * (double)n_bands[t] / total, [&] {
+            hipLaunchKernelGGL(kernel, dim3((uint32_t)n_bands[t]), dim3(threads), 0, ctx->stream, a);
+        });
         RVK_HIP_CHECK(hipGetLastError());
         return RVK_OK;
     };
-    RVK_TRY(launch(k_coverage<(int)rvkr::kCoverageKeys[0]>, bands128, n128));
-    RVK_TRY(launch(k_coverage<(int)rvkr::kCoverageKeys[1]>, bands256, n256));
-    RVK_TRY(launch(k_coverage<(int)rvkr::kCoverageKeys[2]>, bands512, n512));
+    RVK_TRY(launch(k_coverage<(int)rvkr::kCoverageKeys[0]>, 0, kRowWaves * kWave));
+    RVK_TRY(launch(k_coverage<(int)rvkr::kCoverageKeys[1]>, 1, kRowWaves * kWave));
+    RVK_TRY(launch(k_coverage<(int)rvkr::kCoverageKeys[2]>, 2, kRowWaves * kWave));
+    RVK_TRY(launch(k_coverage_many, 3, kWave));
     return RVK_OK;
 }
 

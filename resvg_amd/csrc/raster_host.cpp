@@ -1009,6 +1009,7 @@ void prep_job(const EdgeSet &es, uint32_t rule, bool aa, IRect clip, int32_t lx,
         const uint8_t t = n <= kCoverageKeys[0] ? 0 : n <= kCoverageKeys[1] ? 1 : 2;
         P.tier[(size_t)g] = t;
         P.tier_count[t]++;
+        if (n > kCoverageKeys[2]) P.crowded.push_back((uint32_t)g);
     }
     P.ok = true;
 }

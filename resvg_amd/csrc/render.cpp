@@ -33,11 +33,10 @@ using namespace rvkr;
 namespace rvk {
 rvk_status launch_expand(rvk_context *ctx, const EdgeRec *edges, uint32_t nedges, const EdgeCov *cov,
                          PieceDev *pieces, uint32_t *npieces, int32_t *overflow, double algo_bytes);
-rvk_status launch_coverage(rvk_context *ctx, const CovJob *jobs, uint32_t njobs, const uint2 *bands128,
-                           uint32_t n128, const uint2 *bands256, uint32_t n256, const uint2 *bands512,
-                           uint32_t n512, const EdgeCov *edges, const uint2 *windows, const PieceDev *pieces,
-                           const uint32_t *npieces, uint16_t *table, uint8_t *arena, int32_t *overflow,
-                           double algo_bytes);
+rvk_status launch_coverage(rvk_context *ctx, const CovJob *jobs, const uint2 *const bands[rvkr::kBandLists],
+                           const uint64_t n_bands[rvkr::kBandLists], const EdgeCov *edges, const uint2 *windows,
+                           const PieceDev *pieces, const uint32_t *npieces, uint16_t *table, uint8_t *arena,
+                           int32_t *overflow, double algo_bytes);
 rvk_status launch_draw_items(rvk_context *ctx, uint8_t *target, uint32_t w, uint32_t h, int32_t x0, int32_t y0,
                              int32_t x1, int32_t y1, const DrawItem *items, const DrawCull *cull, uint32_t nitems,
                              const uint16_t *table, const uint8_t *arena, const ShaderParams *shaders,
@@ -78,7 +77,7 @@ struct DrawList {
     std::vector<HairPrep> hair;       // hairline strokes
     std::vector<ShaderParams> shaders;
     uint64_t n_edges = 0, n_windows = 0, piece_slots = 0;
-    uint64_t n_groups[3] = {0, 0, 0};  // bands per coverage kernel variant
+    uint64_t n_groups[kBandLists] = {};  // bands per coverage launch
     uint64_t n_table = 0;              // tile-table entries
     uint64_t n_hair_tiles = 0, n_hair_bins = 0, n_hair_lines = 0;
     uint64_t arena = 0;
@@ -354,7 +353,7 @@ struct Renderer {
         dl.n_windows += P.windows.size();
         P.piece_base = dl.piece_slots;
         dl.piece_slots += P.pieces;
-        for (int t = 0; t < 3; t++) dl.n_groups[t] += P.tier_count[t];
+        for (int t = 0; t < kBandLists; t++) dl.n_groups[t] += P.list_count(t);
         // the slot region holds every tile (at most one slot per tile and band); the
         // coverage kernel writes only the partial ones
         const uint64_t tiles = (uint64_t)j.tiles_x * j.tiles_y;
@@ -545,7 +544,7 @@ struct Renderer {
         return e && *e && *e != '0';
     }
     std::string validate_block(const DrawList &dl, const uint8_t *host, size_t o_jobs, size_t o_edges, size_t o_ecov,
-                               size_t o_win, const size_t o_grp[3], size_t o_ht, size_t o_hb) const {
+                               size_t o_win, const size_t o_grp[kBandLists], size_t o_ht, size_t o_hb) const {
         char buf[256];
         auto bad = [&](const char *what, uint64_t i, uint64_t v, uint64_t lim) {
             std::snprintf(buf, sizeof buf, "%s %llu: %llu not below %llu", what, (unsigned long long)i,
@@ -585,12 +584,14 @@ struct Renderer {
                 prev = e.piece_offset;
             }
         }
-        for (int t = 0; t < 3; t++) {
+        for (int t = 0; t < kBandLists; t++) {
             const uint2 *b = (const uint2 *)(host + o_grp[t]);
             for (uint64_t k = 0; k < dl.n_groups[t]; k++) {
                 if (b[k].x >= njobs) return bad("band job", k, b[k].x, njobs);
                 if (b[k].y >= jobs[b[k].x].tiles_y) return bad("band index", k, b[k].y, jobs[b[k].x].tiles_y);
-                if (dl.jobs[b[k].x].tier[b[k].y] != t) return bad("band tier", k, dl.jobs[b[k].x].tier[b[k].y], t);
+                const JobPrep &P = dl.jobs[b[k].x];
+                const bool crowded = std::binary_search(P.crowded.begin(), P.crowded.end(), b[k].y);
+                if (P.tier[b[k].y] != std::min(t, 2) || crowded != (t == 3)) return bad("band tier", k, P.tier[b[k].y], t);
             }
         }
         const uint32_t *ht = (const uint32_t *)(host + o_ht);
@@ -661,11 +662,11 @@ struct Renderer {
         const size_t o_ht = al(o_cull + nitems * sizeof(DrawCull));
         const size_t o_hb = al(o_ht + dl.n_hair_tiles * 4);
         const size_t o_hl = al(o_hb + dl.n_hair_bins * 4);
-        size_t o_grp[3];
-        o_grp[0] = al(o_hl + dl.n_hair_lines * sizeof(HairLine));
-        o_grp[1] = al(o_grp[0] + dl.n_groups[0] * sizeof(uint2));
-        o_grp[2] = al(o_grp[1] + dl.n_groups[1] * sizeof(uint2));
-        const size_t meta = al(o_grp[2] + dl.n_groups[2] * sizeof(uint2));
+        size_t o_grp[kBandLists], meta = al(o_hl + dl.n_hair_lines * sizeof(HairLine));
+        for (int t = 0; t < kBandLists; t++) {
+            o_grp[t] = meta;
+            meta = al(meta + dl.n_groups[t] * sizeof(uint2));
+        }
         const size_t o_np = meta;
         const size_t o_pc = al(o_np + dl.n_edges * 4);
         const size_t o_tab = al(o_pc + (size_t)dl.piece_slots * sizeof(PieceDev));
@@ -695,13 +696,13 @@ struct Renderer {
             }
         }
         // each job's first entry in the band lists
-        std::vector<uint64_t> gbase(njobs * 3);
+        std::vector<uint64_t> gbase(njobs * kBandLists);
         {
-            uint64_t run[3] = {0, 0, 0};
+            uint64_t run[kBandLists] = {};
             for (size_t i = 0; i < njobs; i++)
-                for (int t = 0; t < 3; t++) {
-                    gbase[i * 3 + t] = run[t];
-                    run[t] += dl.jobs[i].tier_count[t];
+                for (int t = 0; t < kBandLists; t++) {
+                    gbase[i * kBandLists + t] = run[t];
+                    run[t] += dl.jobs[i].list_count(t);
                 }
         }
         auto pack = [&](size_t i) {
@@ -723,9 +724,10 @@ struct Renderer {
                 if (!P.windows.empty())
                     std::memcpy((uint2 *)(host + o_win) + j.window_offset, P.windows.data(),
                                 P.windows.size() * sizeof(uint2));
-                uint2 *gl[3];
-                for (int t = 0; t < 3; t++) gl[t] = (uint2 *)(host + o_grp[t]) + gbase[i * 3 + t];
-                for (size_t g = 0; g < P.tier.size(); g++) *gl[P.tier[g]]++ = uint2{(uint32_t)i, (uint32_t)g};
+                uint2 *gl[kBandLists];
+                for (int t = 0; t < kBandLists; t++) gl[t] = (uint2 *)(host + o_grp[t]) + gbase[i * kBandLists + t];
+                size_t c = 0;
+                for (size_t g = 0; g < P.tier.size(); g++) *gl[P.band_list(g, c)]++ = uint2{(uint32_t)i, (uint32_t)g};
             } else {
                 const size_t k = i - njobs;
                 const HairPrep &P = dl.hair[k];
@@ -808,14 +810,14 @@ struct Renderer {
                 st = rvk::launch_expand(ctx, (const EdgeRec *)(d + o_edges), (uint32_t)dl.n_edges,
                                         (const EdgeCov *)(d + o_ecov), (PieceDev *)(d + o_pc),
                                         (uint32_t *)(d + o_np), dev_overflow, exp_bytes);
-            if (st == RVK_OK)
-                st = rvk::launch_coverage(ctx, (const CovJob *)(d + o_jobs), (uint32_t)njobs,
-                                          (const uint2 *)(d + o_grp[0]), (uint32_t)dl.n_groups[0],
-                                          (const uint2 *)(d + o_grp[1]), (uint32_t)dl.n_groups[1],
-                                          (const uint2 *)(d + o_grp[2]), (uint32_t)dl.n_groups[2],
+            if (st == RVK_OK) {
+                const uint2 *bands[kBandLists];
+                for (int t = 0; t < kBandLists; t++) bands[t] = (const uint2 *)(d + o_grp[t]);
+                st = rvk::launch_coverage(ctx, (const CovJob *)(d + o_jobs), bands, dl.n_groups,
                                           (const EdgeCov *)(d + o_ecov), (const uint2 *)(d + o_win),
                                           (const PieceDev *)(d + o_pc), (const uint32_t *)(d + o_np),
                                           (uint16_t *)(d + o_tab), d + o_arena, dev_overflow, cov_bytes);
+            }
             ctx->stream = main_stream;
         }
         if (st == RVK_OK && side != ctx->stream &&

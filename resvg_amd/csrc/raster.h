@@ -57,6 +57,7 @@ constexpr uint32_t kMaxTilesX = 65279u;  // widest job grid (a u16 table entry a
 // of its own, so a flush has one list of bands per variant and one of the crowded ones
 constexpr uint32_t kCoverageKeys[3] = {128, 256, 512};
 constexpr int kBandLists = 4;
+constexpr uint32_t kMaxSortedEdges = 1u << 22;  // edges of a job whose ids fit the variants' sort keys
 
 // A coverage job computes u8 coverage for the pixel rect [x0, x0+w) x [y0, y0+h)
 // of its pixmap (coordinates of the edge space; coverage is 0 outside the rect).

@@ -21,6 +21,7 @@
 // entry -> coverage -> gradient or solid shade (tiny-skia lowp stages) -> SourceOver
 // into the target (direct items) or into an elided layer pixel that is then
 // composited in f32 with the group's opacity and blend mode (draw_pixmap semantics).
+#include <type_traits>
 #include "rvk_internal.h"
 #include "blend_ops.h"
 #include "raster.h"
@@ -312,81 +313,149 @@ static_assert(rvkr::kMaxTilesX + kStatePartial <= 65536u, "a partial tile's stat
 static_assert(kWin == 8 * kWave, "a lane holds one 8-pixel tile row of a window");
 
 // ---- coverage of a band, one wave per pixel row ----
-// A sub-scanline's crossings, each lane's J of them in v[s] (element lane * J + j,
-// ~0 for none), sorted ascending; n[s] of them are real.  Writes the span events
-// (pixel-rounded supersampled columns; starts and ends alternate) to ev[s] and returns
-// their count.  Every real crossing changes the winding by one, so with U upward
-// crossings before element e the winding there is 2 U - e, and ballots give every
-// prefix; under the even-odd rule every crossing is an event.
 constexpr int32_t kOpenEnd = 0x3fffffff;  // the end of a span that its sub-scanline leaves open
+constexpr int kSettlePasses = 6;          // exchanges of neighbours tried before a full sort
 
-template <int J>
-__device__ __forceinline__ int row_events(const uint64_t (&v)[J], int n, bool evenodd, int32_t *ev, int lane) {
-    int32_t x[J];
-#pragma unroll
-    for (int j = 0; j < J; j++)
-        x[j] = ((int32_t)((uint32_t)(v[j] >> 32) ^ 0x80000000u) + 0x8000) >> 16;
-    if (evenodd) {
-#pragma unroll
-        for (int j = 0; j < J; j++)
-            if (lane * J + j < n) ev[lane * J + j] = x[j];
-        if (n & 1) {
-            if (lane == 0) ev[n] = kOpenEnd;
-            return n + 1;
-        }
-        return n;
-    }
-    bool up[J];
-    int before = -lane * J;  // the winding before this lane's first element
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        up[j] = lane * J + j < n && (v[j] & 1) != 0;
-        before += 2 * lanes_below(__ballot(up[j]));
-    }
-    bool evt[J];
-    int pos = 0, total = 0;
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        const int after = before + (up[j] ? 1 : -1);
-        evt[j] = lane * J + j < n && (before == 0 || after == 0);
-        before = after;
-        const uint64_t m = __ballot(evt[j]);
-        pos += lanes_below(m);
-        total += __popcll(m);
-    }
-#pragma unroll
-    for (int j = 0; j < J; j++)
-        if (evt[j]) ev[pos++] = x[j];
-    if (total & 1) {
-        if (lane == 0) ev[total] = kOpenEnd;
-        total++;
-    }
-    return total;
+// The low word of an edge's key: its id (orders equal x), its slot in the band's list and
+// its direction (1: downwards).  The host keeps jobs of more than 2^22 edges out of
+// k_coverage, whose slots fit 9 bits.
+__device__ __forceinline__ uint32_t edge_low(int32_t id, int slot, int32_t winding) {
+    return ((uint32_t)id << 10) | ((uint32_t)slot << 1) | (winding > 0 ? 1u : 0u);
+}
+__device__ __forceinline__ int low_slot(uint32_t lo) { return (int)((lo >> 1) & 511u); }
+__device__ __forceinline__ uint64_t edge_key(int32_t x, uint32_t lo) {
+    return ((uint64_t)((uint32_t)x ^ 0x80000000u) << 32) | lo;
 }
 
-// The span events of one row's sub-scanlines from the crossings in ev (element e's
-// sub-scanlines in bits shift .. shift + 3 of act[e], its id and direction in meta[e]),
-// which they replace; the event counts in nev.
+// A key of the next lane (~0 past the last) and of the one before (0 before the first).
+__device__ __forceinline__ uint64_t next_lane(uint64_t v) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)(uint32_t)v, 0x130, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)(uint32_t)(v >> 32), 0x130, 0xf, 0xf, false);
+    return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ uint64_t prev_lane(uint64_t v) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, 0x138, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), 0x138, 0xf, 0xf, false);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// Sorts 64 J keys (element lane * J + j in v[0][j]) that are nearly in order: neighbours
+// are exchanged until none is out of order, or the full network sorts them after
+// kSettlePasses rounds.
+template <int J>
+__device__ __forceinline__ void settle(uint64_t (&v)[1][J], int lane) {
+    uint64_t(&u)[J] = v[0];
+    auto order = [&](int a, int b) {
+        const bool sw = u[a] > u[b];
+        const uint64_t x = sw ? u[b] : u[a];
+        u[b] = sw ? u[a] : u[b];
+        u[a] = x;
+    };
+    for (int pass = 0;; pass++) {
+        bool bad = u[J - 1] > next_lane(u[0]);
+#pragma unroll
+        for (int j = 0; j + 1 < J; j++) bad = bad || u[j] > u[j + 1];
+        if (__ballot(bad) == 0) return;
+        if (pass == kSettlePasses) break;
+        if constexpr (J == 1) {
+            // lanes 2 i, 2 i + 1, then 2 i + 1, 2 i + 2
+#pragma unroll
+            for (int odd = 0; odd < 2; odd++) {
+                const uint64_t up = next_lane(u[0]), down = prev_lane(u[0]);
+                if ((lane & 1) == odd) u[0] = up < u[0] ? up : u[0];
+                else u[0] = down > u[0] ? down : u[0];
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j + 1 < J; j += 2) order(j, j + 1);
+#pragma unroll
+            for (int j = 1; j + 1 < J; j += 2) order(j, j + 1);
+            const uint64_t up = next_lane(u[0]), down = prev_lane(u[J - 1]);
+            u[J - 1] = up < u[J - 1] ? up : u[J - 1];
+            u[0] = down > u[0] ? down : u[0];
+        }
+    }
+    bitonic_from<J, 1, 2, 1>(v, lane);
+}
+
+// The span events of one row's sub-scanlines (pixel-rounded supersampled columns; starts
+// and ends alternate) and their counts in nev.  ev[s][slot] holds the x of the band's edge
+// `slot` on sub-scanline s, and is replaced by the events; bit shift + s of act[slot] says
+// that the edge crosses it (where it does not, x is that of its nearer end, so the order
+// stays the same from one sub-scanline to the next); ord holds the edges' low words in the
+// order of their x in the middle of the band.
+// Each sub-scanline starts from the order of the one before it, which is nearly always
+// its own: of the full sorts that took 1300 of 2100 VALU instructions a row (128 edges;
+// 8000 of 9000 with 512), a check or a few exchanges of neighbours remain.
+// Every crossing changes the winding by one, so with U downward crossings among the A
+// before an element the winding there is 2 U - A, and ballots give every prefix; under
+// the even-odd rule every crossing is an event.
 template <int J, int STRIDE>
-__device__ __forceinline__ void sort_row(int32_t (*ev)[STRIDE], const uint32_t *act, int shift, const uint32_t *meta,
-                                         int nact, bool evenodd, int *nev, int lane) {
-    uint64_t v[kMaxSub][J];
-    int cnt[kMaxSub] = {0, 0, 0, 0};
+__device__ __forceinline__ void row_spans(int32_t (*ev)[STRIDE], const uint32_t *act, int shift, const uint32_t *ord,
+                                          int nact, int nsub, bool evenodd, int *nev, int lane) {
+    uint32_t lo[J];
+    bool off = false, on_any = false;
 #pragma unroll
     for (int j = 0; j < J; j++) {
         const int e = lane * J + j;
-        const uint32_t bits = e < nact ? act[e] >> shift : 0u;
-        const uint32_t lo = e < nact ? meta[e] : 0u;
-#pragma unroll
-        for (int s = 0; s < kMaxSub; s++) {
-            const bool on = (bits >> s) & 1u;
-            v[s][j] = on ? ((uint64_t)((uint32_t)ev[s][e] ^ 0x80000000u) << 32) | lo : ~0ull;
-            cnt[s] += __popcll(__ballot(on));
-        }
+        lo[j] = ord[e < nact ? e : 0];
+        const uint32_t bits = (act[low_slot(lo[j])] >> shift) & 15u;
+        off = off || (e < nact && bits != (nsub == 1 ? 1u : 15u));
+        on_any = on_any || (e < nact && bits != 0);
     }
-    if (cnt[0] + cnt[1] + cnt[2] + cnt[3] != 0) bitonic_from<J, kMaxSub, 2, 1>(v, lane);
+    const bool all = __ballot(off) == 0;  // every edge crosses every sub-scanline of the row
+    if (__ballot(on_any) == 0) return;
 #pragma unroll
-    for (int s = 0; s < kMaxSub; s++) nev[s] = row_events<J>(v[s], cnt[s], evenodd, ev[s], lane);
+    for (int s = 0; s < kMaxSub; s++) {
+        if (s >= nsub) break;
+        uint64_t v[1][J];
+#pragma unroll
+        for (int j = 0; j < J; j++)
+            v[0][j] = lane * J + j < nact ? edge_key(ev[s][low_slot(lo[j])], lo[j]) : ~0ull;
+        settle<J>(v, lane);
+        bool on[J], up[J];
+        int32_t x[J];
+        int below = 0, before = 0;
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const bool real = lane * J + j < nact;
+            x[j] = ((int32_t)((uint32_t)(v[0][j] >> 32) ^ 0x80000000u) + 0x8000) >> 16;
+            if (real) lo[j] = (uint32_t)v[0][j];
+            on[j] = real && (all || ((act[low_slot(lo[j])] >> (shift + s)) & 1u) != 0);
+            up[j] = on[j] && (lo[j] & 1u) != 0;
+            below += lanes_below(__ballot(on[j]));
+            before += 2 * lanes_below(__ballot(up[j]));
+        }
+        before -= below;
+        int pos = 0, total = 0;
+        bool evt[J];
+        if (evenodd) {
+            pos = below;
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                evt[j] = on[j];
+                total += __popcll(__ballot(on[j]));
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                const int after = before + (up[j] ? 1 : -1);
+                evt[j] = on[j] && (before == 0 || after == 0);
+                before = on[j] ? after : before;
+                const uint64_t m = __ballot(evt[j]);
+                pos += lanes_below(m);
+                total += __popcll(m);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < J; j++)
+            if (evt[j]) ev[s][pos++] = x[j];
+        if (total & 1) {
+            if (lane == 0) ev[s][total] = kOpenEnd;
+            total++;
+        }
+        nev[s] = total;
+    }
 }
 
 constexpr int kRowWaves = rvkr::kBandRows;        // waves of a block: one per pixel row of the band
@@ -427,8 +496,8 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_coverage(CovArgs a) {
     constexpr int kStride = MK + 4;        // a row of crossings, and its events with an open end
     __shared__ __align__(16) int32_t xs[rvkr::kBandRows * kMaxSub][kStride];
     __shared__ uint32_t act[PARTS][MK];    // bits (row in the part) * 4 + sub-scanline
-    __shared__ uint32_t meta[MK];          // id << 1 | upward
-    __shared__ uint32_t list[MK];
+    __shared__ uint32_t meta[MK];          // low words by slot
+    __shared__ uint32_t list[MK];          // edges by slot, then the low words in x order
     __shared__ __align__(16) uint32_t acc[kRowWaves][kAccWords];
     __shared__ int wcount[kRowWaves];
     __shared__ __align__(16) uint64_t masks[3][2];  // tiles of the window that are 0 / 255 in every row so far
@@ -484,41 +553,65 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_coverage(CovArgs a) {
             const int32_t y0 = row0 + part * J;
             const int32_t s0 = max(y0, ry0) << shift, s1 = min(y0 + J, ry1) << shift;
             uint32_t bits = 0;
-            if (part == 0) meta[slot] = ((uint32_t)e.id << 1) | (e.winding > 0 ? 1u : 0u);
-            if (e.first_y < s1 && e.ymax >= s0) {
+            if (part == 0) meta[slot] = edge_low(e.id, slot, e.winding);
+            if (s0 < s1) {
                 uint32_t k = 0;
-                if (e.first_y < s0) {  // the first piece that reaches s0
-                    uint32_t hi = n;
+                if (e.first_y < s0) {  // the first piece that reaches s0, or the last one
+                    uint32_t hi = n - 1;
                     while (k < hi) {
                         const uint32_t mid = (k + hi) >> 1;
                         if (pc[mid].last_y < s0) k = mid + 1;
                         else hi = mid;
                     }
                 }
-                if (k < n) {
-                    PieceDev p = pc[k];
-                    for (int32_t sy = s0; sy < s1; sy++) {
-                        while (p.last_y < sy && k + 1 < n) p = pc[++k];
-                        if (p.first_y <= sy && p.last_y >= sy) {
-                            const int32_t y = sy >> shift, s = sy - (y << shift);
-                            xs[(y - row0) * kMaxSub + s][slot] =
-                                (int32_t)((uint32_t)p.x + (uint32_t)(sy - p.first_y) * (uint32_t)p.dx);
-                            bits |= 1u << ((y - y0) * kMaxSub + s);
-                        }
-                    }
+                PieceDev p = pc[k];
+                for (int32_t sy = s0; sy < s1; sy++) {
+                    while (p.last_y < sy && k + 1 < n) p = pc[++k];
+                    const int32_t y = sy >> shift, s = sy - (y << shift);
+                    const int32_t at = min(max(sy, p.first_y), p.last_y);
+                    xs[(y - row0) * kMaxSub + s][slot] =
+                        (int32_t)((uint32_t)p.x + (uint32_t)(at - p.first_y) * (uint32_t)p.dx);
+                    if (at == sy) bits |= 1u << ((y - y0) * kMaxSub + s);
                 }
             }
             act[part][slot] = bits;
         }
     }
     __syncthreads();
+    // ---- their order in the middle of the band ----
+    if (r == 0 && nact > 0) {
+        const int32_t sm = (sb0 + sb1) >> 1, ym = sm >> shift;
+        const int32_t *xm = xs[(ym - row0) * kMaxSub + (sm - (ym << shift))];
+        auto sort_slots = [&](auto &v, auto jc) {
+            constexpr int JJ = decltype(jc)::value;
+#pragma unroll
+            for (int j = 0; j < JJ; j++) {
+                const int e = lane * JJ + j;
+                v[0][j] = e < nact ? edge_key(xm[e], meta[e]) : ~0ull;
+            }
+            bitonic_from<JJ, 1, 2, 1>(v, lane);
+#pragma unroll
+            for (int j = 0; j < JJ; j++)
+                if (lane * JJ + j < nact) list[lane * JJ + j] = (uint32_t)v[0][j];
+        };
+        if (J > 1 && nact <= kWave) {
+            uint64_t v[1][1];
+            sort_slots(v, std::integral_constant<int, 1>());
+        } else {
+            uint64_t v[1][J];
+            sort_slots(v, std::integral_constant<int, J>());
+        }
+    }
+    __syncthreads();
     // ---- this row's span events ----
     int32_t(*ev)[kStride] = &xs[r * kMaxSub];
-    int nev[kMaxSub];
-    if (J > 1 && nact <= kWave)
-        sort_row<1>(ev, act[r / J], r % J * kMaxSub, meta, nact, evenodd, nev, lane);
-    else
-        sort_row<J>(ev, act[r / J], r % J * kMaxSub, meta, nact, evenodd, nev, lane);
+    int nev[kMaxSub] = {0, 0, 0, 0};
+    if (nact > 0 && row0 + r >= ry0 && row0 + r < ry1) {
+        if (J > 1 && nact <= kWave)
+            row_spans<1>(ev, act[r / J], r % J * kMaxSub, list, nact, nsub, evenodd, nev, lane);
+        else
+            row_spans<J>(ev, act[r / J], r % J * kMaxSub, list, nact, nsub, evenodd, nev, lane);
+    }
     // ---- windows ----
     const int sl = lane >> 4;  // lanes 16 s .. 16 s + 15 look at sub-scanline s's spans
     const int nspl = (sl < 2 ? (sl == 0 ? nev[0] : nev[1]) : (sl == 2 ? nev[2] : nev[3])) >> 1;

@@ -1006,10 +1006,11 @@ void prep_job(const EdgeSet &es, uint32_t rule, bool aa, IRect clip, int32_t lx,
     for (int32_t g = 0, run = 0; g < bands; g++) {
         run += diff[g];
         const uint32_t n = (uint32_t)run;
-        const uint8_t t = n <= kCoverageKeys[0] ? 0 : n <= kCoverageKeys[1] ? 1 : 2;
+        const bool crowded = n > kCoverageKeys[2] || j.edge_count > kMaxSortedEdges;
+        const uint8_t t = crowded ? 2 : n <= kCoverageKeys[0] ? 0 : n <= kCoverageKeys[1] ? 1 : 2;
         P.tier[(size_t)g] = t;
         P.tier_count[t]++;
-        if (n > kCoverageKeys[2]) P.crowded.push_back((uint32_t)g);
+        if (crowded) P.crowded.push_back((uint32_t)g);
     }
     P.ok = true;
 }

@@ -459,7 +459,7 @@ __device__ __forceinline__ void row_spans(int32_t (*ev)[STRIDE], const uint32_t 
 }
 
 constexpr int kRowWaves = rvkr::kBandRows;        // waves of a block: one per pixel row of the band
-constexpr int kAccWords = kWin / 2 + 4;           // a window's pixel differences, two per word, and their spill
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 // MK: edges that the band holds (128, 256 or 512).  The host sends a band to the
 // smallest variant that holds the edges whose rows meet it.
@@ -472,10 +472,10 @@ constexpr int kAccWords = kWin / 2 + 4;           // a window's pixel difference
 // * Each wave sorts its row's sub-scanlines (a bitonic network over 64 J keys held in
 //   registers, exchanged in the VALU) and turns them into span events, which take the
 //   crossings' place in LDS.
-// * Per 512-pixel window a wave adds its spans' coverage as differences (16 bit, two
-//   pixels a word, exact modulo 2^32), each lane prefix-sums one 8-pixel tile row, and the
-//   waves agree on which of the window's 64 tiles are all 0, all 255 or partial through
-//   two 64-bit masks; each writes its row of the partial tiles.
+// * Per 512- or 1024-pixel window a wave adds its spans' coverage as differences (16 bit,
+//   two pixels a word, exact modulo 2^32), each lane prefix-sums one or two 8-pixel tile
+//   rows, and the waves agree on which of the window's tiles are all 0, all 255 or partial
+//   through 64-bit masks; each writes its row of the partial tiles.
 // Windows alternate between three mask slots, so one barrier a window is enough.
 //
 // Why a wave per row: a row's work is a chain of dependent steps (piece loads, sort
@@ -493,6 +493,11 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_coverage(CovArgs a) {
     constexpr int PARTS = rvkr::kBandRows / J;
     constexpr int kThreads = kRowWaves * kWave;
     static_assert(PARTS * MK == kThreads, "a thread per edge and J rows");
+    // tiles per lane of a window: 1024 pixels (a fifth fewer instructions a row), or 512
+    // where the larger accumulators would cost a block per CU (256: 23% slower with 1024)
+    constexpr int T = MK <= 128 ? 2 : 1;
+    constexpr int32_t kRowWin = rvkr::kTile * kWave * T;
+    constexpr int kAccWords = kRowWin / 2 + 4;  // a window's pixel differences, two per word, and their spill
     constexpr int kStride = MK + 4;        // a row of crossings, and its events with an open end
     __shared__ __align__(16) int32_t xs[rvkr::kBandRows * kMaxSub][kStride];
     __shared__ uint32_t act[PARTS][MK];    // bits (row in the part) * 4 + sub-scanline
@@ -500,7 +505,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_coverage(CovArgs a) {
     __shared__ uint32_t list[MK];          // edges by slot, then the low words in x order
     __shared__ __align__(16) uint32_t acc[kRowWaves][kAccWords];
     __shared__ int wcount[kRowWaves];
-    __shared__ __align__(16) uint64_t masks[3][2];  // tiles of the window that are 0 / 255 in every row so far
+    __shared__ __align__(16) uint64_t masks[3][2 * T];  // tiles of the window that are 0 / 255 in every row so far
     const int tid = threadIdx.x, lane = tid % kWave;
     const int r = __builtin_amdgcn_readfirstlane(tid / kWave);
     const uint2 bj = a.bands[blockIdx.x];
@@ -516,7 +521,7 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_coverage(CovArgs a) {
     const int32_t sb0 = ry0 << shift, sb1 = (ry1 << shift) - 1;  // covered sub-scanlines
     const uint2 win = a.windows[job.window_offset + band];
     for (int i = tid; i < kRowWaves * kAccWords; i += kThreads) (&acc[0][0])[i] = 0;
-    if (tid < 6) masks[tid / 2][tid % 2] = ~0ull;
+    if (tid < 6 * T) masks[tid / (2 * T)][tid % (2 * T)] = ~0ull;
     int nact = 0;
     for (uint32_t base = win.x; base < win.y; base += kThreads) {
         const uint32_t i = base + (uint32_t)tid;
@@ -626,10 +631,10 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_coverage(CovArgs a) {
     uint32_t nslots = 0;  // partial tiles of the band so far
     int kst = 0;          // the first span of this lane's sub-scanline not behind the windows
     int mslot = 0, wi = 0;
-    for (int32_t wx0 = 0; wx0 < cw; wx0 += kWin, wi++) {
-        const int32_t ww = min(kWin, cw - wx0);  // a multiple of kTile
+    for (int32_t wx0 = 0; wx0 < cw; wx0 += kRowWin, wi++) {
+        const int32_t ww = min(kRowWin, cw - wx0);  // a multiple of kTile
         const int32_t wabs = job.gx0 + wx0;
-        uint32_t w0 = 0, w1 = 0;
+        uint32_t w[2 * T] = {};  // this lane's tile rows, 8 bytes each
         if (any) {
             // spans cut to the window and to the job's columns (coverage is 0 outside)
             const int32_t colbase = wabs << shift, wend = colbase + (ww << shift);
@@ -679,44 +684,77 @@ __global__ __launch_bounds__(kRowWaves * kWave) void k_coverage(CovArgs a) {
                 kst += __popc(done);
                 live = done == 0xffffu;
             } while (__ballot(live) != 0);
-            // ---- prefix sum: lane l holds pixels [8 l, 8 l + 8), one tile row; the
+            // ---- prefix sum: lane l holds pixels [8 T l, 8 T (l + 1)), T tile rows; the
             // accumulator is cleared behind the read ----
-            uint4 q = *reinterpret_cast<const uint4 *>(&wacc[4 * lane]);
-            *reinterpret_cast<uint4 *>(&wacc[4 * lane]) = make_uint4(0, 0, 0, 0);
-            if (lane == 0) wacc[kWin / 2] = 0;
+            uint32_t q[4 * T];
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                uint4 *at = reinterpret_cast<uint4 *>(&wacc[4 * (T * lane + t)]);
+                const uint4 u = *at;
+                *at = make_uint4(0, 0, 0, 0);
+                q[4 * t] = u.x;
+                q[4 * t + 1] = u.y;
+                q[4 * t + 2] = u.z;
+                q[4 * t + 3] = u.w;
+            }
+            if (lane == 0) wacc[kRowWin / 2] = 0;
             // a word is lo + 65536 hi of two signed differences, so the words' sum is the
             // sums of both, and word * 65537 the running pair
-            const uint32_t sum = q.x + q.y + q.z + q.w;
+            uint32_t sum = 0;
+#pragma unroll
+            for (int i = 0; i < 4 * T; i++) sum += q[i];
             const int32_t slo = (int32_t)(int16_t)sum;
             const int32_t loc = slo + ((int32_t)(sum - (uint32_t)slo) >> 16);
-            const uint32_t run = (uint32_t)(wave_incl_scan(loc) - loc);
-            auto pair = [](uint32_t before, uint32_t w) { return (before << 16) + before + (w << 16) + w; };
-            const uint32_t p0 = pair(run, q.x), p1 = pair(p0 >> 16, q.y), p2 = pair(p1 >> 16, q.z),
-                           p3 = pair(p2 >> 16, q.w);
+            uint32_t before = (uint32_t)(wave_incl_scan(loc) - loc) << 16;  // the pixel before, in the high half
+#pragma unroll
+            for (int i = 0; i < 4 * T; i++) {
+                before = (q[i] << 16) + __builtin_amdgcn_perm(before, before, 0x03020302u) + q[i];
+                q[i] = before;
+            }
             // each field is a pixel's coverage, at most 256: 256 becomes 255
-            auto clamp2 = [](uint32_t p) { return p - ((p >> 8) & 0x00010001u); };
-            w0 = __builtin_amdgcn_perm(clamp2(p1), clamp2(p0), 0x06040200u);
-            w1 = __builtin_amdgcn_perm(clamp2(p3), clamp2(p2), 0x06040200u);
+            auto clamp2 = [](uint32_t p) {
+                const u16x2 c = {255, 255};
+                return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, p), c));
+            };
+#pragma unroll
+            for (int i = 0; i < 2 * T; i++)
+                w[i] = __builtin_amdgcn_perm(clamp2(q[2 * i + 1]), clamp2(q[2 * i]), 0x06040200u);
         }
-        // ---- the window's tiles ----
-        const bool valid = 8 * lane < ww;
-        const uint64_t mz = __ballot(!valid || (w0 | w1) == 0u), mf = __ballot(valid && (w0 & w1) == ~0u);
-        if (lane == 0) {
-            atomicAnd((unsigned long long *)&masks[mslot][0], (unsigned long long)mz);
-            atomicAnd((unsigned long long *)&masks[mslot][1], (unsigned long long)mf);
+        // ---- the window's tiles: T masks (tile T l + t in bit l of mask t) ----
+        uint64_t mz[T], mf[T];
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            const bool valid = 8 * (T * lane + t) < ww;
+            mz[t] = __ballot(!valid || (w[2 * t] | w[2 * t + 1]) == 0u);
+            mf[t] = __ballot(valid && (w[2 * t] & w[2 * t + 1]) == ~0u);
+        }
+        if (lane < 2 * T) {
+            uint64_t m = lane & 1 ? mf[0] : mz[0];
+            if (T > 1 && lane >= 2) m = lane & 1 ? mf[T - 1] : mz[T - 1];
+            atomicAnd((unsigned long long *)&masks[mslot][lane], (unsigned long long)m);
         }
         const int next = mslot == 2 ? 0 : mslot + 1;
-        if (tid < 2) masks[next][tid] = ~0ull;  // last read before the previous barrier
+        if (tid < 2 * T) masks[next][tid] = ~0ull;  // last read before the previous barrier
         __syncthreads();
-        const uint64_t zero = masks[mslot][0], full = masks[mslot][1];
-        const uint64_t part = ~(zero | full);
-        const uint32_t k = nslots + (uint32_t)lanes_below(part);
-        const bool mine = (part >> lane) & 1ull;
-        if (mine) *reinterpret_cast<uint2 *>(slots + (size_t)k * 64u + r * 8) = make_uint2(w0, w1);
-        if (r == (wi & (kRowWaves - 1)) && valid)
-            tab[wx0 / rvkr::kTile + lane] = (uint16_t)(mine ? rvkr::kTileSlot0 + k
-                                                            : ((zero >> lane) & 1ull ? rvkr::kTileEmpty : rvkr::kTileFull));
-        nslots += (uint32_t)__popcll(part);
+        uint64_t part[T];
+        uint32_t k = nslots;
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            mz[t] = masks[mslot][2 * t];
+            part[t] = ~(mz[t] | masks[mslot][2 * t + 1]);
+            k += (uint32_t)lanes_below(part[t]);
+            nslots += (uint32_t)__popcll(part[t]);
+        }
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            const bool mine = (part[t] >> lane) & 1ull;
+            if (mine) *reinterpret_cast<uint2 *>(slots + (size_t)k * 64u + r * 8) = make_uint2(w[2 * t], w[2 * t + 1]);
+            if (r == ((T * wi + t) & (kRowWaves - 1)) && 8 * (T * lane + t) < ww)
+                tab[wx0 / rvkr::kTile + T * lane + t] =
+                    (uint16_t)(mine ? rvkr::kTileSlot0 + k
+                                    : ((mz[t] >> lane) & 1ull ? rvkr::kTileEmpty : rvkr::kTileFull));
+            k += mine ? 1u : 0u;
+        }
         mslot = next;
     }
 }

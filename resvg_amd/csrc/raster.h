@@ -147,7 +147,7 @@ constexpr uint32_t kModeKind = 3u, kModeRadial = 1u << 2, kModeSpreadShift = 3, 
                    kModeTwoStop = 1u << 6, kModeOpaque = 1u << 7, kModeRTwist = 1u << 8, kModeAsSource = 1u << 9,
                    kModeClear = 1u << 10, kModeF32 = 1u << 11, kModeStopsShift = 16;
 struct ShaderParams : ShaderHead {
-    float t[kMaxStops + 2];
+    float t[kMaxStops + 5];  // thresholds; NaN past the last stop (seal_shader), read in fours from t[1]
     float f[kMaxStops + 2][4];
     float b[kMaxStops + 2][4];
 };
@@ -178,9 +178,14 @@ struct DrawItem {
     float opacity;
     uint32_t blend_mode;
     uint32_t stroke_hair;       // 1: stroke_job is a hairline job
-    uint32_t pad_;
+    uint32_t mode;              // kItem* bits, set once the list is complete (flush)
+    float flx, fly;             // lx, ly
     JobRef fj, sj;              // the fill and stroke jobs
 };
+// DrawItem::mode.  Plain: fill and stroke by tiles (no hairline), both shaders of the u8
+// pipeline (not Clear), drawn directly or through a layer with SourceOver and an opacity
+// in [0, 1]; Scaled: that opacity is not 1.
+constexpr uint32_t kItemPlain = 1, kItemLayer = 2, kItemStrokeFirst = 4, kItemScaled = 8;
 
 // What the compositor's culling pass reads of an item, one lane per item: its target
 // rect in tiles and the two jobs' tile grids and tables.
@@ -221,8 +226,9 @@ void hairline_lines(const rvk_scene &sc, const rvk_path &path, rvkh::Ts ts, uint
                     std::vector<HairLine> &out);
 // tiny-skia shader setup; false when the paint draws nothing.  `extra_opacity`
 // scales the colour's or every stop's alpha (Shader::apply_opacity).
-// Packs the branch fields of a complete shader into its mode word.
-void seal_shader(ShaderHead &s);
+// Packs the branch fields of a complete shader into its mode word and ends its thresholds
+// with NaN.
+void seal_shader(ShaderParams &s);
 bool make_shader(const rvk_scene &sc, const rvk_paint &paint, rvkh::Ts ts, ShaderParams &out,
                  float extra_opacity = 1.0f);
 // render_pattern_pixmap's tile for a pattern paint drawn with `ts` (path.rs:179-205):

@@ -1163,15 +1163,13 @@ __device__ __forceinline__ void grad_color(const ShaderParams &sp, uint32_t m, f
     if (m & rvkr::kModeTwoStop) {
         for (int k = 0; k < 4; k++) c[k] = t * sp.f[0][k] + sp.b[0][k];
     } else {
-        // the thresholds are read four at a time (t has kMaxStops + 2 entries)
+        // the thresholds are read four at a time; those past the last stop are NaN, which
+        // no t reaches
         const uint32_t nstops = m >> rvkr::kModeStopsShift;
         uint32_t idx = 0;
         for (uint32_t i = 1; i < nstops; i += 4) {
-            float q[4];
 #pragma unroll
-            for (int k = 0; k < 4; k++) q[k] = sp.t[min(i + (uint32_t)k, (uint32_t)kMaxStops + 1u)];
-#pragma unroll
-            for (int k = 0; k < 4; k++) idx += i + (uint32_t)k < nstops && t >= q[k] ? 1u : 0u;
+            for (uint32_t k = 0; k < 4; k++) idx += t >= sp.t[i + k] ? 1u : 0u;
         }
         for (int k = 0; k < 4; k++) c[k] = t * sp.f[idx][k] + sp.b[idx][k];
     }
@@ -1315,6 +1313,68 @@ __device__ __forceinline__ uint32_t over_lowp(uint32_t src, uint32_t cov, uint32
     return src + scale_px(d, 255u - (src >> 24));
 }
 
+// ---- the same arithmetic on pixels held as four floats with whole values 0 .. 255 ----
+// Products of two such values plus 255 stay below 2^24, so fma and the division by 256
+// are exact and floor((v + 255) / 256) is div255(v); nothing is converted or packed
+// between one draw item and the next.
+__device__ __forceinline__ F4 px_floats(uint32_t p) {
+    return F4{(float)ch(p, 0), (float)ch(p, 1), (float)ch(p, 2), (float)ch(p, 3)};
+}
+__device__ __forceinline__ uint32_t px_pack(F4 v) {
+    return pack((uint32_t)v.r, (uint32_t)v.g, (uint32_t)v.b, (uint32_t)v.a);
+}
+__device__ __forceinline__ float div256f(float v) { return floorf(v * (1.0f / 256.0f)); }
+__device__ __forceinline__ float scale_f(float v, float m) { return div256f(fmaf(v, m, 255.0f)); }
+__device__ __forceinline__ F4 scale_f4(F4 v, float m) {
+    return F4{scale_f(v.r, m), scale_f(v.g, m), scale_f(v.b, m), scale_f(v.a, m)};
+}
+
+// `shade` without the packing
+__device__ __forceinline__ F4 shade_f(const ShaderParams &sp, uint32_t m, float x, float y) {
+    if ((m & rvkr::kModeKind) == 1u) return px_floats(sp.rgba);
+    float c[4];
+    const float t = grad_t(sp, m, x, y);
+    // (the clamp repeated in both forms folds into the addition before it)
+    if (m & rvkr::kModeTwoStop) {
+        for (int k = 0; k < 4; k++) c[k] = clamp01(t * sp.f[0][k] + sp.b[0][k]);
+    } else {
+        grad_color(sp, m & ~rvkr::kModeTwoStop, t, c);
+        for (int k = 0; k < 4; k++) c[k] = clamp01(c[k]);
+    }
+    for (int k = 0; k < 4; k++) c[k] = floorf(c[k] * 255.0f + 0.5f);
+    if (!(m & rvkr::kModeOpaque))
+        for (int k = 0; k < 3; k++) c[k] = scale_f(c[k], c[3]);
+    return F4{c[0], c[1], c[2], c[3]};
+}
+
+// `over_lowp`: the colour at coverage c (`full`: c is 255 everywhere) onto d
+__device__ __forceinline__ F4 over_f(F4 s, float c, bool full, F4 d, bool as_source) {
+    if (as_source) {
+        if (full) return s;
+        const float ic = 255.0f - c;
+        return F4{div256f(fmaf(s.r, c, fmaf(d.r, ic, 255.0f))), div256f(fmaf(s.g, c, fmaf(d.g, ic, 255.0f))),
+                  div256f(fmaf(s.b, c, fmaf(d.b, ic, 255.0f))), div256f(fmaf(s.a, c, fmaf(d.a, ic, 255.0f)))};
+    }
+    if (!full) s = scale_f4(s, c);
+    const float ia = 255.0f - s.a;
+    return F4{s.r + scale_f(d.r, ia), s.g + scale_f(d.g, ia), s.b + scale_f(d.b, ia), s.a + scale_f(d.a, ia)};
+}
+
+// SourceOver of a layer pixel with the layer's opacity (in [0, 1]) onto d: load_px,
+// blend and store_px.  The sum of a channel exceeds 1 by rounding only, so times 255 it
+// rounds to 255 without the clamp.
+__device__ __forceinline__ float layer_over_f(float s, float ia, float d) {
+    return rintf((s + d * (1.0f / 255.0f) * ia) * 255.0f);
+}
+__device__ __forceinline__ F4 layer_f(F4 s, float opacity, bool scaled, F4 d) {
+    const float k = 1.0f / 255.0f;
+    s.r *= k; s.g *= k; s.b *= k; s.a *= k;
+    if (scaled) { s.r *= opacity; s.g *= opacity; s.b *= opacity; s.a *= opacity; }
+    const float ia = 1.0f - s.a;
+    return F4{layer_over_f(s.r, ia, d.r), layer_over_f(s.g, ia, d.g), layer_over_f(s.b, ia, d.b),
+              layer_over_f(s.a, ia, d.a)};
+}
+
 // one covered pixel (lx, ly), centre (cx, cy), of a draw item: Clear, or the shaded
 // colour composited with over_lowp, or for a shader of the f32 pipeline (two-point
 // conical gradients, patterns) in f32 (scale_1_float by c / 255, SourceOver, store);
@@ -1417,8 +1477,8 @@ __global__ __launch_bounds__(256) void k_draw(uint32_t *px, uint32_t w, uint32_t
     const uint32_t pix = (uint32_t)lane;  // = (y % 8) * 8 + x % 8
     const float fx = (float)x + 0.5f, fy = (float)y + 0.5f;
     const bool inside = x < (int32_t)w && y < (int32_t)h;
-    uint32_t d = inside ? px[(size_t)y * w + x] : 0u;
-    const uint32_t d0 = d;
+    const uint32_t d0 = inside ? px[(size_t)y * w + x] : 0u;
+    F4 df = px_floats(d0);
     for (uint32_t base = 0; base < a.nitems; base += kWave) {
         // ---- cull 64 items, one per lane ----
         const uint32_t i = base + (uint32_t)lane;
@@ -1437,11 +1497,33 @@ __global__ __launch_bounds__(256) void k_draw(uint32_t *px, uint32_t w, uint32_t
             const int kl = __builtin_ctzll(m);
             const uint32_t efk = (uint32_t)__builtin_amdgcn_readlane((int)ef, kl);
             const uint32_t esk = (uint32_t)__builtin_amdgcn_readlane((int)es, kl);
-            const DrawItem item = a.items[base + (uint32_t)kl];  // with its jobs' grids and tables
-            if (!inside) continue;
-            const int32_t lx = x - item.lx, ly = y - item.ly;
+            const DrawItem &item = a.items[base + (uint32_t)kl];  // with its jobs' grids and tables
+            const uint32_t im = item.mode;
             // the pixel centre in layer coordinates, exact in f32 (|x|, |lx| < 2^23)
-            const float cx = fx - (float)item.lx, cy = fy - (float)item.ly;
+            const float cx = fx - item.flx, cy = fy - item.fly;
+            if (im & rvkr::kItemPlain) {
+                // gradients and solids of the u8 pipeline, SourceOver.  Coverage 0 leaves
+                // every value as it is, so the whole wave goes through together
+                F4 t = im & rvkr::kItemLayer ? F4{0.0f, 0.0f, 0.0f, 0.0f} : df;
+#pragma unroll 1
+                for (int pass = 0; pass < 2; pass++) {
+                    const bool stroke = (pass == 0) == ((im & rvkr::kItemStrokeFirst) != 0);
+                    const uint32_t e = stroke ? esk : efk;
+                    if (e == rvkr::kTileEmpty) continue;
+                    const JobRef &job = stroke ? item.sj : item.fj;
+                    const ShaderParams &sp = a.shaders[stroke ? item.stroke_shader : item.fill_shader];
+                    const uint32_t sm = sp.mode;
+                    float c = 255.0f;
+                    if (e != rvkr::kTileFull) c = (float)tile_cov(job, a.arena, e, tty, pix);
+                    t = over_f(shade_f(sp, sm, cx, cy), c, e == rvkr::kTileFull, t,
+                               (sm & rvkr::kModeAsSource) != 0);
+                }
+                df = im & rvkr::kItemLayer ? layer_f(t, item.opacity, (im & rvkr::kItemScaled) != 0, df) : t;
+                continue;
+            }
+            if (!inside) continue;
+            uint32_t d = px_pack(df);
+            const int32_t lx = x - item.lx, ly = y - item.ly;
             const uint32_t cf = tile_cov(item.fj, a.arena, efk, tty, pix);
             uint32_t cs = 0, hb = 0, he = 0;
             if (item.stroke_hair) {
@@ -1483,9 +1565,11 @@ __global__ __launch_bounds__(256) void k_draw(uint32_t *px, uint32_t w, uint32_t
                     }
                     d = store_px(blend(item.blend_mode, s, load_px(d)));
                 }
+                df = px_floats(d);
             }
         }
     }
+    const uint32_t d = px_pack(df);
     if (inside && d != d0) px[(size_t)y * w + x] = d;
 }
 

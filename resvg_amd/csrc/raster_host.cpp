@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <limits>
 
 using namespace rvkh;
 
@@ -742,7 +743,8 @@ static bool poly_to_unit_x(float x0, float y0, float x1, float y1, Ts &out) {
     return true;
 }
 
-void seal_shader(ShaderHead &s) {
+void seal_shader(ShaderParams &s) {
+    for (uint32_t i = s.nstops; i < sizeof s.t / sizeof s.t[0]; i++) s.t[i] = std::numeric_limits<float>::quiet_NaN();
     s.mode = (s.kind & kModeKind) | (s.radial ? kModeRadial : 0u) | ((s.spread & 3u) << kModeSpreadShift) |
              (s.pad_clamp ? kModePadClamp : 0u) | (s.two_stop ? kModeTwoStop : 0u) | (s.opaque ? kModeOpaque : 0u) |
              (s.r_twist ? kModeRTwist : 0u) | (s.as_source ? kModeAsSource : 0u) | (s.clear ? kModeClear : 0u) |

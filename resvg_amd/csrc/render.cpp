@@ -677,6 +677,18 @@ struct Renderer {
         uint8_t *host = (uint8_t *)hostv;
         for (ShaderParams &sp : dl.shaders) seal_shader(sp);
         if (!dl.shaders.empty()) std::memcpy(host + o_sh, dl.shaders.data(), dl.shaders.size() * sizeof(ShaderParams));
+        for (DrawItem &it : dl.items) {
+            auto lowp = [&](int32_t job, int32_t shader) {
+                return job < 0 || !(dl.shaders[shader].mode & (kModeClear | kModeF32));
+            };
+            const bool over = it.blend_mode == RVK_BLEND_SOURCE_OVER && it.opacity >= 0.0f && it.opacity <= 1.0f;
+            const bool plain = !it.stroke_hair && lowp(it.fill_job, it.fill_shader) &&
+                               lowp(it.stroke_job, it.stroke_shader) && (!it.layer || over);
+            it.mode = (plain ? kItemPlain : 0u) | (it.layer ? kItemLayer : 0u) |
+                      (it.stroke_first ? kItemStrokeFirst : 0u) | (it.opacity != 1.0f ? kItemScaled : 0u);
+            it.flx = (float)it.lx;
+            it.fly = (float)it.ly;
+        }
         std::memcpy(host + o_it, dl.items.data(), nitems * sizeof(DrawItem));
         {
             DrawCull *cull = (DrawCull *)(host + o_cull);

@@ -1125,6 +1125,20 @@ __device__ __forceinline__ float spread_t(uint32_t m, float t) {
     return t;
 }
 
+// sqrtf, correctly rounded, for a wave of values: away from 0 < x < 2^-96 (where the
+// residuals below would underflow; the whole wave then takes sqrtf) the hardware root is
+// within one unit in the last place, and the signs of the exact residuals at its two
+// neighbours say which of the three is nearest (Tuckerman's test).  0, infinity and NaN
+// fail both comparisons and stay as they are.
+__device__ __forceinline__ float wave_sqrt(float x) {
+    if (__ballot(x < 0x1p-96f && x > 0.0f) != 0) return sqrtf(x);
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float lo = __uint_as_float(__float_as_uint(s) - 1u), hi = __uint_as_float(__float_as_uint(s) + 1u);
+    // sqrt(x) <= s - half a unit: s * lo >= x; sqrt(x) > s + half a unit: s * hi < x
+    float r = fmaf(-lo, s, x) <= 0.0f ? lo : s;
+    return fmaf(-hi, s, x) > 0.0f ? hi : r;
+}
+
 // gradient coordinate t of a linear or concentric radial shader at the pixel centre
 // (x, y)
 __device__ __forceinline__ float grad_t(const ShaderHead &s, uint32_t m, float x, float y) {
@@ -1132,7 +1146,7 @@ __device__ __forceinline__ float grad_t(const ShaderHead &s, uint32_t m, float x
     float t = tx;
     if (m & rvkr::kModeRadial) {
         const float ty = x * s.ky + (y * s.sy + s.ty);
-        t = sqrtf(tx * tx + ty * ty);
+        t = wave_sqrt(tx * tx + ty * ty);
         if (m & rvkr::kModeRTwist) t = (t - s.r_scale) / s.r_bias;
     }
     return spread_t(m, t);
@@ -1348,31 +1362,42 @@ __device__ __forceinline__ F4 shade_f(const ShaderParams &sp, uint32_t m, float 
 }
 
 // `over_lowp`: the colour at coverage c (`full`: c is 255 everywhere) onto d
-__device__ __forceinline__ F4 over_f(F4 s, float c, bool full, F4 d, bool as_source) {
+__device__ __forceinline__ void over_f(F4 s, float c, bool full, F4 &d, bool as_source) {
     if (as_source) {
-        if (full) return s;
-        const float ic = 255.0f - c;
-        return F4{div256f(fmaf(s.r, c, fmaf(d.r, ic, 255.0f))), div256f(fmaf(s.g, c, fmaf(d.g, ic, 255.0f))),
-                  div256f(fmaf(s.b, c, fmaf(d.b, ic, 255.0f))), div256f(fmaf(s.a, c, fmaf(d.a, ic, 255.0f)))};
+        if (full) {
+            d = s;
+        } else {
+            const float ic = 255.0f - c;
+            d.r = div256f(fmaf(s.r, c, fmaf(d.r, ic, 255.0f)));
+            d.g = div256f(fmaf(s.g, c, fmaf(d.g, ic, 255.0f)));
+            d.b = div256f(fmaf(s.b, c, fmaf(d.b, ic, 255.0f)));
+            d.a = div256f(fmaf(s.a, c, fmaf(d.a, ic, 255.0f)));
+        }
+    } else {
+        if (!full) s = scale_f4(s, c);
+        const float ia = 255.0f - s.a;
+        d.r = s.r + scale_f(d.r, ia);
+        d.g = s.g + scale_f(d.g, ia);
+        d.b = s.b + scale_f(d.b, ia);
+        d.a = s.a + scale_f(d.a, ia);
     }
-    if (!full) s = scale_f4(s, c);
-    const float ia = 255.0f - s.a;
-    return F4{s.r + scale_f(d.r, ia), s.g + scale_f(d.g, ia), s.b + scale_f(d.b, ia), s.a + scale_f(d.a, ia)};
 }
 
 // SourceOver of a layer pixel with the layer's opacity (in [0, 1]) onto d: load_px,
 // blend and store_px.  The sum of a channel exceeds 1 by rounding only, so times 255 it
 // rounds to 255 without the clamp.
-__device__ __forceinline__ float layer_over_f(float s, float ia, float d) {
-    return rintf((s + d * (1.0f / 255.0f) * ia) * 255.0f);
+__device__ __forceinline__ void layer_over_f(float s, float ia, float &d) {
+    d = rintf((s + d * (1.0f / 255.0f) * ia) * 255.0f);
 }
-__device__ __forceinline__ F4 layer_f(F4 s, float opacity, bool scaled, F4 d) {
+__device__ __forceinline__ void layer_f(F4 s, float opacity, bool scaled, F4 &d) {
     const float k = 1.0f / 255.0f;
     s.r *= k; s.g *= k; s.b *= k; s.a *= k;
     if (scaled) { s.r *= opacity; s.g *= opacity; s.b *= opacity; s.a *= opacity; }
     const float ia = 1.0f - s.a;
-    return F4{layer_over_f(s.r, ia, d.r), layer_over_f(s.g, ia, d.g), layer_over_f(s.b, ia, d.b),
-              layer_over_f(s.a, ia, d.a)};
+    layer_over_f(s.r, ia, d.r);
+    layer_over_f(s.g, ia, d.g);
+    layer_over_f(s.b, ia, d.b);
+    layer_over_f(s.a, ia, d.a);
 }
 
 // one covered pixel (lx, ly), centre (cx, cy), of a draw item: Clear, or the shaded
@@ -1504,21 +1529,37 @@ __global__ __launch_bounds__(256) void k_draw(uint32_t *px, uint32_t w, uint32_t
             if (im & rvkr::kItemPlain) {
                 // gradients and solids of the u8 pipeline, SourceOver.  Coverage 0 leaves
                 // every value as it is, so the whole wave goes through together
-                F4 t = im & rvkr::kItemLayer ? F4{0.0f, 0.0f, 0.0f, 0.0f} : df;
-#pragma unroll 1
-                for (int pass = 0; pass < 2; pass++) {
-                    const bool stroke = (pass == 0) == ((im & rvkr::kItemStrokeFirst) != 0);
-                    const uint32_t e = stroke ? esk : efk;
-                    if (e == rvkr::kTileEmpty) continue;
-                    const JobRef &job = stroke ? item.sj : item.fj;
+                const bool swap = (im & rvkr::kItemStrokeFirst) != 0;
+                auto shaded = [&](bool stroke, uint32_t e, float &c, uint32_t &sm) {
                     const ShaderParams &sp = a.shaders[stroke ? item.stroke_shader : item.fill_shader];
-                    const uint32_t sm = sp.mode;
-                    float c = 255.0f;
-                    if (e != rvkr::kTileFull) c = (float)tile_cov(job, a.arena, e, tty, pix);
-                    t = over_f(shade_f(sp, sm, cx, cy), c, e == rvkr::kTileFull, t,
-                               (sm & rvkr::kModeAsSource) != 0);
+                    if (e != rvkr::kTileFull) c = (float)tile_cov(stroke ? item.sj : item.fj, a.arena, e, tty, pix);
+                    sm = sp.mode;
+                    return shade_f(sp, sm, cx, cy);
+                };
+                // the first of fill and stroke in drawing order that touches the tile,
+                // then the other
+                const uint32_t e0 = swap ? esk : efk, e1 = swap ? efk : esk;
+                const bool one = e0 == rvkr::kTileEmpty || e1 == rvkr::kTileEmpty;
+                const bool first = (e0 == rvkr::kTileEmpty) != swap;  // the first is the stroke
+                const uint32_t ea = e0 == rvkr::kTileEmpty ? e1 : e0;
+                float c = 255.0f;
+                uint32_t sm;
+                F4 t = shaded(first, ea, c, sm);
+                if (im & rvkr::kItemLayer) {
+                    // onto a transparent layer pixel: the colour scaled by its coverage
+                    if (ea != rvkr::kTileFull) t = scale_f4(t, c);
+                    if (!one) {
+                        const F4 u = shaded(!first, e1, c = 255.0f, sm);
+                        over_f(u, c, e1 == rvkr::kTileFull, t, (sm & rvkr::kModeAsSource) != 0);
+                    }
+                    layer_f(t, item.opacity, (im & rvkr::kItemScaled) != 0, df);
+                } else {
+                    over_f(t, c, ea == rvkr::kTileFull, df, (sm & rvkr::kModeAsSource) != 0);
+                    if (!one) {
+                        const F4 u = shaded(!first, e1, c = 255.0f, sm);
+                        over_f(u, c, e1 == rvkr::kTileFull, df, (sm & rvkr::kModeAsSource) != 0);
+                    }
                 }
-                df = im & rvkr::kItemLayer ? layer_f(t, item.opacity, (im & rvkr::kItemScaled) != 0, df) : t;
                 continue;
             }
             if (!inside) continue;

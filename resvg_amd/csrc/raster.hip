@@ -1,9 +1,10 @@
 // Device rasterizer: curve expansion, anti-aliased coverage and the fused
 // shade/composite of draw lists.
 //
-// Expansion (k_expand): one thread per edge runs tiny-skia's quadratic / cubic
-// update loop (Skia's forward differencing in 16.16 fixed point) from the state the
-// host left after the first piece, writing every non-empty line piece in order.
+// Expansion (k_expand): tiny-skia's quadratic / cubic update loop (Skia's forward
+// differencing in 16.16 fixed point) from the state the host left after the first piece,
+// a lane per edge, then a lane per segment for its line piece; every non-empty piece is
+// written in order.
 //
 // Coverage (k_coverage): a block of eight 64-lane waves per (coverage job, band of 8
 // pixel rows), one wave per row.  The block's threads leave the crossings of the band's
@@ -54,10 +55,12 @@ __device__ __forceinline__ int32_t fdot6_to_fixed(int32_t x) { return (int32_t)(
 __device__ __forceinline__ int32_t fixed_mul(int32_t a, int32_t b) {
     return (int32_t)(((int64_t)a * (int64_t)b) >> 16);
 }
+// (a << 16) / b truncated towards zero and saturated, b > 0.  The dividend has at most 47
+// bits, so the f64 quotient is off by less than 1 / 64 of the distance 1 / b that a
+// non-integral one keeps from the next integer, and its truncation is the integer
+// quotient (a 64-bit integer division takes ten times the instructions).
 __device__ __forceinline__ int32_t fdot6_div(int32_t a, int32_t b) {
-    if ((int32_t)(int16_t)a == a) return (int32_t)((uint32_t)a << 16) / b;
-    int64_t v = ((int64_t)a << 16) / (int64_t)b;
-    return (int32_t)max((int64_t)INT32_MIN, min((int64_t)INT32_MAX, v));
+    return as_i32d((double)a * 65536.0 / (double)b);
 }
 
 // SkEdge::updateLine on 16.16 inputs
@@ -86,59 +89,88 @@ struct ExpandArgs {
     int32_t *overflow;
 };
 
-__global__ __launch_bounds__(256) void k_expand(ExpandArgs a) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.nedges) return;
-    EdgeRec e = a.edges[i];
-    PieceDev *out = a.pieces + e.piece_offset;
-    const int32_t ymax = a.cov[i].ymax;
-    uint32_t n = 0;
-    out[n++] = PieceDev{e.x, e.dx, e.first_y, e.last_y};
-    int32_t oldx = e.cx, oldy = e.cy;
-    if (e.type == 1) {  // SkQuadraticEdge::updateQuadratic, repeated until exhausted
-        int32_t count = e.count, dx = e.d1x, dy = e.d1y;
-        while (count > 0) {
-            int32_t newx, newy;
-            if (--count > 0) {
-                newx = oldx + (dx >> e.shift);
-                dx += e.d2x;
-                newy = oldy + (dy >> e.shift);
-                dy += e.d2y;
-            } else {
-                newx = e.lx;
-                newy = e.ly;
+constexpr int kExpandSteps = 64;   // curve segments after the first piece (MAX_COEFF_SHIFT 6: at most 63)
+
+// One wave per 16 edges.  A lane per edge runs the curve's update steps, which only add
+// and shift, into LDS; then each half of the wave takes an edge at a time, a lane per
+// segment: the slope's division (most of the work), and the non-empty pieces compacted in
+// order and stored together.  One thread per edge doing both took 15-30 us however few
+// edges there were (30 -> 7 us per launch of a 2048^2 document's clip paths).
+template <int E>
+__global__ __launch_bounds__(kWave) void k_expand(ExpandArgs a) {
+    __shared__ int2 pts[E][kExpandSteps + 1];  // 16.16 points, the first piece's end first
+    __shared__ int4 head[E];                   // segments, first piece slot, row bound, the first piece's last row
+    const int lane = threadIdx.x;
+    const uint32_t first = blockIdx.x * E;
+    if (lane < E && first + lane < a.nedges) {
+        const EdgeRec e = a.edges[first + lane];
+        const int32_t bound = a.cov[first + lane].ymax;
+        a.pieces[e.piece_offset] = PieceDev{e.x, e.dx, e.first_y, e.last_y};
+        int n = 0;
+        int2 at = make_int2(e.cx, e.cy);
+        pts[lane][0] = at;
+        if (e.type == 1) {  // SkQuadraticEdge::updateQuadratic, repeated until exhausted
+            int32_t dx = e.d1x, dy = e.d1y;
+            for (int32_t count = e.count; count > 0 && n < kExpandSteps;) {
+                if (--count > 0) {
+                    at.x += dx >> e.shift;
+                    dx += e.d2x;
+                    at.y += dy >> e.shift;
+                    dy += e.d2y;
+                } else {
+                    at = make_int2(e.lx, e.ly);
+                }
+                pts[lane][++n] = at;
             }
-            PieceDev p;
-            if (line_piece(oldx, oldy, newx, newy, p)) out[n++] = p;
-            oldx = newx;
-            oldy = newy;
-        }
-    } else if (e.type == 2) {  // SkCubicEdge::updateCubic
-        int32_t count = e.count;
-        int32_t d1x = e.d1x, d1y = e.d1y, d2x = e.d2x, d2y = e.d2y;
-        while (count < 0) {
-            int32_t newx, newy;
-            if (++count < 0) {
-                newx = oldx + (d1x >> e.dshift);
-                d1x += d2x >> e.shift;
-                d2x += e.d3x;
-                newy = oldy + (d1y >> e.dshift);
-                d1y += d2y >> e.shift;
-                d2y += e.d3y;
-            } else {
-                newx = e.lx;
-                newy = e.ly;
+        } else if (e.type == 2) {  // SkCubicEdge::updateCubic
+            int32_t d1x = e.d1x, d1y = e.d1y, d2x = e.d2x, d2y = e.d2y;
+            for (int32_t count = e.count; count < 0 && n < kExpandSteps;) {
+                const int32_t oldy = at.y;
+                if (++count < 0) {
+                    at.x += d1x >> e.dshift;
+                    d1x += d2x >> e.shift;
+                    d2x += e.d3x;
+                    at.y += d1y >> e.dshift;
+                    d1y += d2y >> e.shift;
+                    d2y += e.d3y;
+                } else {
+                    at = make_int2(e.lx, e.ly);
+                }
+                at.y = max(at.y, oldy);
+                pts[lane][++n] = at;
             }
-            if (newy < oldy) newy = oldy;
-            PieceDev p;
-            if (line_piece(oldx, oldy, newx, newy, p)) out[n++] = p;
-            oldx = newx;
-            oldy = newy;
         }
+        head[lane] = make_int4(n, (int)e.piece_offset, bound, e.last_y);
     }
-    a.npieces[i] = n;
-    // the host's row bound must cover every piece (else rows would miss the edge)
-    if (out[n - 1].last_y > ymax) atomicAdd(a.overflow, 1);
+    __syncthreads();
+    const int half = lane >> 5, hl = lane & 31;
+    for (int k = half; k < E; k += 2) {
+        const uint32_t i = first + (uint32_t)k;
+        if (i >= a.nedges) break;
+        const int4 h = head[k];
+        const int n = h.x;
+        PieceDev *out = a.pieces + (uint32_t)h.y;
+        uint32_t count = 1;
+        bool over = h.w > h.z;
+        for (int j0 = 0; j0 < n; j0 += 32) {
+            const int j = j0 + hl;
+            PieceDev p;
+            bool ok = false;
+            if (j < n) {
+                const int2 u = pts[k][j], v = pts[k][j + 1];
+                ok = line_piece(u.x, u.y, v.x, v.y, p);
+            }
+            const uint32_t m = (uint32_t)(__ballot(ok) >> (32 * half));
+            if (ok) {
+                out[count + __popc(m & ((1u << hl) - 1u))] = p;
+                over = over || p.last_y > h.z;
+            }
+            count += __popc(m);
+        }
+        if (hl == 0) a.npieces[i] = count;
+        // the host's row bound must cover every piece (else rows would miss the edge)
+        if (over) atomicAdd(a.overflow, 1);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1622,8 +1654,10 @@ rvk_status launch_expand(rvk_context *ctx, const EdgeRec *edges, uint32_t nedges
                          PieceDev *pieces, uint32_t *npieces, int32_t *overflow, double algo_bytes) {
     if (nedges == 0) return RVK_OK;
     ExpandArgs a{edges, nedges, cov, pieces, npieces, overflow};
-    timed_launch(ctx, "expand", algo_bytes,
-                 [&] { hipLaunchKernelGGL(k_expand, dim3(div_up(nedges, 256)), dim3(256), 0, ctx->stream, a); });
+    timed_launch(ctx, "expand", algo_bytes, [&] {
+        if (nedges > 16384u) hipLaunchKernelGGL(k_expand<16>, dim3(div_up(nedges, 16)), dim3(kWave), 0, ctx->stream, a);
+        else hipLaunchKernelGGL(k_expand<4>, dim3(div_up(nedges, 4)), dim3(kWave), 0, ctx->stream, a);
+    });
     RVK_HIP_CHECK(hipGetLastError());
     return RVK_OK;
 }

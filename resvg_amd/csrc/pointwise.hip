@@ -509,6 +509,15 @@ rvk_status launch_copy(rvk_context *ctx, uint8_t *dst, const uint8_t *src, size_
     return RVK_OK;
 }
 
+rvk_status launch_upload(hipStream_t stream, void *dev_dst, const void *pinned_src, size_t bytes) {
+    void *src = nullptr;
+    RVK_HIP_CHECK(hipHostGetDevicePointer(&src, const_cast<void *>(pinned_src), 0));
+    const size_t n = bytes / 16;
+    hipLaunchKernelGGL(k_copy, dim3(grid_for(n)), dim3(kBlock), 0, stream, (uint4 *)dev_dst, (const uint4 *)src, n);
+    RVK_HIP_CHECK(hipGetLastError());
+    return RVK_OK;
+}
+
 }  // namespace rvk
 
 namespace rvkh {

@@ -260,16 +260,24 @@ struct Renderer {
     // the flush before last, the previous reader of the block, is done (or, for a
     // block just taken from the scratch cache, until the context stream's work so far
     // is), so the coverage of a flush overlaps the compositing of the one before.
+    // A small flush (fewer than kOverlapBands coverage bands) runs on the context stream
+    // alone: the events that hand work to the side stream and back cost more than its
+    // coverage takes.
     void *blk[2] = {nullptr, nullptr};
     size_t blk_cap[2] = {0, 0};
     hipEvent_t blk_free[2] = {nullptr, nullptr};  // recorded on the context stream after a block's draw
-    bool blk_used[2] = {false, false};
+    bool blk_used[2] = {false, false};            // the block has a reader on the context stream,
+    bool blk_recorded[2] = {false, false};        // and blk_free was recorded after it
     hipEvent_t ev_cov = nullptr, ev_main = nullptr, ev_side = nullptr;
     uint64_t nflush = 0;
     bool side_used = false;
     // false: a flush runs on the context stream alone (on a batch's lanes, which
     // already run documents side by side)
     const bool overlap = !ctx->is_lane;
+    // A record, a wait and their return on two streams take 23 us of host time more than
+    // the launches alone, about what the coverage of 2000 bands takes on the device (0.65
+    // ms for the 30 000 of a 4096^2 flush)
+    static constexpr uint64_t kOverlapBands = 2048;
 
     ~Renderer() { (void)finish_flushes(); }
 
@@ -291,6 +299,7 @@ struct Renderer {
             blk[b] = nullptr;
             blk_cap[b] = 0;
             blk_used[b] = false;
+            blk_recorded[b] = false;
         }
         for (hipEvent_t *e : {&blk_free[0], &blk_free[1], &ev_cov, &ev_main, &ev_side})
             if (*e) {
@@ -767,13 +776,15 @@ struct Renderer {
         // when it is too small (the old one's last reader is on the context stream)
         const int b = (int)(nflush++ & 1);
         const size_t need = o_arena + dl.arena;
-        RVK_TRY(flush_events());
+        const bool aside = overlap && dl.n_windows >= kOverlapBands;
+        if (aside) RVK_TRY(flush_events());
         bool fresh = false;
         if (blk_cap[b] < need) {
             if (blk[b]) rvk::scratch_release(ctx, blk[b]);
             blk[b] = nullptr;
             blk_cap[b] = 0;
             blk_used[b] = false;
+            blk_recorded[b] = false;
             RVK_TRY(rvk::scratch_alloc(ctx, need, &blk[b]));
             blk_cap[b] = need;
             fresh = true;
@@ -803,14 +814,14 @@ struct Renderer {
         ctx->stats.band_entries += dl.n_windows;
         ctx->stats.upload_bytes += meta;
         hipStream_t side = ctx->stream;
-        if (overlap) {
+        if (aside) {
             RVK_TRY(rvk::side_stream(ctx, &side));
             side_used = true;
-            if (fresh) {
+            if (blk_recorded[b]) {
+                RVK_HIP_CHECK(hipStreamWaitEvent(side, blk_free[b], 0));
+            } else if (fresh || blk_used[b]) {  // after the context stream's work so far
                 RVK_HIP_CHECK(hipEventRecord(ev_main, ctx->stream));
                 RVK_HIP_CHECK(hipStreamWaitEvent(side, ev_main, 0));
-            } else if (blk_used[b]) {
-                RVK_HIP_CHECK(hipStreamWaitEvent(side, blk_free[b], 0));
             }
         }
         rvk_status st = rvk::upload_staged_on(ctx, slot, d, meta, side);
@@ -846,12 +857,14 @@ struct Renderer {
                                         std::any_of(dl.shaders.begin(), dl.shaders.end(),
                                                     [](const ShaderParams &q) { return q.kind == 3; }),
                                         draw_bytes);
-        if (st == RVK_OK) {
+        blk_used[b] = true;
+        blk_recorded[b] = false;
+        if (st == RVK_OK && aside) {
             if (hipEventRecord(blk_free[b], ctx->stream) != hipSuccess) {
                 (void)hipGetLastError();
                 st = RVK_ERR_HIP;
             } else {
-                blk_used[b] = true;
+                blk_recorded[b] = true;
             }
         }
         ctx->stats.flushes++;

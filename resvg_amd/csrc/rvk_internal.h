@@ -151,6 +151,10 @@ rvk_status launch_draw_pixmap(rvk_context *ctx, uint8_t *dst, uint32_t dw, uint3
 rvk_status launch_fill(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, const uint8_t premul[4]);
 rvk_status launch_fill_sub(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, int64_t x0, int64_t y0,
                            int64_t x1, int64_t y1, uint32_t value);
+// dev_dst = `bytes` (a multiple of 16, both 16-byte aligned) of pinned host memory, read
+// by a kernel on `stream`
+constexpr size_t kKernelUploadBytes = (size_t)1 << 20;
+rvk_status launch_upload(hipStream_t stream, void *dev_dst, const void *pinned_src, size_t bytes);
 rvk_status launch_copy(rvk_context *ctx, uint8_t *dst, const uint8_t *src, size_t bytes);
 // Fills a w x h image with the periodic repeat of the tw x th tile at (tx0, ty0)
 // of a sw x sh source, phase (ox, oy): feTile.

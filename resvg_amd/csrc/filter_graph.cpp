@@ -67,8 +67,8 @@ Img take(Img a) {
 Img into_cs(Img im, uint32_t cs) {
     if (im->cs == cs) return im;
     IRect region = im->region;
-    Img c = take(std::move(im));
-    FTRY(rvk::launch_into_cs(c->ctx, c->px, c->w, c->h, cs == RVK_CI_LINEAR_RGB));
+    Img c = im.use_count() == 1 && im->owned ? im : new_img(im->ctx, im->w, im->h, cs, false);
+    FTRY(rvk::launch_into_cs(c->ctx, c->px, im->px, c->w, c->h, cs == RVK_CI_LINEAR_RGB));
     c->cs = cs;
     c->region = region;
     return c;
@@ -79,6 +79,8 @@ Img from_image(Img im, uint32_t cs) {
     im->cs = cs;
     return im;
 }
+
+bool same_size(const Img &a, const Img &b) { return a->w == b->w && a->h == b->h; }
 
 void draw(const Img &dst, const Img &src, int32_t x, int32_t y, uint32_t mode) {
     FTRY(rvk::launch_draw_pixmap(dst->ctx, dst->px, dst->w, dst->h, x, y, src->px, src->w, src->h, 1.0f, mode));
@@ -92,19 +94,47 @@ struct Exec {
     Img source;  // the layer, borrowed
     std::vector<std::pair<int32_t, Img>> results;
     const rvk::FeImageHook *fe_image = nullptr;  // draws feImage content (render walks only)
+    // references to each result that are still to come: its last user takes it over
+    // instead of copying it
+    std::vector<uint32_t> uses;
+
+    size_t find(int32_t id, size_t count) const {  // the newest of the first `count` results
+        while (count > 0 && results[count - 1].first != id) count--;
+        return count;  // one past it; 0: none
+    }
+    // every input a primitive may ask for (asking for fewer keeps an image longer, no more)
+    template <typename F>
+    void for_inputs(const rvk_primitive &p, F f) const {
+        if (p.kind == RVK_FE_MERGE) {
+            for (uint32_t i = 0; data->inputs && i < p.u.merge.input_count; i++)
+                f(data->inputs[p.u.merge.input_offset + i]);
+            return;
+        }
+        f(p.in1);
+        if (p.kind == RVK_FE_BLEND || p.kind == RVK_FE_COMPOSITE || p.kind == RVK_FE_DISPLACEMENT_MAP) f(p.in2);
+    }
+    void count_uses(const rvk_filter &f) {
+        uses.assign(f.primitive_count, 0);
+        const rvk_primitive *prims = data->primitives + f.primitive_offset;
+        for (uint32_t i = 0; i < f.primitive_count; i++)
+            for_inputs(prims[i], [&](int32_t in) {
+                for (uint32_t j = i; in >= 0 && j-- > 0;)
+                    if (prims[j].result == in) { uses[j]++; break; }
+            });
+        if (f.primitive_count) uses.back()++;  // the graph's own result
+    }
 
     // get_input (mod.rs:523-564)
     Img input(int32_t in) {
         if (in >= 0) {
-            for (auto it = results.rbegin(); it != results.rend(); ++it)
-                if (it->first == in) return it->second;
+            if (const size_t i = find(in, results.size()))
+                return --uses[i - 1] == 0 ? std::move(results[i - 1].second) : results[i - 1].second;
             in = RVK_INPUT_SOURCE_GRAPHIC;
         }
         if (in == RVK_INPUT_SOURCE_ALPHA) {
-            Img c = clone_img(source);
+            Img c = new_img(ctx, source->w, source->h, RVK_CI_SRGB, false);
             c->region = region;
-            c->cs = RVK_CI_SRGB;
-            FTRY(rvk::launch_zero_rgb(ctx, c->px, (size_t)c->w * c->h));
+            FTRY(rvk::launch_alpha_only(ctx, c->px, source->px, (size_t)c->w * c->h));
             return c;
         }
         // SourceGraphic: the reference clones the layer for every use; here each use
@@ -121,9 +151,34 @@ struct Exec {
         return c;
     }
 
-    void blur(const Img &im, double sx, double sy, bool box) {
-        if (box) FTRY(rvk::launch_box_blur(ctx, im->px, im->w, im->h, sx, sy));
-        else FTRY(rvk::launch_iir_blur(ctx, im->px, im->w, im->h, sx, sy));
+    Img blur(Img im, double sx, double sy, bool box) {
+        if (!box) {
+            Img out = take(std::move(im));
+            FTRY(rvk::launch_iir_blur(ctx, out->px, out->w, out->h, sx, sy));
+            return out;
+        }
+        const bool own = im.use_count() == 1 && im->owned;  // then it is the work image
+        Img out = new_img(ctx, im->w, im->h, im->cs, false);
+        Img tmp = own ? nullptr : new_img(ctx, im->w, im->h, im->cs, false);
+        FTRY(rvk::launch_box_blur_to(ctx, im->px, out->px, own ? nullptr : tmp->px, im->w, im->h, sx, sy));
+        return out;
+    }
+
+    // src blended onto `below` in a new image of the filter region's size, or in `below`
+    // itself where nothing else holds it
+    Img blend(Img below, const Img &src, uint32_t cs, uint32_t mode) {
+        const IRect whole{0, 0, region.w, region.h};
+        if ((int64_t)below->w == region.w && (int64_t)below->h == region.h && same_size(below, src)) {
+            Img out = below.use_count() == 1 && below->owned ? below
+                                                             : new_img(ctx, region.w, region.h, cs, false);
+            FTRY(rvk::launch_blend_pair(ctx, out->px, below->px, src->px, (size_t)out->w * out->h, mode));
+            out->region = whole;
+            return out;
+        }
+        Img out = new_img(ctx, region.w, region.h, cs);
+        draw(out, below, 0, 0, RVK_BLEND_SOURCE_OVER);
+        draw(out, src, 0, 0, mode);
+        return out;
     }
 
     Img primitive(const rvk_primitive &p, IRect sub) {
@@ -132,11 +187,8 @@ struct Exec {
             case RVK_FE_BLEND: {  // mod.rs:695-729
                 Img i1 = into_cs(input(p.in1), cs);
                 Img i2 = into_cs(input(p.in2), cs);
-                Img out = new_img(ctx, region.w, region.h, cs);
-                draw(out, i2, 0, 0, RVK_BLEND_SOURCE_OVER);
                 if (p.u.blend.mode >= RVK_BLEND_COUNT) throw FilterError{RVK_ERR_INVALID_ARGUMENT};
-                draw(out, i1, 0, 0, p.u.blend.mode);
-                return out;
+                return blend(std::move(i2), i1, cs, p.u.blend.mode);
             }
             case RVK_FE_DROP_SHADOW: {  // mod.rs:581-643
                 const auto &d = p.u.drop_shadow;
@@ -144,14 +196,13 @@ struct Exec {
                 float dx, dy;
                 scale_coords(d.dx, d.dy, ts, dx, dy);
                 Img out = new_img(ctx, in->w, in->h, cs);
-                Img inp = into_cs(in, cs);
-                in.reset();
-                Img shadow = clone_img(inp);
+                Img inp = into_cs(std::move(in), cs);
                 double sx, sy;
                 bool box;
-                if (resolve_std_dev(d.std_dev_x, d.std_dev_y, ts, sx, sy, box)) blur(shadow, sx, sy, box);
+                Img shadow = resolve_std_dev(d.std_dev_x, d.std_dev_y, ts, sx, sy, box) ? blur(inp, sx, sy, box)
+                                                                                       : clone_img(inp);
                 FTRY(launch_shadow_flood(ctx, shadow->px, (size_t)shadow->w * shadow->h, d.color, d.opacity));
-                FTRY(rvk::launch_into_cs(ctx, shadow->px, shadow->w, shadow->h, cs == RVK_CI_LINEAR_RGB));
+                FTRY(rvk::launch_into_cs(ctx, shadow->px, shadow->px, shadow->w, shadow->h, cs == RVK_CI_LINEAR_RGB));
                 draw(out, shadow, as_i32(dx), as_i32(dy), RVK_BLEND_SOURCE_OVER);
                 draw(out, inp, 0, 0, RVK_BLEND_SOURCE_OVER);
                 return out;
@@ -170,9 +221,7 @@ struct Exec {
                 double sx, sy;
                 bool box;
                 if (!resolve_std_dev(p.u.blur.std_dev_x, p.u.blur.std_dev_y, ts, sx, sy, box)) return in;
-                Img out = take(into_cs(std::move(in), cs));
-                blur(out, sx, sy, box);
-                return from_image(out, cs);
+                return from_image(blur(into_cs(std::move(in), cs), sx, sy, box), cs);
             }
             case RVK_FE_OFFSET: {  // mod.rs:668-693
                 Img in = input(p.in1);
@@ -186,29 +235,35 @@ struct Exec {
             case RVK_FE_COMPOSITE: {  // mod.rs:731-793
                 Img i1 = into_cs(input(p.in1), cs);
                 Img i2 = into_cs(input(p.in2), cs);
-                Img out = new_img(ctx, region.w, region.h, cs);
                 const auto &k = p.u.composite;
                 if (k.op == RVK_COMPOSITE_ARITHMETIC) {
-                    size_t n = std::min({i1->bytes(), i2->bytes(), out->bytes()}) / 4;
-                    FTRY(rvk::launch_arithmetic(ctx, i1->px, i2->px, out->px, n, k.k1, k.k2, k.k3, k.k4));
+                    const size_t bytes = std::min(i1->bytes(), i2->bytes());
+                    const bool whole = bytes >= (size_t)region.w * region.h * 4;
+                    Img out = new_img(ctx, region.w, region.h, cs, !whole);
+                    FTRY(rvk::launch_arithmetic(ctx, i1->px, i2->px, out->px, std::min(bytes, out->bytes()) / 4, k.k1,
+                                                k.k2, k.k3, k.k4, whole));
                     return out;
                 }
                 if (k.op > RVK_COMPOSITE_ARITHMETIC) throw FilterError{RVK_ERR_INVALID_ARGUMENT};
-                draw(out, i2, 0, 0, RVK_BLEND_SOURCE_OVER);
                 uint32_t mode = k.op == RVK_COMPOSITE_IN ? RVK_BLEND_SOURCE_IN
                               : k.op == RVK_COMPOSITE_OUT ? RVK_BLEND_SOURCE_OUT
                               : k.op == RVK_COMPOSITE_ATOP ? RVK_BLEND_SOURCE_ATOP
                               : k.op == RVK_COMPOSITE_XOR ? RVK_BLEND_XOR : RVK_BLEND_SOURCE_OVER;
-                draw(out, i1, 0, 0, mode);
-                return out;
+                return blend(std::move(i2), i1, cs, mode);
             }
             case RVK_FE_MERGE: {  // mod.rs:795-818
-                Img out = new_img(ctx, region.w, region.h, cs);
-                for (uint32_t i = 0; i < p.u.merge.input_count; i++) {
-                    if (!data->inputs) throw FilterError{RVK_ERR_INVALID_ARGUMENT};
-                    Img in = into_cs(input(data->inputs[p.u.merge.input_offset + i]), cs);
-                    draw(out, in, 0, 0, RVK_BLEND_SOURCE_OVER);
+                const uint32_t count = p.u.merge.input_count;
+                if (count && !data->inputs) throw FilterError{RVK_ERR_INVALID_ARGUMENT};
+                auto in = [&](uint32_t i) { return into_cs(input(data->inputs[p.u.merge.input_offset + i]), cs); };
+                if (count < 2) {
+                    Img out = new_img(ctx, region.w, region.h, cs);
+                    if (count) draw(out, in(0), 0, 0, RVK_BLEND_SOURCE_OVER);
+                    return out;
                 }
+                Img first = in(0), second = in(1);
+                Img out = blend(std::move(first), second, cs, RVK_BLEND_SOURCE_OVER);
+                second.reset();
+                for (uint32_t i = 2; i < count; i++) draw(out, in(i), 0, 0, RVK_BLEND_SOURCE_OVER);
                 return out;
             }
             case RVK_FE_COMPONENT_TRANSFER: {  // mod.rs:891-903 (demultiply, transfer, multiply fused)
@@ -222,9 +277,13 @@ struct Exec {
                 return from_image(out, cs);
             }
             case RVK_FE_CONVOLVE_MATRIX: {  // mod.rs:919-933
-                Img out = take(into_cs(input(p.in1), cs));
-                if (p.u.convolve.preserve_alpha) FTRY(rvk::launch_demultiply(ctx, out->px, out->w, out->h));
-                FTRY(rvk::launch_convolve(ctx, out->px, out->w, out->h, &p, data->values));
+                Img in = into_cs(input(p.in1), cs);
+                if (p.u.convolve.preserve_alpha) {
+                    in = take(std::move(in));
+                    FTRY(rvk::launch_demultiply(ctx, in->px, in->w, in->h));
+                }
+                Img out = new_img(ctx, in->w, in->h, cs, false);
+                FTRY(rvk::launch_convolve_to(ctx, in->px, out->px, out->w, out->h, &p, data->values));
                 return from_image(out, cs);
             }
             case RVK_FE_MORPHOLOGY: {  // mod.rs:935-956
@@ -242,13 +301,14 @@ struct Exec {
             case RVK_FE_DISPLACEMENT_MAP: {  // mod.rs:958-986
                 Img p1 = into_cs(input(p.in1), cs);
                 Img p2 = into_cs(input(p.in2), cs);
-                Img out = new_img(ctx, region.w, region.h, cs);
+                const bool fits = (int64_t)p1->w == region.w && (int64_t)p1->h == region.h && same_size(p1, p2);
+                Img out = new_img(ctx, region.w, region.h, cs, !fits);
                 float sx, sy;
                 scale_coords(p.u.displacement.scale, p.u.displacement.scale, ts, sx, sy);
-                if (p1->w == out->w && p1->h == out->h && p2->w == out->w && p2->h == out->h)
+                if (fits)
                     FTRY(rvk::launch_displacement(ctx, p1->px, p2->px, out->px, out->w, out->h, sx, sy,
                                                   p.u.displacement.scale, p.u.displacement.x_channel,
-                                                  p.u.displacement.y_channel));
+                                                  p.u.displacement.y_channel, 1));
                 return out;
             }
             case RVK_FE_TURBULENCE: {  // mod.rs:988-1018 (multiply_alpha fused)
@@ -267,9 +327,11 @@ struct Exec {
             case RVK_FE_DIFFUSE_LIGHTING:
             case RVK_FE_SPECULAR_LIGHTING: {  // mod.rs:1020-1060
                 Img in = input(p.in1);
-                Img out = new_img(ctx, region.w, region.h, cs);
+                const bool fits = (int64_t)in->w == region.w && (int64_t)in->h == region.h;
+                // written whole, except that lighting leaves images under 3 pixels a side as they are
+                Img out = new_img(ctx, region.w, region.h, cs, !fits || region.w < 3 || region.h < 3);
                 rvk_light_source l = transform_light(p.u.lighting.light, region, ts);
-                if (in->w == out->w && in->h == out->h)
+                if (fits)
                     FTRY(rvk::launch_lighting(ctx, in->px, out->px, out->w, out->h,
                                               p.kind == RVK_FE_SPECULAR_LIGHTING, p.u.lighting.surface_scale,
                                               p.u.lighting.constant, p.u.lighting.specular_exponent,
@@ -324,14 +386,14 @@ struct Exec {
         if (!fr.ok) throw FilterError{RVK_ERR_INVALID_REGION};
         if (!fit_to_rect(frect_to_int(fr), IRect{0, 0, (int32_t)source->w, (int32_t)source->h}, region))
             throw FilterError{RVK_ERR_INVALID_REGION};
+        count_uses(f);
         for (uint32_t i = 0; i < f.primitive_count; i++) {
             const rvk_primitive &p = data->primitives[f.primitive_offset + i];
             FRect pr = rect_transform(p.rect, ts);
             if (!pr.ok) throw FilterError{RVK_ERR_INVALID_REGION};
             IRect sub = frect_to_int(pr);
             if (p.kind == RVK_FE_OFFSET && p.in1 >= 0) {
-                for (auto it = results.rbegin(); it != results.rend(); ++it)
-                    if (it->first == p.in1) { sub = it->second->region; break; }
+                if (const size_t k = find(p.in1, results.size())) sub = results[k - 1].second->region;
             }
             Img res = primitive(p, sub);
             if (!ir_eq(region, sub)) {
@@ -370,13 +432,14 @@ rvk_status filter_apply(rvk_context *ctx, const rvk_filter *filter, const rvk_fi
         Exec ex{ctx, data, ts, IRect{}, src, {}, fe_image};
         Img res = ex.run(*filter);
         ex.source.reset();
-        res = into_cs(std::move(res), RVK_CI_SRGB);
         if (res->px == px) {
-            // the result is the layer itself (SourceGraphic passed through unchanged)
+            // the result is the layer itself (SourceGraphic passed through unchanged, sRGB)
         } else if (res->w == w && res->h == h) {
             // SourceOver onto a cleared pixmap of the same size is a copy
-            RVK_TRY(launch_copy(ctx, px, res->px, res->bytes()));
+            if (res->cs != RVK_CI_SRGB) RVK_TRY(launch_into_cs(ctx, px, res->px, w, h, 0));
+            else RVK_TRY(launch_copy(ctx, px, res->px, res->bytes()));
         } else {
+            res = into_cs(std::move(res), RVK_CI_SRGB);
             RVK_TRY(launch_fill_sub(ctx, px, w, h, 0, 0, w, h, 0u));
             RVK_TRY(launch_draw_pixmap(ctx, px, w, h, 0, 0, res->px, res->w, res->h, 1.0f, RVK_BLEND_SOURCE_OVER));
         }
@@ -411,11 +474,11 @@ extern "C" {
 
 rvk_status rvk_into_linear_rgb(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h) {
     CHECK_PX(ctx, px, w, h);
-    return rvk::launch_into_cs(ctx, px, w, h, 1);
+    return rvk::launch_into_cs(ctx, px, px, w, h, 1);
 }
 rvk_status rvk_into_srgb(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h) {
     CHECK_PX(ctx, px, w, h);
-    return rvk::launch_into_cs(ctx, px, w, h, 0);
+    return rvk::launch_into_cs(ctx, px, px, w, h, 0);
 }
 rvk_status rvk_demultiply_alpha(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h) {
     CHECK_PX(ctx, px, w, h);
@@ -462,7 +525,7 @@ rvk_status rvk_composite_arithmetic(rvk_context *ctx, const uint8_t *s1, const u
                                     uint32_t h, float k1, float k2, float k3, float k4) {
     CHECK_PX(ctx, dst, w, h);
     if (!s1 || !s2) return RVK_ERR_INVALID_ARGUMENT;
-    return rvk::launch_arithmetic(ctx, s1, s2, dst, (size_t)w * h, k1, k2, k3, k4);
+    return rvk::launch_arithmetic(ctx, s1, s2, dst, (size_t)w * h, k1, k2, k3, k4, 0);
 }
 rvk_status rvk_turbulence(rvk_context *ctx, uint8_t *dst, uint32_t w, uint32_t h, double ox, double oy, double sx,
                           double sy, double bfx, double bfy, uint32_t octaves, int32_t seed, uint32_t stitch,
@@ -481,7 +544,7 @@ rvk_status rvk_displacement_map(rvk_context *ctx, const uint8_t *src, const uint
                                 uint32_t h, float sx, float sy, float scale, uint32_t xch, uint32_t ych) {
     CHECK_PX(ctx, dst, w, h);
     if (!src || !map) return RVK_ERR_INVALID_ARGUMENT;
-    return rvk::launch_displacement(ctx, src, map, dst, w, h, sx, sy, scale, xch, ych);
+    return rvk::launch_displacement(ctx, src, map, dst, w, h, sx, sy, scale, xch, ych, 0);
 }
 rvk_status rvk_draw_pixmap(rvk_context *ctx, uint8_t *dst, uint32_t dw, uint32_t dh, int32_t x, int32_t y,
                            const uint8_t *src, uint32_t sw, uint32_t sh, float opacity, uint32_t mode) {

@@ -367,7 +367,8 @@ __global__ __launch_bounds__(64) void k_iir_chains(const uint8_t *in_u8, const d
 // x * h + y) -> the RGBA pixmap, through a 32 x 32 pixel tile in LDS.
 __global__ __launch_bounds__(256) void k_planes_to_rgba(const uint8_t *planes, uint32_t *px, uint32_t w, uint32_t h) {
     __shared__ uint8_t tile[4][32][33];
-    const uint32_t x0 = blockIdx.x * 32u, y0 = blockIdx.y * 32u, tx = threadIdx.x, ty = threadIdx.y;
+    const uint2 piece = xcd_tile();
+    const uint32_t x0 = piece.x * 32u, y0 = piece.y * 32u, tx = threadIdx.x, ty = threadIdx.y;
     const size_t plane = (size_t)w * h;
     for (uint32_t j = ty; j < 32u; j += 8u) {
         const uint32_t x = x0 + j, y = y0 + tx;

@@ -116,24 +116,23 @@ __global__ __launch_bounds__(kMThreads) void k_morph(const uint32_t *__restrict_
     const int cs = cw | 1;
     uint32_t *in = sm;              // rows x cs
     uint32_t *mid = sm + rows * cs;  // rows x ms
-    const int x0 = blockIdx.x * MTW, y0 = blockIdx.y * MTH;
+    const uint2 tile = xcd_tile();
+    const int x0 = (int)tile.x * MTW, y0 = (int)tile.y * MTH;
     const uint32_t id = ERODE ? 0xffffffffu : 0u;
-    // the tile and its halo, in chunks of 4 pixels aligned in memory: chunk c of a row
-    // holds global x in [a0 + 4c, a0 + 4c + 3]; 16-byte loads where the image and its
-    // rows are 16-byte aligned and the chunk lies inside the image, single pixels
-    // elsewhere
+    // the tile and its halo, in chunks of 4 pixels: chunk c of a row holds global x in
+    // [a0 + 4c, a0 + 4c + 3]; 16-byte loads (which need 4-byte alignment only) where the
+    // chunk lies inside the image, single pixels elsewhere
     const int gx0 = x0 - tx0, gy0 = y0 - ty0;
     const int a0 = gx0 & ~3;
     const int nc = (gx0 + cw - a0 + 3) >> 2;
     const float inv_nc = 1.0f / (float)nc;  // (i + 0.5) / nc truncates exactly for these sizes
-    const bool vec = (w & 3u) == 0 && (reinterpret_cast<uintptr_t>(src) & 15u) == 0;
     for (int i = threadIdx.x; i < rows * nc; i += kMThreads) {
         const int ly = (int)(((float)i + 0.5f) * inv_nc), c = i - ly * nc;
         const int gy = gy0 + ly, gx = a0 + 4 * c;
         uint32_t v[4];
-        if (gy >= 0 && gy < (int)h && vec && gx >= 0 && gx + 3 < (int)w) {
-            const uint4 q = *reinterpret_cast<const uint4 *>(src + (size_t)gy * w + gx);
-            v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+        if (gy >= 0 && gy < (int)h && gx >= 0 && gx + 3 < (int)w) {
+            const px4 q = *reinterpret_cast<const px4 *>(src + (size_t)gy * w + gx);
+            v[0] = q[0], v[1] = q[1], v[2] = q[2], v[3] = q[3];
         } else {
 #pragma unroll
             for (int e = 0; e < 4; e++)

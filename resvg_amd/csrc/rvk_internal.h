@@ -115,10 +115,15 @@ static inline bool valid_dims(uint32_t w, uint32_t h) {
 }
 
 // ---- kernel launchers (defined in the .hip files) ----
-rvk_status launch_into_cs(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, int to_linear);
+// src converted to dst, which may be src
+rvk_status launch_into_cs(rvk_context *ctx, uint8_t *dst, const uint8_t *src, uint32_t w, uint32_t h, int to_linear);
 rvk_status launch_demultiply(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h);
 rvk_status launch_multiply(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h);
 rvk_status launch_box_blur(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, double sx, double sy);
+// src -> dst with the work image tmp, three distinct buffers; tmp null: src is the work
+// image and lost
+rvk_status launch_box_blur_to(rvk_context *ctx, uint8_t *src, uint8_t *dst, uint8_t *tmp, uint32_t w, uint32_t h,
+                              double sx, double sy);
 // rvk_box_blur_noalloc: the back buffer is a file-scope device array of this size
 constexpr size_t kNoAllocBoxBlurBytes = (size_t)64 << 20;
 rvk_status noalloc_init(int device);  // looks the array up on `device` (current)
@@ -131,12 +136,15 @@ rvk_status launch_morphology_to(rvk_context *ctx, const uint8_t *src, uint8_t *d
                                 uint32_t op, float rx, float ry);
 rvk_status launch_convolve(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, const rvk_primitive *p,
                            const float *values);
+rvk_status launch_convolve_to(rvk_context *ctx, const uint8_t *src, uint8_t *dst, uint32_t w, uint32_t h,
+                              const rvk_primitive *p, const float *values);
 rvk_status launch_color_matrix(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, const rvk_primitive *p,
                                int fuse_alpha);
 rvk_status launch_component_transfer(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h,
                                      const rvk_primitive *p, const float *values, int fuse_alpha);
+// `whole`: every destination pixel is written (zero where the rule leaves it as it was)
 rvk_status launch_arithmetic(rvk_context *ctx, const uint8_t *s1, const uint8_t *s2, uint8_t *dst, size_t n,
-                             float k1, float k2, float k3, float k4);
+                             float k1, float k2, float k3, float k4, int whole);
 rvk_status launch_turbulence(rvk_context *ctx, uint8_t *dst, uint32_t w, uint32_t h, double ox, double oy,
                              double sx, double sy, double bfx, double bfy, uint32_t octaves, int32_t seed,
                              uint32_t stitch, uint32_t fractal, int premultiply);
@@ -145,9 +153,12 @@ rvk_status launch_lighting(rvk_context *ctx, const uint8_t *src, uint8_t *dst, u
                            const uint8_t color[4], const rvk_light_source *light);
 rvk_status launch_displacement(rvk_context *ctx, const uint8_t *src, const uint8_t *map, uint8_t *dst,
                                uint32_t w, uint32_t h, float sx, float sy, float scale, uint32_t xch,
-                               uint32_t ych);
+                               uint32_t ych, int whole);
 rvk_status launch_draw_pixmap(rvk_context *ctx, uint8_t *dst, uint32_t dw, uint32_t dh, int32_t x, int32_t y,
                               const uint8_t *src, uint32_t sw, uint32_t sh, float opacity, uint32_t mode);
+// dst = src blended onto below, n pixels; dst may be either
+rvk_status launch_blend_pair(rvk_context *ctx, uint8_t *dst, const uint8_t *below, const uint8_t *src, size_t n,
+                             uint32_t mode);
 rvk_status launch_fill(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, const uint8_t premul[4]);
 rvk_status launch_fill_sub(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, int64_t x0, int64_t y0,
                            int64_t x1, int64_t y1, uint32_t value);
@@ -160,7 +171,7 @@ rvk_status launch_copy(rvk_context *ctx, uint8_t *dst, const uint8_t *src, size_
 // of a sw x sh source, phase (ox, oy): feTile.
 rvk_status launch_tile(rvk_context *ctx, uint8_t *dst, uint32_t w, uint32_t h, const uint8_t *src, uint32_t sw,
                        uint32_t sh, uint32_t tx0, uint32_t ty0, uint32_t tw, uint32_t th, uint32_t ox, uint32_t oy);
-rvk_status launch_zero_rgb(rvk_context *ctx, uint8_t *px, size_t n);
+rvk_status launch_alpha_only(rvk_context *ctx, uint8_t *dst, const uint8_t *src, size_t n);
 // px = div255(px * m) per channel, m from `src` (0 alpha, 1 inverted alpha, 2 luminance)
 rvk_status launch_apply_mask(rvk_context *ctx, uint8_t *px, const uint8_t *src, size_t n, uint32_t mode);
 // tiny_skia::Mask operations on u8 planes of n bytes (mask 4-byte, pixmap 16-byte aligned)

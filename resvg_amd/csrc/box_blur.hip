@@ -27,14 +27,12 @@ __device__ __forceinline__ uint32_t round_pass(uint32_t s, float iarr) {
     return (uint32_t)rintf((float)s * iarr);
 }
 
-// The same rounding, as the bits of a float: the product rounded to f32 (no fused
-// multiply-add), plus 1.5 * 2^23, whose unit in the last place is 1, so the sum is
-// rounded to the nearest integer (ties to even) and that integer, at most 255, is the
-// low byte of the sum's bits.
+// The same integer, as the low byte of a float's bits: the product plus 1.5 * 2^23, whose
+// unit in the last place is 1.  The product isn't rounded by itself first, which makes no
+// difference: s / (2 r + 1) has an odd divisor and so stays 1 / (4 r + 2), at least 0.01,
+// away from every tie, and both products lie within 2^-15 of it.
 __device__ __forceinline__ uint32_t round_pass_bits(uint32_t s, float iarr) {
-#pragma clang fp contract(off)
-    const float prod = (float)s * iarr;
-    return __float_as_uint(prod + 12582912.0f);
+    return __float_as_uint(__builtin_fmaf((float)s, iarr, 12582912.0f));
 }
 
 // Sums four u8 channels of packed pixels into four 16-bit lanes of two u32s.
@@ -54,68 +52,76 @@ struct Acc {
 };
 
 // One round: dst = H_rh(V_rv(src)).  Tile covers output [x0, x0+TW) x [y0, y0+TH).
-// LDS: in[(TH + 2 rv) rows][(TW + 2 rh) cols], mid[TH rows][(TW + 2 rh) | 1 cols].
+// LDS: in[TH + 2 rv rows][TW + 2 rh cols, to whole chunks], mid[TH rows][(TW + 2 rh) | 1
+// cols].  Bound by the vector instructions of the passes and of the staging (a copy of a 4096^2
+// image takes 27 us): with LDS addresses by division and a checked store a pixel a round
+// of radii 3 took 46.4 us there, now 42.1; 1601 x 1131 9.3 us, now 8.3.
 __global__ __launch_bounds__(kThreads) void k_box_round(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst,
                                                         uint32_t w, uint32_t h, int rh, int rv) {
-    extern __shared__ uint32_t lds[];
+    extern __shared__ __align__(16) uint32_t lds[];
     const int cw = TW + 2 * rh;   // staged columns
     const int ch_ = TH + 2 * rv;  // staged rows
     const int ms = cw | 1;  // odd row stride of mid: the horizontal pass's lanes (rows) hit distinct banks
-    uint32_t *in = lds;
-    uint32_t *mid = lds + cw * ch_;
     const uint2 tile = xcd_tile();
     const int x0 = (int)tile.x * TW, y0 = (int)tile.y * TH;
-    // stage the input tile with zero padding outside the image (fv = lv = 0), in chunks
-    // of 4 pixels: chunk c of a tile row holds global x in [a0 + 4c, a0 + 4c + 3]; 16-byte
-    // loads (which need 4-byte alignment only) where the chunk lies inside the image,
-    // single pixels elsewhere.  With 16-byte loads for widths of a multiple of 4 alone a
-    // round over 1601 x 1131 took 15.8 us.
+    // the input tile with zero padding outside the image (fv = lv = 0), in chunks of 4
+    // pixels: chunk c of a tile row holds global x in [a0 + 4c, a0 + 4c + 3] and goes to
+    // LDS whole, so a row there starts up to 3 columns before the tile
+    const int gx0 = x0 - rh, gy0 = y0 - rv;
+    const int a0 = gx0 & ~3;
+    const int nc = (gx0 + cw - a0 + 3) >> 2, is = 4 * nc;
+    uint32_t *in = lds;
+    uint32_t *mid = lds + is * ch_;
+    // 16-byte loads (which need 4-byte alignment only) where the chunk lies inside the
+    // image, single pixels elsewhere
     {
-        const int gx0 = x0 - rh, gy0 = y0 - rv;
-        const int a0 = gx0 & ~3;
-        const int nc = (gx0 + cw - a0 + 3) >> 2;
         const float inv_nc = 1.0f / (float)nc;  // (i + 0.5) / nc truncates exactly for these sizes
-        for (int i = threadIdx.x; i < ch_ * nc; i += kThreads) {
-            const int ly = (int)(((float)i + 0.5f) * inv_nc), c = i - ly * nc;
-            const int gy = gy0 + ly, gx = a0 + 4 * c;
-            uint32_t v[4];
-            if (gy >= 0 && gy < (int)h && gx >= 0 && gx + 3 < (int)w) {
-                const px4 q = *reinterpret_cast<const px4 *>(src + (size_t)gy * w + gx);
-                v[0] = q[0], v[1] = q[1], v[2] = q[2], v[3] = q[3];
+        const bool inner = a0 >= 0 && a0 + is <= (int)w && gy0 >= 0 && gy0 + ch_ <= (int)h;
+        const uint32_t *corner = src + ((int64_t)gy0 * w + a0);  // dereferenced inside the image only
+        for (uint32_t i = threadIdx.x; i < (uint32_t)(ch_ * nc); i += kThreads) {
+            const uint32_t ly = (uint32_t)(((float)i + 0.5f) * inv_nc), c = i - __umul24(ly, nc);
+            uint4 v;
+            const uint32_t at = __umul24(ly, w) + 4 * c;  // ly < 2^7, w <= 2^16
+            const int gy = gy0 + (int)ly, gx = a0 + 4 * (int)c;
+            if (inner || (gy >= 0 && gy < (int)h && gx >= 0 && gx + 3 < (int)w)) {
+                const px4 q = *reinterpret_cast<const px4 *>(corner + at);
+                v = make_uint4(q[0], q[1], q[2], q[3]);
             } else {
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    v[e] = (gy >= 0 && gy < (int)h && gx + e >= 0 && gx + e < (int)w) ? src[(size_t)gy * w + gx + e] : 0u;
+                auto px = [&](int x) {
+                    return gy >= 0 && gy < (int)h && x >= 0 && x < (int)w ? src[(size_t)gy * w + x] : 0u;
+                };
+                v = make_uint4(px(gx), px(gx + 1), px(gx + 2), px(gx + 3));
             }
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int lx = gx + e - gx0;
-                if (lx >= 0 && lx < cw) in[ly * cw + lx] = v[e];
-            }
+            reinterpret_cast<uint4 *>(in)[i] = v;
         }
     }
+    in += gx0 - a0;
     __syncthreads();
     // vertical pass: each thread walks one staged column over TH/segs rows
     if (rv == 0) {
         for (int i = threadIdx.x; i < cw * TH; i += kThreads) {
             const int ly = i / cw;
-            mid[ly * ms + (i - ly * cw)] = in[i];
+            mid[ly * ms + (i - ly * cw)] = in[ly * is + (i - ly * cw)];
         }
     } else {
         const float iarr = 1.0f / (float)(2 * rv + 1);
         // two segments of TH / 2 rows per column: every column's 2 jobs fit one pass of
         // the block (cw <= 112), and the window sum is started (2 rv + 1 adds) only twice
-        const int segs = 2, seg_len = TH / segs;
-        for (int job = threadIdx.x; job < cw * segs; job += kThreads) {
-            int col = job % cw, seg = job / cw;
-            int t0 = seg * seg_len;
+        constexpr int segs = 2, seg_len = TH / segs;
+        static_assert(segs * (TW + 2 * kMaxFusedR) <= kThreads, "a job a thread");
+        const int seg = (int)threadIdx.x >= cw, col = (int)threadIdx.x - (seg ? cw : 0);
+        if (col < cw) {
+            const uint32_t *head = in + seg * seg_len * is + col, *tail = head;
+            uint32_t *m = mid + seg * seg_len * ms + col;
             Acc acc; acc.zero();
-            for (int k = 0; k <= 2 * rv; k++) acc.add(in[(t0 + k) * cw + col]);
-            mid[t0 * ms + col] = acc.out(iarr);
-            for (int t = t0 + 1; t < t0 + seg_len; t++) {
-                acc.add(in[(t + 2 * rv) * cw + col]);
-                acc.sub(in[(t - 1) * cw + col]);
-                mid[t * ms + col] = acc.out(iarr);
+            for (int k = 0; k <= 2 * rv; k++, head += is) acc.add(*head);
+            *m = acc.out(iarr);
+#pragma unroll 5
+            for (int t = 1; t < seg_len; t++) {
+                acc.add(*head);
+                acc.sub(*tail);
+                head += is, tail += is, m += ms;
+                *m = acc.out(iarr);
             }
         }
     }
@@ -229,7 +235,8 @@ static void box_gauss_sizes(float sigma, int32_t out[5]) {
 
 // one fused round, a to b (both radii at most kMaxFusedR)
 static rvk_status box_round(rvk_context *ctx, const uint32_t *a, uint32_t *b, uint32_t w, uint32_t h, int rh, int rv) {
-    size_t lds = (size_t)((TW + 2 * rh) * (TH + 2 * rv) + ((TW + 2 * rh) | 1) * TH) * 4;
+    // a staged row: at most 3 columns before and 3 behind the tile's
+    size_t lds = (size_t)(((TW + 2 * rh + 6) & ~3) * (TH + 2 * rv) + ((TW + 2 * rh) | 1) * TH) * 4;
     dim3 grid(div_up(w, TW), div_up(h, TH));
     // algorithmic bytes: the image read once and written once per blur (8 B/px,
     // whatever the pass count), split evenly over the five rounds

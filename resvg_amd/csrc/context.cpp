@@ -97,6 +97,27 @@ void scratch_release(rvk_context *ctx, void *p) {
     }
 }
 
+rvk_status result_slot(rvk_context *ctx, void **out) {
+    {
+        std::lock_guard<std::mutex> g(ctx->mu);
+        if (!ctx->result_slots.empty()) {
+            *out = ctx->result_slots.back();
+            ctx->result_slots.pop_back();
+            return RVK_OK;
+        }
+    }
+    if (hipHostMalloc(out, 16, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return RVK_ERR_OUT_OF_MEMORY;
+    }
+    return RVK_OK;
+}
+
+void result_release(rvk_context *ctx, void *slot) {
+    std::lock_guard<std::mutex> g(ctx->mu);
+    ctx->result_slots.push_back(slot);
+}
+
 rvk_status lanes_prepare(rvk_context *ctx, uint32_t n) {
     while (ctx->lanes.size() < n) {
         rvk_context *l = new rvk_context();
@@ -265,6 +286,7 @@ rvk_status rvk_context_destroy(rvk_context *ctx) {
     }
     for (auto &f : ctx->free_list) (void)hipFree(f.second);
     for (auto &f : ctx->live) (void)hipFree(f.second);
+    for (void *s : ctx->result_slots) (void)hipHostFree(s);
     if (ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return RVK_OK;

@@ -557,6 +557,14 @@ rvk_status launch_upload(hipStream_t stream, void *dev_dst, const void *pinned_s
     return RVK_OK;
 }
 
+rvk_status launch_download(hipStream_t stream, void *pinned_dst, const void *dev_src) {
+    void *dst = nullptr;
+    RVK_HIP_CHECK(hipHostGetDevicePointer(&dst, pinned_dst, 0));
+    hipLaunchKernelGGL(k_copy, dim3(1), dim3(64), 0, stream, (uint4 *)dst, (const uint4 *)dev_src, (size_t)1);
+    RVK_HIP_CHECK(hipGetLastError());
+    return RVK_OK;
+}
+
 }  // namespace rvk
 
 namespace rvkh {

@@ -95,7 +95,7 @@ constexpr int kExpandSteps = 64;   // curve segments after the first piece (MAX_
 // and shift, into LDS; then each half of the wave takes an edge at a time, a lane per
 // segment: the slope's division (most of the work), and the non-empty pieces compacted in
 // order and stored together.  One thread per edge doing both took 15-30 us however few
-// edges there were (30 -> 7 us per launch of a 2048^2 document's clip paths).
+// edges there were (29.8 -> 11.6 us per launch of a 2048^2 document's clip paths).
 template <int E>
 __global__ __launch_bounds__(kWave) void k_expand(ExpandArgs a) {
     __shared__ int2 pts[E][kExpandSteps + 1];  // 16.16 points, the first piece's end first
@@ -516,7 +516,7 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 // variant's VALU 13% busy).  Per row the old form issued 2400 VALU, 1600 SALU and 450 LDS
 // wave instructions, the LDS pipe as busy as the VALU; scans and sort exchanges moved to
 // DPP, winding prefixes to ballots, and differences instead of two packed sums.  With
-// 28 KB of LDS and 32 VGPRs the 128 variant runs 8 waves per SIMD (4 before).  Renders:
+// 37 KB of LDS and 38 VGPRs the 128 variant runs 8 waves per SIMD (4 before).  Renders:
 // 4096^2, 2000 paths 150.4 -> 120.7 ms; 1201x843, 64 paths 3.36 -> 1.95 ms; 2048^2 with
 // 150 clipped or masked groups 90.1 -> 64.6 ms; 64 documents in a batch 109 -> 87 ms.
 template <int MK>
@@ -1654,6 +1654,9 @@ rvk_status launch_expand(rvk_context *ctx, const EdgeRec *edges, uint32_t nedges
                          PieceDev *pieces, uint32_t *npieces, int32_t *overflow, double algo_bytes) {
     if (nedges == 0) return RVK_OK;
     ExpandArgs a{edges, nedges, cov, pieces, npieces, overflow};
+    // few edges: four a wave, so that there are enough waves (the clip paths above took
+    // 16.4 us with 16 a wave, 11.6 with 4); past 1024 waves of 16 the chip is full either
+    // way and the second half of the kernel fills more lanes
     timed_launch(ctx, "expand", algo_bytes, [&] {
         if (nedges > 16384u) hipLaunchKernelGGL(k_expand<16>, dim3(div_up(nedges, 16)), dim3(kWave), 0, ctx->stream, a);
         else hipLaunchKernelGGL(k_expand<4>, dim3(div_up(nedges, 4)), dim3(kWave), 0, ctx->stream, a);

@@ -1242,13 +1242,15 @@ rvk_status render_walk(rvk_context *ctx, const rvk_scene *scene, Ts ts, uint32_t
                        uint64_t *overflow_rows, Walk walk, rvk_node_ref node, const IRect *max_bbox) {
     Renderer r{ctx, *scene, max_bbox ? *max_bbox : max_filter_bbox(w, h)};
     r.build_aux();
-    void *ovbuf = nullptr;
+    void *ovbuf = nullptr, *result = nullptr;
     RVK_TRY(rvk::scratch_alloc(ctx, 256, &ovbuf));
     r.dev_overflow = (int32_t *)ovbuf;
     {
-        const rvk_status s = rvk::launch_fill_sub(ctx, (uint8_t *)ovbuf, 1, 1, 0, 0, 1, 1, 0u);  // counter = 0
+        rvk_status s = rvk::result_slot(ctx, &result);
+        if (s == RVK_OK) s = rvk::launch_fill_sub(ctx, (uint8_t *)ovbuf, 4, 1, 0, 0, 4, 1, 0u);  // counter = 0
         if (s != RVK_OK) {
             rvk::scratch_release(ctx, ovbuf);
+            if (result) rvk::result_release(ctx, result);
             return s;
         }
     }
@@ -1278,13 +1280,16 @@ rvk_status render_walk(rvk_context *ctx, const rvk_scene *scene, Ts ts, uint32_t
     run(root);
     if (r.err == RVK_OK) r.fail(r.flush(root));
     r.fail(r.finish_flushes());  // the side stream joins the context stream
-    // the one wait of a render: read the overflow counter
+    // the one wait of a render: read the overflow counter, which a kernel stores to pinned
+    // memory (copied to pageable memory instead, a filtered
+    // 512^2 path took 160 us, now 130)
     int32_t ov = 0;
     {
         const auto t0 = std::chrono::steady_clock::now();
-        hipError_t e = hipMemcpyAsync(&ov, ovbuf, 4, hipMemcpyDeviceToHost, ctx->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-        if (e != hipSuccess) {
+        const rvk_status s = rvk::launch_download(ctx->stream, result, ovbuf);
+        const hipError_t e = hipStreamSynchronize(ctx->stream);
+        if (s == RVK_OK && e == hipSuccess) ov = *(const volatile int32_t *)result;
+        if (s != RVK_OK || e != hipSuccess) {
             (void)hipGetLastError();
             r.fail(RVK_ERR_HIP);
         }
@@ -1292,6 +1297,7 @@ rvk_status render_walk(rvk_context *ctx, const rvk_scene *scene, Ts ts, uint32_t
             std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
     rvk::scratch_release(ctx, ovbuf);
+    rvk::result_release(ctx, result);
     for (void *t : r.pattern_tiles) rvk::scratch_release(ctx, t);
     r.overflow_rows = (uint64_t)(ov > 0 ? ov : 0);
     if (overflow_rows) *overflow_rows = r.overflow_rows;

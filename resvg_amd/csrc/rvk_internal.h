@@ -51,6 +51,8 @@ struct rvk_context {
     // Simple size-bucketed cache of device scratch buffers (layers, filter images).
     std::vector<std::pair<size_t, void *>> free_list;
     std::vector<std::pair<size_t, void *>> live;
+    // Pinned 16-byte results of renders (see result_slot): one per render under way.
+    std::vector<void *> result_slots;
     std::mutex mu;
     // Sub-contexts with their own streams, scratch caches and staging rings on the
     // same device; rvk_render_batch spreads documents over them.
@@ -69,6 +71,10 @@ void set_last_error(const char *what, const char *where);
 // Scratch device memory owned by the context (returned to its cache on release).
 rvk_status scratch_alloc(rvk_context *ctx, size_t bytes, void **out);
 void scratch_release(rvk_context *ctx, void *p);
+// 16 bytes of pinned host memory from the context's pool, for launch_download; back to
+// the pool with result_release once the stream has been waited for
+rvk_status result_slot(rvk_context *ctx, void **out);
+void result_release(rvk_context *ctx, void *slot);
 
 // Copies host memory to the device on the context stream and waits for it.
 rvk_status upload_sync(rvk_context *ctx, void *dev_dst, const void *host_src, size_t bytes);
@@ -166,6 +172,8 @@ rvk_status launch_fill_sub(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h
 // by a kernel on `stream`
 constexpr size_t kKernelUploadBytes = (size_t)1 << 20;
 rvk_status launch_upload(hipStream_t stream, void *dev_dst, const void *pinned_src, size_t bytes);
+// 16 bytes of device memory into pinned host memory, by a kernel on `stream`
+rvk_status launch_download(hipStream_t stream, void *pinned_dst, const void *dev_src);
 rvk_status launch_copy(rvk_context *ctx, uint8_t *dst, const uint8_t *src, size_t bytes);
 // Fills a w x h image with the periodic repeat of the tw x th tile at (tx0, ty0)
 // of a sw x sh source, phase (ox, oy): feTile.

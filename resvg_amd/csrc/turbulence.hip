@@ -1,5 +1,7 @@
 // feTurbulence (crates/resvg/src/filter/turbulence.rs).  Write-only and FP64-VALU
-// bound: per pixel and channel an octave loop of Perlin noise2 in f64.  The
+// bound: per pixel an octave loop of Perlin noise2 in f64, the four channels together
+// (with a loop per channel, which finds the lattice cell four times, and a division a
+// term, 1601 x 1131 pixels took 132 us, now 56).  The
 // Park–Miller seeded lattice and gradient tables (turbulence.rs:93-140) are built on
 // the host and staged into LDS per workgroup (34.9 KB); every f64 operation follows
 // the reference's order, so the output is bit-identical.

@@ -121,3 +121,22 @@ def test_results_used_again(ctx, seed):
     t, e = _dev(layer), layer.copy()
     assert ctx.filter_apply(g, ts, t) == orc.filter_apply(g, ts, e)
     assert np.array_equal(t.cpu().numpy(), e)
+
+
+@pytest.mark.parametrize("order", [(5, 5), (7, 9), (64, 1), (1, 64), (1, 1)])
+@pytest.mark.parametrize("edge", [abi.EDGE_NONE, abi.EDGE_DUPLICATE, abi.EDGE_WRAP])
+@pytest.mark.parametrize("shape", [(1, 1), (3, 2), (17, 65), (33, 130)])
+def test_convolution_tiles(ctx, order, edge, shape):
+    # both kernels (a tile of 64 x 16 with its halo in LDS, or straight from memory), images
+    # smaller and larger than a tile and than the matrix, an infinite coefficient
+    rng = np.random.default_rng(order[0] * 100 + order[1] + edge)
+    k = rng.uniform(-1, 1, order[0] * order[1])
+    for k0, preserve in ((k[0], False), (k[0], True), (float("inf"), False)):
+        k[0] = k0
+        g = FilterGraph((0, 0, 1, 1))
+        g.convolve_matrix(order[0], order[1], k, 1.5, 0.1, edge_mode=edge, preserve_alpha=preserve)
+        px = _random(*shape, 7)
+        t, e = _dev(px), px.copy()
+        ctx.convolve_matrix(t, g.primitives[0], g.values)
+        orc.convolve_matrix(e, g.primitives[0], g.values)
+        assert np.array_equal(t.cpu().numpy(), e), (k0, preserve)

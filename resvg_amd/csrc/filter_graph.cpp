@@ -152,12 +152,13 @@ struct Exec {
     }
 
     Img blur(Img im, double sx, double sy, bool box) {
+        const bool own = im.use_count() == 1 && im->owned;
         if (!box) {
-            Img out = take(std::move(im));
-            FTRY(rvk::launch_iir_blur(ctx, out->px, out->w, out->h, sx, sy));
+            Img out = own ? im : new_img(ctx, im->w, im->h, im->cs, false);
+            FTRY(rvk::launch_iir_blur(ctx, im->px, out->px, out->w, out->h, sx, sy));
             return out;
         }
-        const bool own = im.use_count() == 1 && im->owned;  // then it is the work image
+        // an image of its own is the work image
         Img out = new_img(ctx, im->w, im->h, im->cs, false);
         Img tmp = own ? nullptr : new_img(ctx, im->w, im->h, im->cs, false);
         FTRY(rvk::launch_box_blur_to(ctx, im->px, out->px, own ? nullptr : tmp->px, im->w, im->h, sx, sy));
@@ -498,7 +499,7 @@ rvk_status rvk_box_blur_noalloc(rvk_context *ctx, uint8_t *px, uint32_t w, uint3
 }
 rvk_status rvk_iir_blur(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, double sx, double sy) {
     CHECK_PX(ctx, px, w, h);
-    return rvk::launch_iir_blur(ctx, px, w, h, sx, sy);
+    return rvk::launch_iir_blur(ctx, px, px, w, h, sx, sy);
 }
 rvk_status rvk_morphology(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, uint32_t op, float rx, float ry) {
     CHECK_PX(ctx, px, w, h);

@@ -439,15 +439,15 @@ static void launch_chains(hipStream_t st, const uint8_t *in_u8, const double *in
 
 // Both sides at most kChainMax: rows (u8 in, f64 plane out) then columns (f64 in, u8
 // out), or one of them u8 to u8, or (both sigmas off) only the conversion round trip.
-static rvk_status iir_on_chip(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, bool rows, bool cols,
-                              double dx, double dy, double post) {
+static rvk_status iir_on_chip(rvk_context *ctx, const uint8_t *src, uint8_t *px, uint32_t w, uint32_t h, bool rows,
+                              bool cols, double dx, double dy, double post) {
     const size_t n = (size_t)w * h;
     const uint32_t n32 = (uint32_t)n;
     // algorithmic bytes of the whole blur: the u8 image read once and written once
     const double pxb = 4.0 * (double)n;
     if (!cols) {  // rows only, or (both sigmas off) the conversion round trip
         timed_launch(ctx, "iir_rows", 2.0 * pxb, [&] {
-            launch_chains(ctx->stream, px, nullptr, px, nullptr, w, h, 1u, w, n32, dx, rows ? 4 : 0, post, 0);
+            launch_chains(ctx->stream, src, nullptr, px, nullptr, w, h, 1u, w, n32, dx, rows ? 4 : 0, post, 0);
         });
         RVK_HIP_CHECK(hipGetLastError());
         return RVK_OK;
@@ -474,7 +474,7 @@ static rvk_status iir_on_chip(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_
     double *planes = (double *)pa, *tplanes = (double *)pt;
     if (rows) {
         timed_launch(ctx, "iir_rows", pxb, [&] {
-            launch_chains(ctx->stream, px, nullptr, nullptr, planes, w, h, 1u, w, n32, dx, 4, 1.0, 0);
+            launch_chains(ctx->stream, src, nullptr, nullptr, planes, w, h, 1u, w, n32, dx, 4, 1.0, 0);
         });
         if (transposed) {
             // row-major planes (h rows of w) read as column-major ones of h x w
@@ -492,7 +492,7 @@ static rvk_status iir_on_chip(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_
         }
     } else {
         timed_launch(ctx, "iir_cols", pxb, [&] {
-            launch_chains(ctx->stream, px, nullptr, cplanes, nullptr, h, w, w, 1u, n32, dy, 4, post, 1);
+            launch_chains(ctx->stream, src, nullptr, cplanes, nullptr, h, w, w, 1u, n32, dy, 4, post, 1);
         });
     }
     timed_launch(ctx, "iir_interleave", pxb, [&] {
@@ -507,7 +507,8 @@ static rvk_status iir_on_chip(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_
     return RVK_OK;
 }
 
-rvk_status launch_iir_blur(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, double sx, double sy) {
+rvk_status launch_iir_blur(rvk_context *ctx, const uint8_t *src, uint8_t *px, uint32_t w, uint32_t h, double sx,
+                           double sy) {
     double lx = 1.0, dx = 1.0, ly = 1.0, dy = 1.0;
     if (sx > 0.0) coefficients(sx, &lx, &dx);
     if (sy > 0.0) coefficients(sy, &ly, &dy);
@@ -521,7 +522,8 @@ rvk_status launch_iir_blur(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h
     // on chip: both sides within kChainMax and each coefficient in (0, 1) (it is for
     // every finite positive sigma; the zero-start argument needs dnu * 0 == 0)
     const bool coef_ok = (!(sx > 0.0) || (dx > 0.0 && dx < 1.0)) && (!(sy > 0.0) || (dy > 0.0 && dy < 1.0));
-    if (w <= kChainMax && h <= kChainMax && coef_ok) return iir_on_chip(ctx, px, w, h, sx > 0.0, sy > 0.0, dx, dy, post);
+    if (w <= kChainMax && h <= kChainMax && coef_ok)
+        return iir_on_chip(ctx, src, px, w, h, sx > 0.0, sy > 0.0, dx, dy, post);
     size_t bytes = n * 4 * sizeof(double);
     void *pa = nullptr, *pb = nullptr;
     RVK_TRY(scratch_alloc(ctx, bytes, &pa));
@@ -535,7 +537,7 @@ rvk_status launch_iir_blur(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h
     // planes are this implementation's intermediates and are not credited
     const double pxb = 4.0 * (double)n;
     timed_launch(ctx, "iir_to_f64", pxb, [&] {
-        hipLaunchKernelGGL(k_to_f64_colmajor, tgrid, tblk, 0, ctx->stream, (const uint32_t *)px, colmajor, w, h);
+        hipLaunchKernelGGL(k_to_f64_colmajor, tgrid, tblk, 0, ctx->stream, (const uint32_t *)src, colmajor, w, h);
     });
     if (sx > 0.0) {
         timed_launch(ctx, "iir_rows", 0.0, [&] {

@@ -134,7 +134,9 @@ rvk_status launch_box_blur_to(rvk_context *ctx, uint8_t *src, uint8_t *dst, uint
 constexpr size_t kNoAllocBoxBlurBytes = (size_t)64 << 20;
 rvk_status noalloc_init(int device);  // looks the array up on `device` (current)
 rvk_status launch_box_blur_noalloc(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, double sx, double sy);
-rvk_status launch_iir_blur(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, double sx, double sy);
+// src -> px, which may be src
+rvk_status launch_iir_blur(rvk_context *ctx, const uint8_t *src, uint8_t *px, uint32_t w, uint32_t h, double sx,
+                           double sy);
 rvk_status launch_morphology(rvk_context *ctx, uint8_t *px, uint32_t w, uint32_t h, uint32_t op, float rx,
                              float ry);
 // src -> dst, distinct buffers

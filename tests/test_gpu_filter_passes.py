@@ -140,3 +140,19 @@ def test_convolution_tiles(ctx, order, edge, shape):
         ctx.convolve_matrix(t, g.primitives[0], g.values)
         orc.convolve_matrix(e, g.primitives[0], g.values)
         assert np.array_equal(t.cpu().numpy(), e), (k0, preserve)
+
+
+@pytest.mark.parametrize("sig", [(1.2, 0.7), (0.0, 1.1), (1.4, 0.0)])
+@pytest.mark.parametrize("shape", [(38, 125), (5, 3)])
+def test_small_blur_of_a_shared_image(ctx, sig, shape):
+    # the IIR blur reads the layer, or a result that is used again, and writes its own image
+    h, w = shape
+    g = FilterGraph((0, 0, w, h))
+    a = g.gaussian_blur(*sig, cs=abi.CI_SRGB)
+    b = g.gaussian_blur(*sig, in1=a, cs=abi.CI_SRGB)
+    g.merge([a, b, SOURCE_GRAPHIC], cs=abi.CI_SRGB)
+    layer = _random(h, w, 5, 0.3)
+    t, e = _dev(layer), layer.copy()
+    ts = abi.Transform(1.0, 0.0, 0.0, 1.0, 0.0, 0.0)
+    assert ctx.filter_apply(g, ts, t) == orc.filter_apply(g, ts, e)
+    assert np.array_equal(t.cpu().numpy(), e)

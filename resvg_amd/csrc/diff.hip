@@ -134,14 +134,14 @@ __device__ __forceinline__ void segment_coverage(const Cov &cv, const Dims &d, u
 // ---- paint ------------------------------------------------------------------
 // What the path kernels read of a path, in scalar registers (written by k_diff_prepare): the
 // gradient's start and direction, its squared length and that one's reciprocal, tint,
-// opacity and offsets; then per stop interval its lower offset, width, the width's
-// reciprocal and the two stops.
+// opacity and offsets; `one`, whether the wave may draw it by one interval's record; then per
+// stop interval its lower offset, width, the width's reciprocal and the two stops.
 struct Interval {
     float lo, span, rs, pad;
     float c0[4], c1[4];
 };
 struct PathHead {
-    float x0, y0, dx, dy, dd, rdd, opacity, tint[3], o0, o1, o2, o3, rs_min, pad;
+    float x0, y0, dx, dy, dd, rdd, opacity, tint[3], o0, o1, o2, o3, one, pad;
 };
 struct PathRec {
     PathHead head;
@@ -196,12 +196,14 @@ __device__ __forceinline__ Along along_path(const PathHead &h, float px, float p
     e.inside = ~(before | __ballot(t >= h.o3));
     return e;
 }
-// Whether the covered pixels of the wave (touched, not none) share a stop interval, k0, of a
-// width that div_by takes.
+// Whether the covered pixels of the wave (touched, not none) share a stop interval, k0, and
+// the path's record is one for it: widths that div_by takes, and paint whose products with
+// a zero coverage are zeros (a non-finite value would reach the uncovered pixels, which
+// only the form for several intervals keeps apart).
 __device__ __forceinline__ bool one_interval(const PathHead &h, const Along &e, uint64_t touched, int &k0) {
     const uint64_t a = e.past1 & touched, b = e.past2 & touched;
     k0 = __builtin_amdgcn_readfirstlane(b != 0 ? 2 : (a != 0 ? 1 : 0));
-    return (a == 0 || a == touched) && (b == 0 || b == touched) && h.rs_min != 0.0f;
+    return (a == 0 || a == touched) && (b == 0 || b == touched) && h.one != 0.0f;
 }
 
 // A pixel's stop colour (unpremultiplied) and where it lies between the stops.
@@ -382,7 +384,9 @@ __global__ void k_diff_prepare(Dims d, const float *params, const float4 *ends, 
         h.o1 = off[1];
         h.o2 = off[2];
         h.o3 = off[3];
-        h.rs_min = 1.0f;
+        h.one = 1.0f;
+        for (int k = 0; k < 20; k++)
+            if (!(fabsf(pp[k]) < 0x1p60f)) h.one = 0.0f;
         h.pad = 0.0f;
         for (int k = 0; k < 3; k++) {
             Interval &iv = r.iv[k];
@@ -390,7 +394,7 @@ __global__ void k_diff_prepare(Dims d, const float *params, const float4 *ends, 
             iv.span = off[k + 1] - off[k];
             iv.rs = div_ready(iv.span);
             iv.pad = 0.0f;
-            if (iv.rs == 0.0f) h.rs_min = 0.0f;
+            if (iv.rs == 0.0f) h.one = 0.0f;
             for (int ch = 0; ch < 4; ch++) {
                 iv.c0[ch] = pp[4 + 4 * k + ch];
                 iv.c1[ch] = pp[8 + 4 * k + ch];
@@ -734,7 +738,8 @@ __global__ __launch_bounds__(kPathThreads, kArea ? 4 : 5) void k_diff_paths_bwd(
             float v = 0.0f;     // this wave's sum of the path's gradient `lane`
             const uint64_t touched = __ballot(c != 0.0f);
             if (touched != 0) {
-                // every lane evaluates; those without coverage (A = 0) contribute zeros
+                // every lane evaluates; those without coverage contribute zeros, whatever
+                // their dL/dS and canvas hold: A is 0 there and gc and gA are set to it
                 const Along e = along_path(h, px, py);
                 const float4 sb = canv[j];
                 int k0;
@@ -749,10 +754,13 @@ __global__ __launch_bounds__(kPathThreads, kArea ? 4 : 5) void k_diff_paths_bwd(
                 } else {
                     st = stop_any(r, k, e.t, h.o0, h.o3);
                 }
-                const float A = c * h.opacity * st.rgba[3];
+                float A = c * h.opacity * st.rgba[3];
+                if (!one && c == 0.0f) A = 0.0f;  // with `one` it is
                 // after = (rgb·tint·A, A) + (1 - A)·before
-                const float gc[3] = {g.x, g.y, g.z};
+                const bool on = c != 0.0f;
+                const float gc[3] = {on ? g.x : 0.0f, on ? g.y : 0.0f, on ? g.z : 0.0f};
                 float gA = g.w - fmaf(g.w, sb.w, fmaf(g.z, sb.z, fmaf(g.y, sb.y, g.x * sb.x)));
+                gA = on ? gA : 0.0f;
                 float gt[4];    // tint, opacity
                 float gcol[4];  // interpolated stop colour and alpha
 #pragma unroll
@@ -765,7 +773,7 @@ __global__ __launch_bounds__(kPathThreads, kArea ? 4 : 5) void k_diff_paths_bwd(
                 const float gAc = gA * c, gAo = gA * h.opacity;
                 gt[3] = gAc * st.rgba[3];
                 gcol[3] = gAc * h.opacity;
-                gcov = c != 0.0f ? gAo * st.rgba[3] : 0.0f;
+                gcov = on ? gAo * st.rgba[3] : 0.0f;
                 const float ia = 1.0f - A;
                 g = make_float4(g.x * ia, g.y * ia, g.z * ia, g.w * ia);
                 const bool in = (e.inside >> lane) & 1;
@@ -794,7 +802,7 @@ __global__ __launch_bounds__(kPathThreads, kArea ? 4 : 5) void k_diff_paths_bwd(
                     float gu = 0.0f;
                     for (int ch = 0; ch < 4; ch++) gu = fmaf(gcol[ch], lv.c1[ch] - lv.c0[ch], gu);
                     float ga_lo = 0.0f, ga_hi = 0.0f;
-                    if (in && lv.span > 0.0f && c != 0.0f) {
+                    if (in && lv.span > 0.0f && on) {
                         ga_lo = gu * -(1.0f - st.u) / lv.span;
                         ga_hi = gu * -st.u / lv.span;
                     }
@@ -804,9 +812,9 @@ __global__ __launch_bounds__(kPathThreads, kArea ? 4 : 5) void k_diff_paths_bwd(
                                          k == 2 ? w0 : (k == 1 ? w1 : 0.0f), k == 2 ? w1 : 0.0f};
 #pragma unroll
                     for (int ch = 0; ch < 4; ch++) {
-                        gp[ch] = c != 0.0f ? gt[ch] : 0.0f;
+                        gp[ch] = on ? gt[ch] : 0.0f;
 #pragma unroll
-                        for (int q = 0; q < 4; q++) gp[4 + 4 * q + ch] = c != 0.0f ? gcol[ch] * ws[q] : 0.0f;
+                        for (int q = 0; q < 4; q++) gp[4 + 4 * q + ch] = on ? gcol[ch] * ws[q] : 0.0f;
                     }
                     gp[20] = k == 0 ? ga_lo : 0.0f;
                     gp[21] = k == 1 ? ga_lo : (k == 0 ? ga_hi : 0.0f);

@@ -68,3 +68,59 @@ def test_long_area_rows_match_short_ones(ctx, w):
         outs.append(r.forward(torch.as_tensor(p0, device="cuda"), r.geom0).cpu().numpy()[:, :8000])
     assert np.abs(outs[0]).max() > 0.1
     assert np.array_equal(outs[0], outs[1])
+
+
+# ---- non-finite values stay where they are -----------------------------------------
+def _rect(x0, x1, h):
+    from resvg_amd import abi
+    pts = [(x0, 0), (x1, 0), (x1, h), (x0, h)]
+    return [abi.VERB_MOVE, abi.VERB_LINE, abi.VERB_LINE, abi.VERB_LINE, abi.VERB_CLOSE], np.asarray(pts, np.float32)
+
+
+def _columns(ctx, w, h, spans, wide):
+    """Opaque-edged columns x0 <= x < x1 under a zero colour matrix: the picture is the paths'
+    canvas and, within the blur's reach of finite pixels, dL/d(canvas) is dL/d(picture), so a
+    path's gradient comes from its pixels alone.
+    `wide`: the gradients' stops far apart (a wave in one interval) or close (in several)."""
+    n = len(spans)
+    rng = np.random.default_rng(7)
+    ends = np.float32([(-200.0, 0.0, 300.0, 0.0) if wide else (x0, 0.0, x1, 0.0) for x0, x1 in spans])
+    p = np.zeros(diff.n_params(n), np.float32)
+    for i in range(n):
+        q = p[i * diff.PATH_PARAMS:(i + 1) * diff.PATH_PARAMS]
+        q[:20] = rng.uniform(0.3, 0.9, 20)
+        q[20:24] = (0.1, 0.3, 0.6, 0.9)
+    p[n * diff.PATH_PARAMS] = 0.05  # radius 1
+    return diff.Renderer(ctx, w, h, [_rect(x0, x1, h) for x0, x1 in spans], ends), p
+
+
+def _grad(r, p, go):
+    import torch
+    params = torch.as_tensor(p, device="cuda")
+    r.forward(params)
+    return r.backward(params, torch.as_tensor(go, device="cuda")).cpu().numpy()
+
+
+@pytest.mark.parametrize("wide", [True, False])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_upstream_at_uncovered_pixels(ctx, value, wide):
+    # the gradient of a path does not depend on dL/d(picture) where it has no coverage, also
+    # where its wave of 16 x 4 pixels has some
+    r, p = _columns(ctx, 16, 4, [(0, 8)], wide)
+    go = np.random.default_rng(1).normal(0.0, 1.0, (4, 16, 4)).astype(np.float32)
+    want = _grad(r, p, go)[:diff.PATH_PARAMS]
+    go[1, 12] = value
+    assert np.isfinite(want).all() and want.any()
+    assert np.array_equal(_grad(r, p, go)[:diff.PATH_PARAMS], want)
+
+
+@pytest.mark.parametrize("wide", [True, False])
+@pytest.mark.parametrize("param,value", [(0, np.nan), (3, np.inf), (3, np.nan), (7, np.inf), (11, np.nan)])
+def test_paint_at_uncovered_pixels(ctx, param, value, wide):
+    # nor on the paint of another path over other pixels of the wave
+    r, p = _columns(ctx, 16, 4, [(10, 16), (0, 2)], wide)
+    go = np.random.default_rng(2).normal(0.0, 1.0, (4, 16, 4)).astype(np.float32)
+    want = _grad(r, p, go)[:diff.PATH_PARAMS]
+    p[diff.PATH_PARAMS + param] = value
+    assert np.isfinite(want).all() and want.any()
+    assert np.array_equal(_grad(r, p, go)[:diff.PATH_PARAMS], want)

@@ -459,16 +459,31 @@ inline uint32_t blur_blocks_x(uint32_t w, uint32_t h) { return ((w + 255) / 256)
 
 template <int N> struct Weights { float w[N]; };
 
-// adds input v's contribution to N outputs o: weight k = o - i (or its mirror i - o)
+// adds input i's value v to outputs lo .. hi - 1 of N: weight k = o - i (or its mirror i - o)
 template <int N>
-__device__ __forceinline__ void blur_add(float4 (&acc)[N], const float *w, int R, int i, float4 v) {
+__device__ __forceinline__ void blur_add(float4 (&acc)[N], const float *w, int R, int i, float4 v, int lo, int hi) {
     const Weights<N> k = scalar_rec(reinterpret_cast<const Weights<N> *>(w + kWeightPad + R - i));
 #pragma unroll
     for (int o = 0; o < N; o++) {
+        if (o < lo || o >= hi) continue;
         acc[o].x = fmaf(k.w[o], v.x, acc[o].x);
         acc[o].y = fmaf(k.w[o], v.y, acc[o].y);
         acc[o].z = fmaf(k.w[o], v.z, acc[o].z);
         acc[o].w = fmaf(k.w[o], v.w, acc[o].w);
+    }
+}
+// All inputs -R .. R + N - 1 of N outputs.  The first and last N - 1 of them are further
+// than R from some outputs, which then take nothing (a zero weight times an infinity would
+// be a NaN).
+template <int N, typename F> __device__ __forceinline__ void blur_taps(float4 (&acc)[N], const float *w, int R, F at) {
+    if (2 * R + 1 >= N) {
+#pragma unroll
+        for (int j = 0; j < N - 1; j++) blur_add<N>(acc, w, R, j - R, at(j - R), 0, j + 1);
+        for (int i = N - 1 - R; i <= R; i++) blur_add<N>(acc, w, R, i, at(i), 0, N);
+#pragma unroll
+        for (int j = 1; j < N; j++) blur_add<N>(acc, w, R, R + j, at(R + j), j, N);
+    } else {
+        for (int i = -R; i < R + N; i++) blur_add<N>(acc, w, R, i, at(i), i - R, i + R + 1);
     }
 }
 __device__ __forceinline__ void blur_part(float dot, float *part, float *red) {
@@ -498,12 +513,10 @@ __global__ __launch_bounds__(64 * kBlurWaves) void k_diff_blur_y(Dims d, BlurJob
     float4 acc[kBlurY];
 #pragma unroll
     for (int o = 0; o < kBlurY; o++) acc[o] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int i = -R; i < R + kBlurY; i++) {
+    blur_taps<kBlurY>(acc, w, R, [&](int i) {
         const int y = y0 + i;
-        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (live && y >= 0 && y < (int)d.h) v = in[(size_t)y * d.w + x];
-        blur_add<kBlurY>(acc, w, R, i, v);
-    }
+        return live && y >= 0 && y < (int)d.h ? in[(size_t)y * d.w + x] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    });
     float dot = 0.0f;
 #pragma unroll
     for (int o = 0; o < kBlurY; o++) {
@@ -545,10 +558,10 @@ __global__ __launch_bounds__(64 * kBlurWaves) void k_diff_blur_x(Dims d, BlurJob
     for (int o = 0; o < kBlurX; o++) acc[o] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     float dot = 0.0f;
     if (y < (int)d.h) {
-        for (int i = -R; i < R + kBlurX; i++) {
+        blur_taps<kBlurX>(acc, w, R, [&](int i) {
             const int c = kBlurX * lane + i + R;
-            blur_add<kBlurX>(acc, w, R, i, row[c + c / kBlurX]);
-        }
+            return row[c + c / kBlurX];
+        });
 #pragma unroll
         for (int o = 0; o < kBlurX; o++) {
             const int x = x0 + kBlurX * lane + o;

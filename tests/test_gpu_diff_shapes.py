@@ -71,9 +71,9 @@ def test_long_area_rows_match_short_ones(ctx, w):
 
 
 # ---- non-finite values stay where they are -----------------------------------------
-def _rect(x0, x1, h):
+def _rect(x0, x1, y1, y0=0):
     from resvg_amd import abi
-    pts = [(x0, 0), (x1, 0), (x1, h), (x0, h)]
+    pts = [(x0, y0), (x1, y0), (x1, y1), (x0, y1)]
     return [abi.VERB_MOVE, abi.VERB_LINE, abi.VERB_LINE, abi.VERB_LINE, abi.VERB_CLOSE], np.asarray(pts, np.float32)
 
 
@@ -124,3 +124,39 @@ def test_paint_at_uncovered_pixels(ctx, param, value, wide):
     p[diff.PATH_PARAMS + param] = value
     assert np.isfinite(want).all() and want.any()
     assert np.array_equal(_grad(r, p, go)[:diff.PATH_PARAMS], want)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("sigma,radius", [(0.05, 1), (0.6, 2), (1.0, 3), (2.5, 8)])
+def test_blur_reaches_its_radius_only(ctx, sigma, radius, value):
+    # a blur thread makes several outputs from each input it reads; those further than the
+    # radius from a non-finite pixel keep their bits, in the picture and in the gradients
+    import torch
+    n, bad = 45, 21
+    lo, hi = bad - radius, bad + radius + 1
+    rects = [_rect(bad, bad + 1, bad + 1, bad), _rect(0, lo, n), _rect(hi, n, n), _rect(0, n, lo), _rect(0, n, n, hi)]
+    r = diff.Renderer(ctx, n, n, rects, np.float32([(-90.0, -80.0, 120.0, 90.0)] * 5))
+    P = diff.PATH_PARAMS
+    p = np.zeros(diff.n_params(5), np.float32)
+    for i in range(5):
+        p[i * P:i * P + 20] = np.random.default_rng(i).uniform(0.3, 0.6, 20)
+        p[i * P + 20:i * P + 24] = (0.1, 0.3, 0.6, 0.9)
+    p[5 * P] = sigma
+    p[5 * P + 1:] = np.float32([[0.8, 0, 0, 0, 0.1], [0, 0.8, 0, 0, 0.1], [0, 0, 0.8, 0, 0.1], [0, 0, 0, 0.8, 0.1]]).ravel()
+
+    def run(p, go):
+        params = torch.as_tensor(p, device="cuda")
+        img = r.forward(params).cpu().numpy()
+        return img, r.backward(params, torch.as_tensor(go, device="cuda")).cpu().numpy()
+
+    go = np.random.default_rng(9).normal(0.0, 1.0, (n, n, 4)).astype(np.float32)
+    go[lo:hi, lo:hi] = 0.0
+    img, grad = run(p, go)
+    assert np.isfinite(img).all() and np.isfinite(grad).all() and grad[P:2 * P].any()
+    q = p.copy()
+    q[0] = value  # the tint of the path that covers the pixel alone
+    far = np.ones((n, n), bool)
+    far[lo:hi, lo:hi] = False
+    assert np.array_equal(run(q, go)[0][far], img[far])
+    go[bad, bad] = value
+    assert np.array_equal(run(p, go)[1][P:5 * P], grad[P:5 * P])

@@ -169,7 +169,7 @@ template <class T> __device__ __forceinline__ T scalar_rec(const T *p) {
 // 1 / d for div_by, 0 where d is too small or large for it (or not a width at all)
 __device__ __forceinline__ float div_ready(float d) { return d > 0x1p-60f && d < 0x1p60f ? 1.0f / d : 0.0f; }
 // n / d by the rounded reciprocal r and one exact residual (Markstein): the quotient that
-// the division rounds to, in 3 operations instead of 10
+// the division rounds to, in 3 operations instead of 10; q must not overflow
 __device__ __forceinline__ float div_by(float n, float d, float r) {
     const float q = n * r;
     return fmaf(fmaf(-q, d, n), r, q);
@@ -796,7 +796,8 @@ __global__ __launch_bounds__(kPathThreads, kArea ? 4 : 5) void k_diff_paths_bwd(
                     float gu = gcol[0] * (iv.c1[0] - iv.c0[0]);
 #pragma unroll
                     for (int ch = 1; ch < 4; ch++) gu = fmaf(gcol[ch], iv.c1[ch] - iv.c0[ch], gu);
-                    const float gs = in ? div_by(gu, iv.span, iv.rs) : 0.0f;
+                    const float q = gu * iv.rs;  // div_by, but an overflow stays an infinity
+                    const float gs = !in ? 0.0f : (fabsf(q) < INFINITY ? fmaf(fmaf(-q, iv.span, gu), iv.rs, q) : q);
                     // one stop interval: 14 sums instead of 24
                     float gp[16];
                     const float w1 = st.u, w0 = 1.0f - w1;

@@ -126,6 +126,22 @@ def test_paint_at_uncovered_pixels(ctx, param, value, wide):
     assert np.array_equal(_grad(r, p, go)[:diff.PATH_PARAMS], want)
 
 
+def test_overflowing_slope_is_infinite(ctx):
+    # finite values whose product overflows along the gradient: the offsets of the stops on
+    # either side take an infinity of its sign, not a NaN
+    r, p = _columns(ctx, 16, 4, [(0, 8)], True)
+    p[:4] = 1.0
+    p[4:20] = np.float32([[0, 0, 0, 1], [0, 0, 0, 1], [100, 0, 0, 1], [0, 0, 0, 1]]).ravel()
+    p[20:24] = (0.1, 0.39, 0.6, 0.9)
+    go = np.zeros((4, 16, 4), np.float32)
+    go[1, 3, 0] = 1e37  # at u = 0.08 of the second interval: times 100 past the largest float
+    g = _grad(r, p, go)
+    assert g[21] == g[22] == -np.inf
+    go[1, 3, 0] = -1e37
+    g = _grad(r, p, go)
+    assert g[21] == g[22] == np.inf
+
+
 @pytest.mark.parametrize("value", [np.inf, np.nan])
 @pytest.mark.parametrize("sigma,radius", [(0.05, 1), (0.6, 2), (1.0, 3), (2.5, 8)])
 def test_blur_reaches_its_radius_only(ctx, sigma, radius, value):

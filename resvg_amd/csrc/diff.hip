@@ -191,9 +191,9 @@ __device__ __forceinline__ Along along_path(const PathHead &h, float px, float p
     t = fminf(fmaxf(t, 0.0f), 1.0f);
     e.t = t;
     const uint64_t before = __ballot(t <= h.o0), after = ~before & __ballot(t >= h.o3);
-    e.past1 = ~before & (after | __ballot(t >= h.o1));
-    e.past2 = e.past1 & (after | __ballot(t >= h.o2));
-    e.inside = ~(before | __ballot(t >= h.o3));
+    e.past1 = ~before & (after | __ballot(!(t < h.o1)));  // not below: also where an offset is a NaN
+    e.past2 = e.past1 & (after | __ballot(!(t < h.o2)));
+    e.inside = __ballot(t > h.o0) & __ballot(t < h.o3);
     return e;
 }
 // Whether the covered pixels of the wave (touched, not none) share a stop interval, k0, and

@@ -142,6 +142,23 @@ def test_overflowing_slope_is_infinite(ctx):
     assert g[21] == g[22] == np.inf
 
 
+@pytest.mark.parametrize("k", [0, 1, 2, 3])
+def test_offsets_that_are_no_numbers(ctx, k):
+    # a pixel is in the interval whose upper offset it is below; an interval with a NaN end
+    # has no width (the lower stop's colour), and no pixel lies between stops of which the
+    # first or last is one
+    r, p = _columns(ctx, 32, 4, [(0, 32)], False)
+    p[20 + k] = np.nan
+    go = np.random.default_rng(3).normal(0.0, 1.0, (4, 32, 4)).astype(np.float32)
+    import torch
+    out = r.forward(torch.as_tensor(p, device="cuda")).cpu().numpy()
+    with np.errstate(invalid="ignore"):
+        ref = D.forward(r.coverage.cpu().numpy(), r.ends.cpu().numpy()[0], p, 32, 4)
+    assert np.abs(out - ref).max() < 2e-5  # as in the tests above
+    g = _grad(r, p, go)[:diff.PATH_PARAMS]
+    assert np.isfinite(g).all() and (k in (1, 2) or not g[20:24].any())
+
+
 @pytest.mark.parametrize("value", [np.inf, np.nan])
 @pytest.mark.parametrize("sigma,radius", [(0.05, 1), (0.6, 2), (1.0, 3), (2.5, 8)])
 def test_blur_reaches_its_radius_only(ctx, sigma, radius, value):

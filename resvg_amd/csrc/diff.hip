@@ -877,15 +877,8 @@ __device__ __forceinline__ void bern(float t, float b[4]) {
     b[3] = t * t * t;
 }
 
-__global__ void k_diff_flatten(Dims d, const float *__restrict__ geom, float2 *vert) {
-    geom = scene_at(geom, geom_bytes(d));
-    vert = scene_at(vert, d.ws);
-    const uint32_t n = d.n, k = d.k;
-    const uint32_t nv = k * kFlat + 1;
-    const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= n * nv) return;
-    const uint32_t i = gid / nv, j = gid % nv;
-    const float *g = geom + (size_t)i * (6 + 2 * (3 * k + 1));
+// vertex j of a path of k cubics
+__device__ __forceinline__ float2 flat_vertex(const float *g, uint32_t k, uint32_t j) {
     const uint32_t c = j / kFlat < k ? j / kFlat : k - 1;  // the last vertex is t = 1 of the last cubic
     const float t = (float)(j - c * kFlat) / (float)kFlat;
     float b[4];
@@ -895,7 +888,37 @@ __global__ void k_diff_flatten(Dims d, const float *__restrict__ geom, float2 *v
         x += b[m] * g[6 + 2 * (3 * c + m)];
         y += b[m] * g[6 + 2 * (3 * c + m) + 1];
     }
-    vert[gid] = make_float2(g[0] * x + g[2] * y + g[4], g[1] * x + g[3] * y + g[5]);
+    return make_float2(g[0] * x + g[2] * y + g[4], g[1] * x + g[3] * y + g[5]);
+}
+
+// A thread per vertex and, of the kFlat edges of each cubic and the closing one, the least and
+// the largest y of their ends (everything where one of them is a NaN):
+// bounds[i * (k + 1) + j / kFlat].
+__global__ __launch_bounds__(256) void k_diff_flatten(Dims d, const float *__restrict__ geom, float2 *vert,
+                                                      float2 *bounds) {
+    static_assert(kFlat == 16, "a group's lanes are a row of 16");
+    geom = scene_at(geom, geom_bytes(d));
+    vert = scene_at(vert, d.ws);
+    bounds = scene_at(bounds, d.ws);
+    const uint32_t k = d.k, nv = k * kFlat + 1, lanes = (k + 1) * kFlat;
+    const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = gid / lanes, j = gid % lanes;
+    float lo = INFINITY, hi = -INFINITY;
+    if (i < d.n && j < nv) {
+        const float *g = geom + (size_t)i * (6 + 2 * (3 * k + 1));
+        const float2 v = flat_vertex(g, k, j);
+        vert[(size_t)i * nv + j] = v;
+        // the group's last edge ends at the next group's first vertex, or closes the path
+        const float e = j % kFlat == kFlat - 1 || j + 1 == nv ? flat_vertex(g, k, j + 1 == nv ? 0 : j + 1).y : v.y;
+        const bool nan = v.y != v.y || e != e;
+        lo = nan ? -INFINITY : fminf(v.y, e);
+        hi = nan ? INFINITY : fmaxf(v.y, e);
+    }
+    for (int m = 1; m < kFlat; m <<= 1) {
+        lo = fminf(lo, __shfl_xor(lo, m, kFlat));
+        hi = fmaxf(hi, __shfl_xor(hi, m, kFlat));
+    }
+    if (i < d.n && j % kFlat == 0) bounds[(size_t)i * (k + 1) + j / kFlat] = make_float2(lo, hi);
 }
 
 __global__ void k_diff_zero(float *p, size_t n, size_t stride) {
@@ -993,32 +1016,97 @@ __device__ __forceinline__ bool edge_down(const float2 *vert, uint32_t nv, uint3
 }
 
 // The winding areas of a band of `rows` pixel rows of one path, in LDS from the edges to the
-// prefix sums: a thread per (edge, row) adds the row's differences, then a wave per row sums
-// along it in exact integer arithmetic and writes the floats.  The planes are written once
-// (they were cleared, added to with global atomics, read and written again: 16 scenes of
-// 512^2 with 128 paths 1.92 ms, 2.15 GB of planes); the integers, and so the areas, are the
-// same.  For rows of at most kAreaCells cells.
+// prefix sums: of the cubics whose bounds meet the band the edges that do are gathered,
+// kAreaEdges at a time, a thread per gathered (edge, row) adds the row's differences, then a
+// wave per row sums along it in exact integer arithmetic and writes the floats.  The planes
+// are written once (they were cleared, added to with global atomics, read and written
+// again); the integers, and so the areas, are the same.  For rows of at most kAreaCells cells.
+// Bound by the planes' stores with few cubics (16 scenes of 512^2 with 128 paths of 8 cubics:
+// 2.15 GB, 1.92 -> 0.65 ms), by the gathers with many: looking at every edge for every row
+// instead, a forward of 16 wobbly circles of 4096 cubics at 64 x 4096 took 5.9 ms, where the
+// form below, which visits an edge's own rows, took 0.20; now 0.15 (32 of 512 cubics at
+// 512^2: 0.38, 0.12 and 0.09).  Cubics through all of the canvas, 32 of 512 at 512^2: 0.43,
+// 0.75 and 0.17.
 constexpr int kAreaCells = 8192;  // 32 KB of LDS
-__global__ __launch_bounds__(256) void k_diff_area(Dims d, const float2 *__restrict__ vert, float *area, uint32_t rows,
+constexpr int kAreaEdges = 512;
+constexpr int kAreaGroups = 512;  // cubics looked at together
+
+// Appends `value` of the lanes with `keep` to a list in LDS of which `count` entries are used.
+__device__ __forceinline__ void gather(bool keep, uint32_t value, uint16_t *list, uint32_t &count, int lane) {
+    const uint64_t m = __ballot(keep);
+    uint32_t at = 0;
+    if (lane == 0 && m != 0) at = atomicAdd(&count, (uint32_t)__popcll(m));
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    if (keep) list[at + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)value;
+}
+// whether rows y0 .. y1 - 1 meet a stretch from lo down to hi, as k_diff_area's rows take it
+// (a NaN lo is above them all, a NaN hi ends before them)
+__device__ __forceinline__ bool meets_rows(float lo, float hi, uint32_t y0, uint32_t y1) {
+    return !(floorf(lo) >= (float)y1) && ceilf(hi) > (float)y0;
+}
+__global__ __launch_bounds__(256) void k_diff_area(Dims d, const float2 *__restrict__ vert,
+                                                   const float2 *__restrict__ bounds, float *area, uint32_t rows,
                                                    uint32_t bands) {
     __shared__ int cells[kAreaCells];
+    __shared__ uint16_t groups[kAreaGroups], list[kAreaEdges];  // cubics; 16 * a cubic's place in its batch + edge
+    __shared__ uint32_t ngroups, nedges;
     vert = scene_at(vert, d.ws);
+    bounds = scene_at(bounds, d.ws);
     area = scene_at(area, d.ws);
     const uint32_t i = blockIdx.x / bands, y0 = blockIdx.x % bands * rows, y1 = min(y0 + rows, d.h);
-    const uint32_t stride = d.w + 2, nv = d.k * kFlat + 1;
+    const uint32_t stride = d.w + 2, nv = d.k * kFlat + 1, batch = kAreaEdges / kFlat;
+    const int lane = (int)(threadIdx.x % 64);
     for (uint32_t c = threadIdx.x; c < rows * stride; c += 256) cells[c] = 0;
-    __syncthreads();
-    for (uint32_t q = threadIdx.x; q < nv * rows; q += 256) {
-        const uint32_t j = q / rows;
-        const int y = (int)(y0 + q % rows);
-        float2 a, b;
-        float dir;
-        if (!edge_down(vert, nv, i, j, a, b, dir)) continue;
-        if (y >= (int)y1 || y < (int)floorf(a.y) || y >= (int)ceilf(b.y)) continue;  // a row the edge spans
-        accum_row(cells + ((uint32_t)y - y0) * stride, d, a, b, (b.x - a.x) / (b.y - a.y), dir, y);
+    for (uint32_t c0 = 0; c0 <= d.k; c0 += kAreaGroups) {
+        __syncthreads();
+        if (threadIdx.x == 0) ngroups = nedges = 0;
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < kAreaGroups; k += 256) {
+            bool meets = false;
+            if (c0 + k <= d.k) {
+                const float2 b = bounds[(size_t)i * (d.k + 1) + c0 + k];
+                meets = meets_rows(b.x, b.y, y0, y1);
+            }
+            gather(meets, c0 + k, groups, ngroups, lane);
+        }
+        __syncthreads();
+        for (uint32_t g0 = 0; g0 < ngroups; g0 += batch) {
+            for (uint32_t k = threadIdx.x; k < kAreaEdges; k += 256) {
+                bool meets = false;
+                if (g0 + k / kFlat < ngroups) {
+                    const uint32_t j = groups[g0 + k / kFlat] * kFlat + k % kFlat;
+                    float2 a, b;
+                    float dir;
+                    meets = j < nv && edge_down(vert, nv, i, j, a, b, dir) && meets_rows(a.y, b.y, y0, y1);
+                }
+                gather(meets, k, list, nedges, lane);
+            }
+            __syncthreads();
+            // a thread per edge where there are enough of them, else per edge and row
+            const uint32_t split = nedges < 256 ? rows : 1;
+            for (uint32_t q = threadIdx.x; q < nedges * split; q += 256) {
+                const uint32_t k = list[q / split], j = groups[g0 + k / kFlat] * kFlat + k % kFlat;
+                float2 a, b;
+                float dir;
+                if (!edge_down(vert, nv, i, j, a, b, dir)) continue;
+                // the rows that the edge spans
+                int ya = max((int)y0, (int)floorf(a.y)), yb = min((int)y1, (int)ceilf(b.y));
+                if (split > 1) {
+                    const int y = (int)(y0 + q % split);
+                    ya = max(ya, y);
+                    yb = min(yb, y + 1);
+                }
+                for (int y = ya; y < yb; y++)
+                    accum_row(cells + ((uint32_t)y - y0) * stride, d, a, b, (b.x - a.x) / (b.y - a.y), dir, y);
+            }
+            __syncthreads();
+            if (g0 + batch < ngroups) {  // uniform
+                if (threadIdx.x == 0) nedges = 0;
+                __syncthreads();
+            }
+        }
     }
     __syncthreads();
-    const int lane = (int)(threadIdx.x % 64);
     const float inv = 1.0f / d.qscale;
     for (uint32_t r = threadIdx.x / 64; r < y1 - y0; r += 4) {
         const int *c = cells + r * stride;
@@ -1261,7 +1349,7 @@ __global__ __launch_bounds__(1024) void k_diff_reduce(ReducePart paths, ReducePa
 // Workspace layout (bytes, 256-aligned): canvas S | T | B | gB | gS | gS2 | weights |
 // path records | checkpoints | partial rows (paths) | partial rows (matrix) | σ partials (2 rows).
 struct Layout {
-    size_t S, T, B, gB, gS, gS2, wts, rec, ck, part_p, part_m, part_s, area, gW, vert, egrad, total;
+    size_t S, T, B, gB, gS, gS2, wts, rec, ck, part_p, part_m, part_s, area, gW, vert, egrad, bounds, total;
 };
 uint32_t squares(uint32_t side, int square) { return (side + square - 1) / square; }
 Layout layout(uint32_t w, uint32_t h, uint32_t n, uint32_t k) {
@@ -1286,7 +1374,8 @@ Layout layout(uint32_t w, uint32_t h, uint32_t n, uint32_t k) {
     L.gW = L.area + (k ? al((size_t)n * h * (w + 2) * sizeof(float)) : 0);
     L.vert = L.gW + (k ? al((size_t)n * w * h * sizeof(float)) : 0);
     L.egrad = L.vert + (k ? al((size_t)n * nv * sizeof(float2)) : 0);
-    L.total = L.egrad + (k ? al((size_t)n * nv * sizeof(float4)) : 0);
+    L.bounds = L.egrad + (k ? al((size_t)n * nv * sizeof(float4)) : 0);
+    L.total = L.bounds + (k ? al((size_t)n * (k + 1) * sizeof(float2)) : 0);
     return L;
 }
 
@@ -1346,17 +1435,19 @@ rvk_status rvk_diff_forward_batch(rvk_context *ctx, const rvk_diff_scene *scene,
     if (k) {
         // analytic coverage: flatten, accumulate winding area, prefix along rows
         float *area = (float *)(ws + L.area);
-        float2 *vert = (float2 *)(ws + L.vert);
+        float2 *vert = (float2 *)(ws + L.vert), *bounds = (float2 *)(ws + L.bounds);
         const size_t nv = (size_t)k * kFlat + 1, cells = (size_t)n * h * (w + 2);
         const unsigned ge = (unsigned)((n * nv + 255) / 256);
         const unsigned gz = (unsigned)((cells + 255) / 256 < 65535 ? (cells + 255) / 256 : 65535);
         rvk::timed_launch(ctx, "diff_coverage", (double)cells * 8.0 * batch, [&] {
-            hipLaunchKernelGGL(k_diff_flatten, dim3(ge, batch), dim3(256), 0, ctx->stream, d, dev_geom, vert);
+            const size_t lanes = (size_t)n * (k + 1) * kFlat;
+            hipLaunchKernelGGL(k_diff_flatten, dim3((unsigned)((lanes + 255) / 256), batch), dim3(256), 0, ctx->stream,
+                               d, dev_geom, vert, bounds);
             const uint32_t rows = std::min<uint32_t>({(uint32_t)kAreaCells / (w + 2), 16u, h});
             if (rows > 0) {
                 const uint32_t bands = (h + rows - 1) / rows;
                 hipLaunchKernelGGL(k_diff_area, dim3(n * bands, batch), dim3(256), 0, ctx->stream, d,
-                                   (const float2 *)vert, area, rows, bands);
+                                   (const float2 *)vert, (const float2 *)bounds, area, rows, bands);
             } else {
                 hipLaunchKernelGGL(k_diff_zero, dim3(gz, batch), dim3(256), 0, ctx->stream, area, cells, L.total);
                 hipLaunchKernelGGL(k_diff_accum, dim3(ge, batch), dim3(256), 0, ctx->stream, d, (const float2 *)vert,

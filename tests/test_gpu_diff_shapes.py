@@ -70,6 +70,33 @@ def test_long_area_rows_match_short_ones(ctx, w):
     assert np.array_equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("k", [1, 31, 32, 33, 511, 512, 600])
+@pytest.mark.parametrize("kind", ["outline", "wild", "nan"])
+def test_areas_of_many_cubics(ctx, k, kind):
+    # bands gather the cubics, then the edges, that meet them (512 at a time): the areas have
+    # the bits of the form for long rows, which visits every edge's own rows
+    import torch
+    from resvg_amd import abi
+    rng = np.random.default_rng(k)
+    t = np.linspace(0.0, 2.0 * np.pi, 3 * k + 1)
+    paths = []
+    for i in range(3):
+        r = 0.4 + 0.05 * np.sin(7 * t + i) + (rng.uniform(-0.4, 0.4, t.size) if kind != "outline" else 0.0)
+        pts = np.stack([150.0 + 180.0 * r * np.cos(t), 18.0 + 60.0 * r * np.sin(t)], 1).astype(np.float32)
+        if kind == "nan" and i == 1:
+            pts[3 * k // 2, 1] = np.nan
+        paths.append(([abi.VERB_MOVE] + [abi.VERB_CUBIC] * k + [abi.VERB_CLOSE], pts))
+    p = np.zeros(diff.n_params(3), np.float32)
+    p[:72] = 0.5
+    p[72] = 0.05  # no colour matrix: the picture is the paths' canvas
+    outs = []
+    for width in (300, 8200):
+        r = diff.Renderer(ctx, width, 37, paths, np.zeros((3, 4), np.float32), cubics=k)
+        outs.append(r.forward(torch.as_tensor(p, device="cuda"), r.geom0).cpu().numpy()[:, :299])
+    assert outs[0][..., 3].max() > 0.1
+    assert np.array_equal(outs[0], outs[1], equal_nan=True)
+
+
 # ---- non-finite values stay where they are -----------------------------------------
 def _rect(x0, x1, y1, y0=0):
     from resvg_amd import abi

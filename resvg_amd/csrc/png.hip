@@ -5,8 +5,8 @@
 // alpha 255 unchanged, otherwise each colour channel c / (a / 255) + 0.5 in f64 and
 // cast to u8 (saturating, NaN to 0) -- the reference's test harness restates the same
 // rule at crates/resvg/tests/integration/main.rs:204-211.  On the device a channel is
-// floor(c * r(a) + 0.5) in f32 with an r(a) near 255 / a that gives the f64 rule's value
-// for all 256 channel values (checked on the host, where the r's are chosen); the six
+// floor(c * r(a) + 0.5) in f32, fused, with an r(a) near 255 / a that gives the f64 rule's value
+// for all 256 channel values (checked on the host by the same function, png_demul.h); the six
 // alphas whose ties no single r gets right have their 256 values in a table.  Each row is
 // then filtered with one of the five PNG filter types (ISO/IEC 15948 section 9: None, Sub,
 // Up, Average, Paeth; 4 bytes per pixel, bytes left of the row and the row above the
@@ -21,58 +21,23 @@
 // Paeth on 16-bit pairs).  Rows too long for LDS are read and demultiplied again instead.
 // Bound by the VALU (Paeth is half of it).  With byte-wise filters, a 64 KB table read
 // three times a pixel, twice a pass, and a launch to build it: 92 us at 3001 x 2003.
+#include "png_demul.h"
 #include "rvk_internal.h"
-#include <cmath>
+
+using namespace rvk_png;
 
 namespace {
 
 constexpr int kPngBlock = 256;
 constexpr uint32_t kPngLdsWidth = 4096;  // widest row whose pixels stay in LDS (two rows: 32 KB)
-constexpr int kSpecial = 6;
-
-// per alpha the factor r, or -1 - k where table row k holds the values
-struct Demul {
-    float r[256];
-    uint8_t special[kSpecial][256];
-};
-
-// The f64 rule for channel c at alpha a.
-uint32_t demul_rule(uint32_t c, uint32_t a) {
-    if (a == 255u) return c;
-    const double d = (double)c / ((double)a / 255.0) + 0.5;
-    return d != d ? 0u : d >= 255.0 ? 255u : d <= 0.0 ? 0u : (uint32_t)d;
-}
-
-bool make_demul(Demul &t) {
-    int nspecial = 0;
-    for (uint32_t a = 0; a < 256; a++) {
-        const float r0 = a ? 255.0f / (float)a : 1e30f;
-        const float tries[3] = {r0, std::nextafter(r0, 0.0f), std::nextafter(r0, 1e38f)};
-        bool found = false;
-        for (int k = 0; k < 3 && !found; k++) {
-            found = true;
-            for (uint32_t c = 0; c < 256 && found; c++) {
-                const float p = (float)c * tries[k];
-                const float v = p + 0.5f;
-                found = (v >= 255.0f ? 255u : (uint32_t)v) == demul_rule(c, a);
-            }
-            t.r[a] = tries[k];
-        }
-        if (found) continue;
-        if (nspecial == kSpecial) return false;
-        for (uint32_t c = 0; c < 256; c++) t.special[nspecial][c] = (uint8_t)demul_rule(c, a);
-        t.r[a] = -1.0f - (float)nspecial++;
-    }
-    return true;
-}
 
 // the straight pixel of p
 __device__ __forceinline__ uint32_t straight(const float *r, const uint8_t (*special)[256], uint32_t p) {
     const float f = r[p >> 24];
-    auto ch = [&](uint32_t c) { return min((uint32_t)((float)c * f + 0.5f), 255u); };
+    auto ch = [&](uint32_t c) { return straight_channel(c, f); };
     uint32_t v = ch(p & 0xffu) | (ch((p >> 8) & 0xffu) << 8) | (ch((p >> 16) & 0xffu) << 16);
-    if (f < 0.0f) {
-        const uint8_t *row = special[(int)(-1.0f - f)];
+    if (by_table(f)) {
+        const uint8_t *row = special[table_row(f)];
         v = (uint32_t)row[p & 0xffu] | ((uint32_t)row[(p >> 8) & 0xffu] << 8) | ((uint32_t)row[(p >> 16) & 0xffu] << 16);
     }
     return v | (p & 0xff000000u);

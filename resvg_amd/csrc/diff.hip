@@ -1312,7 +1312,8 @@ __global__ __launch_bounds__(64) void k_diff_geom_chain(Dims d, const float *__r
 }
 
 // Sums partial rows into the gradients, in a fixed order: a block of 16 columns x 64 row
-// lanes, each lane summing every 64th row of a column, then the lanes in order.  Blocks
+// lanes, each lane summing every 64th row of a column in eight sums, then those and the
+// lanes in pairs, which keeps the rounding of many rows down.  Blocks
 // below `blocks` take the paths' partial rows; the last two σ (both passes' block sums, one
 // column) and the matrix (20 columns).
 struct ReducePart {
@@ -1332,18 +1333,20 @@ __global__ __launch_bounds__(1024) void k_diff_reduce(ReducePart paths, ReducePa
     const float *part = scene_at(r.part, part_stride);
     const uint32_t tx = threadIdx.x % 16, ty = threadIdx.x / 16;
     c += tx;
-    float s = 0.0f;
+    float s[8] = {};
     if (c < r.cols) {
-#pragma unroll 8
-        for (uint32_t row = ty; row < r.rows; row += 64) s += part[(size_t)row * r.cols + c];
+        for (uint32_t row = ty; row < r.rows; row += 512) {
+#pragma unroll
+            for (uint32_t k = 0; k < 8; k++)
+                if (row + 64 * k < r.rows) s[k] += part[(size_t)(row + 64 * k) * r.cols + c];
+        }
     }
-    acc[ty][tx] = s;
-    __syncthreads();
-    if (ty == 0 && c < r.cols) {
-        float t = 0.0f;
-        for (int k = 0; k < 64; k++) t += acc[k][tx];
-        scene_at(r.out, out_stride)[c] = t;
+    acc[ty][tx] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    for (uint32_t half = 32; half > 0; half >>= 1) {
+        __syncthreads();
+        if (ty < half) acc[ty][tx] += acc[ty + half][tx];
     }
+    if (ty == 0 && c < r.cols) scene_at(r.out, out_stride)[c] = acc[0][tx];
 }
 
 // Workspace layout (bytes, 256-aligned): canvas S | T | B | gB | gS | gS2 | weights |

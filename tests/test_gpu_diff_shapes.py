@@ -220,3 +220,25 @@ def test_blur_reaches_its_radius_only(ctx, sigma, radius, value):
     assert np.array_equal(run(q, go)[0][far], img[far])
     go[bad, bad] = value
     assert np.array_equal(run(p, go)[1][P:5 * P], grad[P:5 * P])
+
+
+@pytest.mark.parametrize("w,h", [(1024, 1024), (2048, 1536), (1000, 700)])
+def test_rounding_of_the_sum_over_pixels(ctx, w, h):
+    # every pixel of a full canvas adds the same value to the tint's gradient, so all rounding
+    # is that of the sum.  A pixel's value passes the wave's tree (6 additions), the block's
+    # 4 waves, one of 8 sums of up to `chain` partial rows, 3 and 6 levels of pairs; each
+    # rounds by at most half a unit, 2^-24 of the sum
+    r = diff.Renderer(ctx, w, h, [_rect(0, w, h)], np.zeros((1, 4), np.float32))
+    P = diff.PATH_PARAMS
+    p = np.zeros(diff.n_params(1), np.float32)
+    p[:20] = 1.0
+    p[20:24] = (0.1, 0.3, 0.6, 0.9)
+    p[P] = 0.05  # no colour matrix: dL/d(canvas) is dL/d(picture)
+    tiles = -(-w // 64) * -(-h // 4)
+    chain = -(-tiles // 512)
+    for seed in range(4):
+        g = np.random.default_rng(seed).uniform(1.0, 2.0, 3).astype(np.float32)
+        go = np.zeros((h, w, 4), np.float32)
+        go[..., :3] = g
+        rel = np.abs(_grad(r, p, go)[:3].astype(np.float64) / (g.astype(np.float64) * (w * h)) - 1.0)
+        assert rel.max() <= (6 + 3 + chain + 9) * 2.0 ** -24

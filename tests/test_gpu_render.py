@@ -8,6 +8,7 @@ import pytest
 
 from oracle import bindings as orc
 from resvg_amd import abi
+from resvg_amd.filters import FilterGraph
 from resvg_amd.scene import PaintSpec, Scene, ellipse_path, rect_path
 from resvg_amd.workloads import blur_offset_composite_doc, document_batch, full_filter_doc
 
@@ -444,6 +445,42 @@ def test_many_small_flushes(ctx, monkeypatch):
     got = _gpu(ctx, sc, ts, w, h)
     assert ctx.stats().flushes >= 10
     _assert_same(got, _oracle(sc, ts, w, h), "many flushes")
+
+
+@pytest.mark.parametrize("order", ["LLSSLLSSLSLSSL", "SLLSSLLSSLLSLSL", "LSSSLSLLSLL", "SSSLSLSLLL"])
+def test_flushes_of_both_sizes_share_the_blocks(ctx, monkeypatch, order):
+    # flushes of 2048 coverage bands or more prepare on the side stream, smaller ones on the
+    # context stream, and both take the two blocks in turn: each order of two flushes on a
+    # block, the first use and the growth of a block among them.  One flush per filtered
+    # group; a large one has 20 paths of 128 bands
+    monkeypatch.setenv("RVK_VALIDATE", "1")
+    w, h = 96, 1024
+    rng = np.random.default_rng(len(order))
+
+    def doc(order):
+        sc = Scene(w, h)
+        for kind in order:
+            g = FilterGraph((0.0, 0.0, float(w), float(h)))
+            g.offset(1.0, 2.0)
+            grp = sc.group(sc.root, filters=[g], opacity=0.9)
+            for _ in range(20 if kind == "L" else 1):
+                bottom = h if kind == "L" else 48
+                pts = np.concatenate([rng.uniform(0, w, (7, 1)), rng.uniform(0, bottom, (7, 1))], 1).astype(np.float32)
+                pts[0, 1], pts[3, 1] = 0.0, bottom
+                paint = PaintSpec.solid(tuple(int(v) for v in rng.integers(0, 256, 3)), 0.7)
+                sc.path(grp, [abi.VERB_MOVE, abi.VERB_CUBIC, abi.VERB_CUBIC, abi.VERB_CLOSE], pts, fill=paint)
+        return sc
+
+    ts = abi.Transform.identity()
+    _gpu(ctx, doc("L"), ts, w, h)
+    assert ctx.stats().flushes == 1 and ctx.stats().band_entries >= 2048
+    _gpu(ctx, doc("S"), ts, w, h)
+    assert ctx.stats().flushes == 1 and ctx.stats().band_entries < 2048
+    for _ in range(3):
+        sc = doc(order)
+        got = _gpu(ctx, sc, ts, w, h)
+        assert ctx.stats().flushes == ctx.stats().validated_flushes == len(order)
+        _assert_same(got, _oracle(sc, ts, w, h), order)
 
 
 def test_flush_budget_does_not_change_pixels(ctx, monkeypatch):

@@ -44,6 +44,22 @@ def test_stop_intervals_without_width(ctx):
     assert np.abs(out - D.forward(cov, ends, params.cpu().numpy(), 65, 40)).max() < 2e-5
 
 
+def test_gradient_through_stop_intervals_without_width(ctx):
+    # the offsets of a path with such an interval have no derivative there; every other
+    # parameter, and the other paths' offsets, do
+    import torch
+    w, h, n = 65, 17, 9
+    r, params, cov, ends = _planes(ctx, w, h, n, seed=4, equal_offsets=True)
+    go = np.random.default_rng(4).normal(0.0, 1.0, (h, w, 4)).astype(np.float32)
+    r.forward(params)
+    g = r.backward(params, torch.as_tensor(go, device="cuda")).cpu().numpy().astype(np.float64)
+    assert np.isfinite(g).all()
+    P = diff.PATH_PARAMS
+    idx = [j for j in range(len(g)) if j >= n * P or j % P < 20 or (j // P) % 3 == 2]
+    ref = D.grad_fd(cov, ends, params.cpu().numpy(), w, h, go, idx)
+    assert np.linalg.norm(g[idx] - ref[idx]) / np.linalg.norm(ref[idx]) < 1e-3  # as for the oracle tests
+
+
 @pytest.mark.parametrize("w,h,n", [(63, 5, 3), (66, 9, 9)])
 def test_shapes_gradient(ctx, w, h, n):
     import torch

@@ -260,9 +260,8 @@ struct Renderer {
     // the flush before last, the previous reader of the block, is done (or, for a
     // block just taken from the scratch cache, until the context stream's work so far
     // is), so the coverage of a flush overlaps the compositing of the one before.
-    // A small flush (fewer than kOverlapBands coverage bands) runs on the context stream
-    // alone: the events that hand work to the side stream and back cost more than its
-    // coverage takes.
+    // A small flush (see on_side) runs on the context stream alone: the events that hand
+    // work to the side stream and back cost more than its coverage takes.
     void *blk[2] = {nullptr, nullptr};
     size_t blk_cap[2] = {0, 0};
     hipEvent_t blk_free[2] = {nullptr, nullptr};  // recorded on the context stream after a block's draw
@@ -274,10 +273,22 @@ struct Renderer {
     // false: a flush runs on the context stream alone (on a batch's lanes, which
     // already run documents side by side)
     const bool overlap = !ctx->is_lane;
-    // A record, a wait and their return on two streams take 23 us of host time more than
-    // the launches alone, about what the coverage of 2000 bands takes on the device (0.65
-    // ms for the 30 000 of a 4096^2 flush)
-    static constexpr uint64_t kOverlapBands = 2048;
+    // Whether a flush prepares on the side stream.  A record, a wait and their return on two
+    // streams take 23 us of host time more than the launches alone, about what the coverage
+    // of 2000 bands takes on the device (0.65 ms for the 30 000 of a 4096^2 flush).  With
+    // 2048 bands or more the side stream gives 5% there (101.6 against 106.5 ms a render;
+    // 104.3 with 8192) and costs nothing at 1024^2 (300 paths: 6.3 ms either way).  A
+    // smaller flush gains where the device is behind the host: where its target is large
+    // and flushes are under way.  Documents of 60 clipped or masked groups, on one stream
+    // and on two from 64 bands: 2048^2 15.5 and 13.2 ms (150 groups: 37.9 and 31.4), 1600^2
+    // 13.0 and 11.9, 1448^2 12.2 and 11.7, 1200^2 10.9 and 11.6, 1024^2 10.0 and 11.4; from
+    // 128 bands 2048^2 takes 14.0, and from 1 band 256^2 9.6 against 8.1.
+    static constexpr uint64_t kOverlapBands = 2048, kOverlapSmall = 64, kOverlapPixels = 1u << 21;
+    bool on_side(const DrawList &dl) const {
+        if (!overlap) return false;
+        if (dl.n_windows >= kOverlapBands) return true;
+        return nflush > 0 && dl.n_windows >= kOverlapSmall && (uint64_t)dl.w * dl.h >= kOverlapPixels;
+    }
 
     ~Renderer() { (void)finish_flushes(); }
 
@@ -774,9 +785,9 @@ struct Renderer {
         }
         // the flush's block (see blk), replaced by a larger one from the scratch cache
         // when it is too small (the old one's last reader is on the context stream)
+        const bool aside = on_side(dl);
         const int b = (int)(nflush++ & 1);
         const size_t need = o_arena + dl.arena;
-        const bool aside = overlap && dl.n_windows >= kOverlapBands;
         if (aside) RVK_TRY(flush_events());
         bool fresh = false;
         if (blk_cap[b] < need) {

@@ -447,14 +447,16 @@ def test_many_small_flushes(ctx, monkeypatch):
     _assert_same(got, _oracle(sc, ts, w, h), "many flushes")
 
 
-@pytest.mark.parametrize("order", ["LLSSLLSSLSLSSL", "SLLSSLLSSLLSLSL", "LSSSLSLLSLL", "SSSLSLSLLL"])
-def test_flushes_of_both_sizes_share_the_blocks(ctx, monkeypatch, order):
-    # flushes of 2048 coverage bands or more prepare on the side stream, smaller ones on the
-    # context stream, and both take the two blocks in turn: each order of two flushes on a
-    # block, the first use and the growth of a block among them.  One flush per filtered
-    # group; a large one has 20 paths of 128 bands
+@pytest.mark.parametrize("w,h,order", [(96, 1024, "LLSSLLSSLSLSSL"), (96, 1024, "SLLSSLLSSLLSLSL"),
+                                       (96, 1024, "LSSSLSLLSLL"), (96, 1024, "SSSLSLSLLL"),
+                                       (1024, 2048, "SMMSSMMSSM"), (1024, 2048, "MMSSMSMMSSLM")])
+def test_flushes_of_both_sizes_share_the_blocks(ctx, monkeypatch, w, h, order):
+    # flushes of 2048 coverage bands or more, and of 64 or more on 2^21 pixels after the
+    # first, prepare on the side stream, smaller ones on the context stream, and both take
+    # the two blocks in turn: each order of two flushes on a block, the first use and the
+    # growth of a block among them.  One flush per filtered group: a large one has 20 paths
+    # of at least 128 bands, a middle one 1 of 256, a small one 1 of 6
     monkeypatch.setenv("RVK_VALIDATE", "1")
-    w, h = 96, 1024
     rng = np.random.default_rng(len(order))
 
     def doc(order):
@@ -464,7 +466,7 @@ def test_flushes_of_both_sizes_share_the_blocks(ctx, monkeypatch, order):
             g.offset(1.0, 2.0)
             grp = sc.group(sc.root, filters=[g], opacity=0.9)
             for _ in range(20 if kind == "L" else 1):
-                bottom = h if kind == "L" else 48
+                bottom = h if kind != "S" else 48
                 pts = np.concatenate([rng.uniform(0, w, (7, 1)), rng.uniform(0, bottom, (7, 1))], 1).astype(np.float32)
                 pts[0, 1], pts[3, 1] = 0.0, bottom
                 paint = PaintSpec.solid(tuple(int(v) for v in rng.integers(0, 256, 3)), 0.7)
@@ -475,8 +477,8 @@ def test_flushes_of_both_sizes_share_the_blocks(ctx, monkeypatch, order):
     _gpu(ctx, doc("L"), ts, w, h)
     assert ctx.stats().flushes == 1 and ctx.stats().band_entries >= 2048
     _gpu(ctx, doc("S"), ts, w, h)
-    assert ctx.stats().flushes == 1 and ctx.stats().band_entries < 2048
-    for _ in range(3):
+    assert ctx.stats().flushes == 1 and ctx.stats().band_entries < 64
+    for _ in range(3 if w == 96 else 1):
         sc = doc(order)
         got = _gpu(ctx, sc, ts, w, h)
         assert ctx.stats().flushes == ctx.stats().validated_flushes == len(order)

@@ -23,6 +23,14 @@ struct ConvArgs {
 // the matrix, then columns).  Bound by arithmetic: with a pixel a thread and an IEEE
 // division a channel and tap a 5 x 5 matrix over 1601 x 1131 took 86 us, now 39.
 constexpr int kConvPx = 4;
+// Images below this many pixels have too few threads for that: a thread's taps follow each
+// other, and four pixels of them take longer than one while lanes stand idle.  Four and one
+// pixel a thread, matrix of 9 x 9 and of 1 x 40: 17 x 13 70 and 32, 64 and 22 us; 600 x 600
+// 63 and 47, 63 and 38; 1031 x 777 79 and 75, 72 and 62; 2048^2 210 and 278, 196 and 230.
+// The tiles below hold four pixels a thread as well and stage their halo first: 40 x 1 as a
+// tile and from memory 31 and 19 us at 130 x 127, 29 and 20 at 400 x 300; 5 x 5 22 and 18 at
+// 400 x 300, 23 and 20 at 600 x 600, 28 and 32 at 1031 x 777; 8 x 8 35 and 34 at 600 x 600.
+constexpr size_t kConvFewPixels = (size_t)1 << 20, kConvUntiledPixels = (size_t)1 << 18;
 
 // the pixel of a matrix's four sums; p the source pixel (read with preserve_alpha only)
 __device__ __forceinline__ uint32_t conv_result(const float (&sum)[4], uint32_t p, const ConvArgs &a) {
@@ -42,8 +50,8 @@ __device__ __forceinline__ uint32_t conv_result(const float (&sum)[4], uint32_t 
 // (zero outside the image in edge mode none, where a tap then adds nothing), a thread
 // taking four rows of a column, so a value read serves up to four of its sums.  Each sum
 // still runs over the matrix's rows, then its columns.  5 x 5 over 1601 x 1131: 31 us, 39
-// with the form below, which larger matrices and infinite coefficients (times zero a NaN,
-// where the reference leaves the tap out) take.
+// with the form below, which small images, larger matrices and infinite coefficients (times
+// zero a NaN, where the reference leaves the tap out) take.
 constexpr int kTileW = 64, kTileH = 16;
 inline size_t conv_tile_bytes(uint32_t columns, uint32_t rows) {
     return (size_t)(kTileW + columns - 1) * (kTileH + rows - 1) * sizeof(float4);
@@ -107,16 +115,17 @@ __global__ __launch_bounds__(256) void k_convolve_tile(const uint32_t *__restric
     }
 }
 
-// kBig: the matrix in memory, not among the arguments
-template <bool kBig>
-__global__ __launch_bounds__(256) void k_convolve(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst, uint32_t w, uint32_t h,
-                           ConvArgs a, const float *__restrict__ big_k) {
+// kBig: the matrix in memory, not among the arguments; kPx: adjacent pixels a thread
+template <bool kBig, int kPx>
+__global__ __launch_bounds__(256) void k_convolve(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst,
+                                                  uint32_t w, uint32_t h, ConvArgs a,
+                                                  const float *__restrict__ big_k) {
     const int32_t wmax = (int32_t)w - 1, hmax = (int32_t)h - 1, cols = (int32_t)a.columns;
     const uint2 tile = xcd_tile();
-    const int32_t x0 = (int32_t)(tile.x * 64 + threadIdx.x) * kConvPx;
+    const int32_t x0 = (int32_t)(tile.x * 64 + threadIdx.x) * kPx;
     if (x0 > wmax) return;
     for (uint32_t y = tile.y * 4 + threadIdx.y; y < h; y += gridDim.y * 4) {
-        float sum[kConvPx][4] = {};
+        float sum[kPx][4] = {};
         for (uint32_t oy = 0; oy < a.rows; oy++) {
             int32_t ty = (int32_t)y - (int32_t)a.ty + (int32_t)oy;
             if (a.edge == RVK_EDGE_NONE) {
@@ -128,7 +137,7 @@ __global__ __launch_bounds__(256) void k_convolve(const uint32_t *__restrict__ s
                 ty %= (int32_t)h; if (ty < 0) ty += (int32_t)h;
             }
             const uint32_t *row = src + (size_t)ty * w;
-            for (int32_t t = 0; t < cols + kConvPx - 1; t++) {
+            for (int32_t t = 0; t < cols + kPx - 1; t++) {
                 int32_t tx = x0 - (int32_t)a.tx + t;
                 bool in = true;
                 if (a.edge == RVK_EDGE_NONE) {
@@ -140,7 +149,7 @@ __global__ __launch_bounds__(256) void k_convolve(const uint32_t *__restrict__ s
                 const uint32_t p = row[max(0, min(wmax, tx))];
                 const float c0 = unit(ch(p, 0)), c1 = unit(ch(p, 1)), c2 = unit(ch(p, 2)), c3 = unit(ch(p, 3));
 #pragma unroll
-                for (int j = 0; j < kConvPx; j++) {
+                for (int j = 0; j < kPx; j++) {
                     const int32_t ox = t - j;  // pixel x0 + j meets this source pixel at column ox
                     if (ox < 0 || ox >= cols) continue;
                     const uint32_t e = oy * a.columns + (uint32_t)ox;
@@ -154,7 +163,7 @@ __global__ __launch_bounds__(256) void k_convolve(const uint32_t *__restrict__ s
             }
         }
 #pragma unroll
-        for (int j = 0; j < kConvPx; j++) {
+        for (int j = 0; j < kPx; j++) {
             if (x0 + j > wmax) break;
             const size_t i = (size_t)y * w + (size_t)(x0 + j);
             dst[i] = conv_result(sum[j], a.preserve_alpha ? src[i] : 0u, a);
@@ -330,15 +339,20 @@ rvk_status launch_convolve_to(rvk_context *ctx, const uint8_t *src, uint8_t *dst
         rvk_status ust = upload_async(ctx, bigk, flipped.data(), nk * sizeof(float));
         if (ust != RVK_OK) { scratch_release(ctx, bigk); return ust; }
     }
-    bool tiled = !bigk && conv_tile_bytes(cm.columns, cm.rows) <= kMaxConvTile;
+    bool tiled = !bigk && (size_t)w * h >= kConvUntiledPixels && conv_tile_bytes(cm.columns, cm.rows) <= kMaxConvTile;
     for (size_t i = 0; tiled && i < nk; i++) tiled = std::isfinite(a.k[i]);
     timed_launch(ctx, "convolve_matrix", 8.0 * (double)w * h, [&] {
         if (tiled)
             hipLaunchKernelGGL(k_convolve_tile, dim3((w + kTileW - 1) / kTileW, (h + kTileH - 1) / kTileH), dim3(64, 4),
                                conv_tile_bytes(cm.columns, cm.rows), ctx->stream, (const uint32_t *)src, (uint32_t *)dst,
                                w, h, a);
-        else hipLaunchKernelGGL(bigk ? k_convolve<true> : k_convolve<false>, grid2((w + kConvPx - 1) / kConvPx, h), dim3(64, 4), 0, ctx->stream,
-                           (const uint32_t *)src, (uint32_t *)dst, w, h, a, (const float *)bigk);
+        else if ((size_t)w * h < kConvFewPixels)
+            hipLaunchKernelGGL((bigk ? k_convolve<true, 1> : k_convolve<false, 1>), grid2(w, h), dim3(64, 4), 0,
+                               ctx->stream, (const uint32_t *)src, (uint32_t *)dst, w, h, a, (const float *)bigk);
+        else
+            hipLaunchKernelGGL((bigk ? k_convolve<true, kConvPx> : k_convolve<false, kConvPx>),
+                               grid2((w + kConvPx - 1) / kConvPx, h), dim3(64, 4), 0, ctx->stream,
+                               (const uint32_t *)src, (uint32_t *)dst, w, h, a, (const float *)bigk);
     });
     const hipError_t e = hipGetLastError();
     if (bigk) scratch_release(ctx, bigk);

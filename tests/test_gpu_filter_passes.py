@@ -127,8 +127,8 @@ def test_results_used_again(ctx, seed):
 @pytest.mark.parametrize("edge", [abi.EDGE_NONE, abi.EDGE_DUPLICATE, abi.EDGE_WRAP])
 @pytest.mark.parametrize("shape", [(1, 1), (3, 2), (17, 65), (33, 130)])
 def test_convolution_tiles(ctx, order, edge, shape):
-    # both kernels (a tile of 64 x 16 with its halo in LDS, or straight from memory), images
-    # smaller and larger than a tile and than the matrix, an infinite coefficient
+    # images smaller and larger than a block's 64 x 4 pixels and than the matrix, an infinite
+    # coefficient; images large enough for tiles in LDS are in the test below
     rng = np.random.default_rng(order[0] * 100 + order[1] + edge)
     k = rng.uniform(-1, 1, order[0] * order[1])
     for k0, preserve in ((k[0], False), (k[0], True), (float("inf"), False)):
@@ -140,6 +140,27 @@ def test_convolution_tiles(ctx, order, edge, shape):
         ctx.convolve_matrix(t, g.primitives[0], g.values)
         orc.convolve_matrix(e, g.primitives[0], g.values)
         assert np.array_equal(t.cpu().numpy(), e), (k0, preserve)
+
+
+@pytest.mark.parametrize("edge", [abi.EDGE_NONE, abi.EDGE_DUPLICATE, abi.EDGE_WRAP])
+@pytest.mark.parametrize("shape", [(1021, 1029), (1025, 1023), (1023, 1025), (17, 61681), (1031, 1018),
+                                   (17, 15421), (513, 511), (514, 511)])
+def test_convolution_by_size(ctx, edge, shape):
+    # from memory a thread takes one pixel, or four from 2^20 pixels on, with every remainder
+    # of a row (matrices of more than 64 entries and with an infinite one); the others are
+    # tiled from 2^18 pixels on
+    rng = np.random.default_rng(edge)
+    px = _random(*shape, 7)
+    inf = rng.uniform(-1, 1, 6)
+    inf[1] = float("inf")
+    for order, k in (((5, 13), rng.uniform(-1, 1, 65)), ((3, 2), inf), ((5, 5), rng.uniform(-1, 1, 25)),
+                     ((40, 1), rng.uniform(-1, 1, 40)), ((1, 23), rng.uniform(-1, 1, 23))):
+        g = FilterGraph((0, 0, 1, 1))
+        g.convolve_matrix(order[0], order[1], k, 1.5, 0.1, edge_mode=edge)
+        t, e = _dev(px), px.copy()
+        ctx.convolve_matrix(t, g.primitives[0], g.values)
+        orc.convolve_matrix(e, g.primitives[0], g.values)
+        assert np.array_equal(t.cpu().numpy(), e), order
 
 
 @pytest.mark.parametrize("sig", [(1.2, 0.7), (0.0, 1.1), (1.4, 0.0)])

@@ -1058,16 +1058,21 @@ __global__ __launch_bounds__(256) void k_diff_area(Dims d, const float2 *__restr
     const int lane = (int)(threadIdx.x % 64);
     for (uint32_t c = threadIdx.x; c < rows * stride; c += 256) cells[c] = 0;
     for (uint32_t c0 = 0; c0 <= d.k; c0 += kAreaGroups) {
-        __syncthreads();
-        if (threadIdx.x == 0) ngroups = nedges = 0;
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < kAreaGroups; k += 256) {
-            bool meets = false;
-            if (c0 + k <= d.k) {
-                const float2 b = bounds[(size_t)i * (d.k + 1) + c0 + k];
-                meets = meets_rows(b.x, b.y, y0, y1);
+        if (d.k < batch) {  // all of them fit a batch: their edges are looked at anyway
+            if (threadIdx.x <= d.k) groups[threadIdx.x] = (uint16_t)threadIdx.x;
+            if (threadIdx.x == 0) ngroups = d.k + 1, nedges = 0;
+        } else {
+            __syncthreads();
+            if (threadIdx.x == 0) ngroups = nedges = 0;
+            __syncthreads();
+            for (uint32_t k = threadIdx.x; k < kAreaGroups; k += 256) {
+                bool meets = false;
+                if (c0 + k <= d.k) {
+                    const float2 b = bounds[(size_t)i * (d.k + 1) + c0 + k];
+                    meets = meets_rows(b.x, b.y, y0, y1);
+                }
+                gather(meets, c0 + k, groups, ngroups, lane);
             }
-            gather(meets, c0 + k, groups, ngroups, lane);
         }
         __syncthreads();
         for (uint32_t g0 = 0; g0 < ngroups; g0 += batch) {

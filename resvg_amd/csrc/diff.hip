@@ -1340,10 +1340,16 @@ __global__ __launch_bounds__(1024) void k_diff_reduce(ReducePart paths, ReducePa
     c += tx;
     float s[8] = {};
     if (c < r.cols) {
-        for (uint32_t row = ty; row < r.rows; row += 512) {
+        uint32_t row = ty;
+        for (; row + 7 * 64 < r.rows; row += 512) {
 #pragma unroll
-            for (uint32_t k = 0; k < 8; k++)
-                if (row + 64 * k < r.rows) s[k] += part[(size_t)(row + 64 * k) * r.cols + c];
+            for (uint32_t k = 0; k < 8; k++) s[k] += part[(size_t)(row + 64 * k) * r.cols + c];
+        }
+        // the last ones: loads without a branch, which go out together
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++) {
+            const float v = part[(size_t)min(row + 64 * k, r.rows - 1) * r.cols + c];
+            s[k] += row + 64 * k < r.rows ? v : 0.0f;
         }
     }
     acc[ty][tx] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));

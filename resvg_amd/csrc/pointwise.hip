@@ -1,9 +1,11 @@
 // Per-pixel kernels: colour-space conversion (filter/mod.rs:115-238), colour matrix
 // (filter/color_matrix.rs), component transfer (filter/component_transfer.rs),
 // arithmetic composite (filter/composite.rs), displacement map
-// (filter/displacement_map.rs), fills and copies.  All are bound by memory: a thread
-// takes four pixels of packed RGBA8 a step, in one 16-byte load and store, which need
-// 4-byte alignment only, so widths and offsets of any remainder take them.
+// (filter/displacement_map.rs), feTile, masks, fills and copies.  All are bound by memory.
+// Those that map a pixel to itself (masks aside) take four pixels of packed RGBA8 a thread in one 16-byte
+// load and store, which need 4-byte alignment only, so widths and offsets of any remainder
+// take them; the displacement and the tile gather, a pixel a thread, and the arithmetic
+// composite takes its four one by one.
 #include "rvk_internal.h"
 #include "device_math.h"
 

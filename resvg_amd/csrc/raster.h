@@ -47,7 +47,7 @@ struct PieceDev {
 // the job's slot region of the arena.
 constexpr int kTile = 8;
 constexpr int kBandRows = kTile;    // pixel rows of one coverage band (one tile row)
-constexpr int kChunkTiles = 1024;   // tiles of one band a coverage block handles at a time
+constexpr int kChunkTiles = 1024;   // tiles of a crowded band that its wave handles at a time
 // Tile table entries (u16): empty, full, or kTileSlot0 + k for the band's k-th partial
 // tile, whose bytes (8 rows of 8, row-major) sit at slot (band * tiles_x + k).
 constexpr uint32_t kTileEmpty = 0, kTileFull = 1, kTileSlot0 = 2;

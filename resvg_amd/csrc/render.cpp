@@ -274,7 +274,7 @@ struct Renderer {
     // already run documents side by side)
     const bool overlap = !ctx->is_lane;
     // Whether a flush prepares on the side stream.  A record, a wait and their return on two
-    // streams take 23 us of host time more than the launches alone, about what the coverage
+    // streams take 22 us of host time more than the launches alone, about what the coverage
     // of 2000 bands takes on the device (0.65 ms for the 30 000 of a 4096^2 flush).  With
     // 2048 bands or more the side stream gives 5% there (101.6 against 106.5 ms a render;
     // 104.3 with 8192) and costs nothing at 1024^2 (300 paths: 6.3 ms either way).  A

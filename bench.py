@@ -471,16 +471,21 @@ def _counter_per_dispatch(csv_dir: str, counter: str) -> dict:
     return vals
 
 
-def live_traffic(args):
-    """HBM bytes per launch of the compositor kernel, measured in this run: two child
+# the device kernels behind a profiled launch name whose traffic can be measured
+TRAFFIC_KERNELS = {"draw_items": ("k_draw<false>", "k_draw<true>"), "coverage": ("k_coverage<", "k_coverage_many"),
+                   "expand": ("k_expand<",)}
+
+
+def live_traffic(args, name: str):
+    """HBM bytes per launch of the kernels launched as `name`, measured in this run: two child
     processes render one step of the same document under rocprofv3 --pmc (FETCH_SIZE,
     then WRITE_SIZE; one counter per pass), after a 1 GiB device copy whose counter
     values give the scale from counter units to bytes.  None when rocprofv3 is not
-    available or a pass fails."""
+    available, a pass fails or `name` is not one of TRAFFIC_KERNELS."""
     import shutil
     import subprocess
     import tempfile
-    if shutil.which("rocprofv3") is None:
+    if shutil.which("rocprofv3") is None or name not in TRAFFIC_KERNELS:
         return None
     child = [sys.executable, str(Path(__file__).resolve()), "--steps", "1", "--warmup", "0", "--no-cpu-baseline",
              "--batch-docs", "0", "--diff-size", "0", "--fit-scenes", "0", "--png-reps", "0", "--clip-groups", "0",
@@ -502,11 +507,11 @@ def live_traffic(args):
         # the 1 GiB copy is the largest copy dispatch; the profiler may end with a
         # crash after writing complete results, so the results decide
         cal = max(vals.get("__amd_rocclr_copyBuffer", [0.0]))
-        draw = [x for k, v in vals.items() if "k_draw<false>" in k or "k_draw<true>" in k for x in v]
-        if cal <= 0 or not draw:
+        moved = [x for k, v in vals.items() if any(n in k for n in TRAFFIC_KERNELS[name]) for x in v]
+        if cal <= 0 or not moved:
             print(f"[bench] traffic: {counter} pass gave no values (exit {r.returncode})", file=sys.stderr, flush=True)
             return None
-        per[counter] = sum(draw) / len(draw) * 1024.0 * ((1 << 20) / cal)  # KiB -> bytes, times GiB / copy value
+        per[counter] = sum(moved) / len(moved) * 1024.0 * ((1 << 20) / cal)  # KiB -> bytes, times GiB / copy value
     return {"bytes_per_launch": round(per["FETCH_SIZE"] + per["WRITE_SIZE"]),
             "fetch_bytes": round(per["FETCH_SIZE"]), "write_bytes": round(per["WRITE_SIZE"])}
 
@@ -640,7 +645,7 @@ def main() -> int:
             if rec and rec.get("workload") == f"full-filter {args.size} {args.paths} {args.seed}":
                 traffic, source = rec.get("bytes_per_launch"), "profiles/traffic.json"
         if args.traffic == "live":
-            live = live_traffic(args)
+            live = live_traffic(args, dom["name"])
             if live:
                 traffic, source = live["bytes_per_launch"], "rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE in this run"
         roofline = {
@@ -658,7 +663,7 @@ def main() -> int:
         }
         if traffic:
             # the bytes the kernel actually moves (the rocprofv3 counters above) at its
-            # live launch time: far below `achieved`, since the fused compositor reads
+            # live launch time: for the compositor far below `achieved`, since it reads
             # and writes each target pixel once per flush rather than once per path
             moved = traffic / (dom["total_ms"] / dom["launches"] / 1e3) / 1e9
             roofline["moved_GBps"] = round(moved, 2)

@@ -1022,7 +1022,7 @@ __device__ __forceinline__ bool edge_down(const float2 *vert, uint32_t nv, uint3
 // are written once (they were cleared, added to with global atomics, read and written
 // again); the integers, and so the areas, are the same.  For rows of at most kAreaCells cells.
 // Bound by the planes' stores with few cubics (16 scenes of 512^2 with 128 paths of 8 cubics:
-// 2.15 GB, 1.92 -> 0.65 ms), by the gathers with many: looking at every edge for every row
+// 2.15 GB, 1.92 -> 0.61 ms), by the gathers with many: looking at every edge for every row
 // instead, a forward of 16 wobbly circles of 4096 cubics at 64 x 4096 took 5.9 ms, where the
 // form below, which visits an edge's own rows, took 0.20; now 0.15 (32 of 512 cubics at
 // 512^2: 0.38, 0.12 and 0.09).  Cubics through all of the canvas, 32 of 512 at 512^2: 0.43,

@@ -28,10 +28,12 @@ inline uint32_t demul_rule(uint32_t c, uint32_t a) {
     return d != d ? 0u : d >= 255.0 ? 255u : d <= 0.0 ? 0u : (uint32_t)d;
 }
 
-// floor(c r + 0.5) with one rounding, at most 255.  Clamped before the conversion: at alpha 0 the product is
-// about 1e30, and converting a value out of an integer's range is undefined.
+// floor(c r + 0.5) with one rounding, at most 255.  The factors are at most 1024 (at alpha 0,
+// where every channel but 0 gives 255), so the sum is well within an integer's range, out of
+// which the conversion would be undefined.
 RVK_HOST_DEVICE uint32_t straight_channel(uint32_t c, float r) {
-    return (uint32_t)fminf(fmaf((float)c, r, 0.5f), 255.0f);
+    const uint32_t v = (uint32_t)fmaf((float)c, r, 0.5f);
+    return v < 255u ? v : 255u;
 }
 RVK_HOST_DEVICE bool by_table(float r) { return r < 1.0f; }
 RVK_HOST_DEVICE int table_row(float r) { return (int)(8.0f * r); }
@@ -39,7 +41,7 @@ RVK_HOST_DEVICE int table_row(float r) { return (int)(8.0f * r); }
 inline bool make_demul(Demul &t) {
     int nspecial = 0;
     for (uint32_t a = 0; a < 256; a++) {
-        const float r0 = a ? 255.0f / (float)a : 1e30f;
+        const float r0 = a ? 255.0f / (float)a : 1024.0f;
         const float tries[3] = {r0, std::nextafter(r0, 0.0f), std::nextafter(r0, 1e38f)};
         bool found = false;
         for (int k = 0; k < 3 && !found; k++) {
